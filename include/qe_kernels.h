@@ -191,9 +191,9 @@ void qe_gemm_w4_s(const void* q, const void* s, int n, int k, const uint16_t* x,
  * Replaces reference src/capi.cpp:114 (gemm_set_out_bf16, gemm.cu:4363-4375). */
 void qe_gemm_set_out_bf16(int on);
 /* run-time cap of the stream-K split: later prefill GEMM calls (W4, W8 / Q8 bf16-activation GEMMs) split the tiles
- * of their last partial round into at most n K ranges (n <= 0: no cap, the default; splits here are 1, 2 or 4, so
- * n = 1 turns the split off and n = 2 or 3 allows 2). Applies to the cost model's, the tuner's and a stored choice
- * alike (a stored split above the cap runs as the largest allowed one). Replaces reference src/capi.cpp:115
+ * of their last partial round into at most n K ranges (n <= 0: no cap, the default; splits here are 1..16, n = 1
+ * turns the split off). Applies to the cost model's, the tuner's and a stored choice alike (the cost model picks among
+ * the allowed ones; a stored split above the cap is halved until it fits). Replaces reference src/capi.cpp:115
  * (gemm_set_sk_maxparts, gemm.cu:3485-3496,4359). */
 void qe_gemm_set_sk_maxparts(int n);
 

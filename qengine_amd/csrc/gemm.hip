@@ -42,8 +42,9 @@ struct Cfg {
     static constexpr int kLdsW4 = 2 * kStage + 2 * kRaw + 2 * kSc;
 };
 
-// Split tiles: the tiles from `ndirect` on run as `ks` K ranges each (stream-K of the last, partly filled
-// round); their fp32 partials go to part [(tile - ndirect) * ks + split][BM][BN] and splitk_reduce_kernel adds them
+// Split tiles: the tiles from `ndirect` on run as `ks` K ranges of whole 128-k groups each (the last, partly filled
+// round, or every tile when they do not fill one round); their fp32 partials go to
+// part [(tile - ndirect) * ks + split][BM][BN] and splitk_reduce_kernel adds them
 struct SplitArgs {
     int ndirect = 1 << 30;
     int ks = 1;
@@ -76,12 +77,15 @@ __global__ void __launch_bounds__(NTH) gemm_kernel(const uint4* __restrict__ q, 
         tile = (b & 7) * per + (b >> 3);
         if (tile >= sp.ndirect) return;
     } else {
-        const int j = b - 8 * per;
-        tile = sp.ndirect + j / sp.ks;
-        if (tile >= ntiles) return;
-        KTL = K / BK / sp.ks;
-        kt0 = (j % sp.ks) * KTL;
-        split_slot = j;
+        // ranges outermost: consecutive items of an XCD's band read the same K range of one X tile
+        const int nsplit = ntiles - sp.ndirect, items = nsplit * sp.ks;
+        const int j = b - 8 * per, it = (j & 7) * ((items + 7) >> 3) + (j >> 3);
+        if (it >= items || (j >> 3) >= ((items + 7) >> 3)) return;
+        const int z = it / nsplit, ts = it - z * nsplit, groups = K >> 7;
+        tile = sp.ndirect + ts;
+        kt0 = 2 * (z * groups / sp.ks);
+        KTL = 2 * ((z + 1) * groups / sp.ks) - kt0;
+        split_slot = ts * sp.ks + z;
     }
     n0 = (tile % nbn) * BN;
     t0 = (tile / nbn) * BM;
@@ -386,19 +390,22 @@ __global__ void __launch_bounds__(NTH) gemm_kernel(const uint4* __restrict__ q, 
     //      r + 4 of the same lane.
     const int cj = lane & 31, ci = 4 * (lane >> 5);
     if (split_slot >= 0) {
-        // raw fp32 partial of the whole BM x BN tile, [token][row] (rows past N / tokens past T included)
+        // raw fp32 partial of the BM x BN tile, [token][row] (rows past N included, tokens past T not)
         float* pp = sp.part + (size_t)split_slot * BM * BN;
 #pragma unroll
-        for (int a = 0; a < WMT; a++)
+        for (int a = 0; a < WMT; a++) {
+            const int tl = wm * 32 * WMT + a * 32 + cj;
+            if (t0 + tl >= T) continue;
 #pragma unroll
             for (int bb = 0; bb < WNT; bb++)
 #pragma unroll
                 for (int rb = 0; rb < 4; rb++) {
-                    const int tl = wm * 32 * WMT + a * 32 + cj, nl = wn * 32 * WNT + bb * 32 + 8 * rb + ci;
+                    const int nl = wn * 32 * WNT + bb * 32 + 8 * rb + ci;
                     const f32x16_v& v = acc[a][bb];
                     *reinterpret_cast<f32x4_v*>(pp + (size_t)tl * BN + nl) =
                         f32x4_v{v[4 * rb], v[4 * rb + 1], v[4 * rb + 2], v[4 * rb + 3]};
                 }
+        }
         return;
     }
     const bool vec = (ldc & 3) == 0 && ((uintptr_t)c & (out == kOutF32 ? 15u : 7u)) == 0;
@@ -448,48 +455,55 @@ __global__ void __launch_bounds__(NTH) gemm_kernel(const uint4* __restrict__ q, 
         }
 }
 
-// Split tiles' partials -> outputs: one thread per (split tile, token row, 16 output columns); the ks partials are
-// added in split order (fixed order: the result does not depend on timing), then the epilogue of the GEMM
-template <int BM, int BN>
+// Split tiles' partials -> outputs: one thread per (split tile, token row, 4 input columns; GLU: 4 gate columns and
+// the 4 up columns 8 to the right); the ks partials are added in split order (fixed order: the result does not depend
+// on timing), then the epilogue of the GEMM. Reads are 16 bytes a lane, consecutive lanes consecutive.
+template <int BM, int BN, bool GLU>
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* __restrict__ part, int ks, int ndirect,
                                                             int nsplit, int nbn, int T, int N, void* __restrict__ c,
                                                             int ldc, int out) {
-    constexpr int CB = BN / 16;
+    constexpr int CB = GLU ? BN / 8 : BN / 4;  // threads per row
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= (size_t)nsplit * BM * CB) return;
     const int st = (int)(idx / ((size_t)BM * CB)), r = (int)((idx / CB) % BM), cb = (int)(idx % CB);
     const int tile = ndirect + st;
-    const int tok = (tile / nbn) * BM + r, n = (tile % nbn) * BN + 16 * cb;
+    const int col = GLU ? 16 * (cb >> 1) + 4 * (cb & 1) : 4 * cb;
+    const int tok = (tile / nbn) * BM + r, n = (tile % nbn) * BN + col;
     if (tok >= T || n >= N) return;
-    float v[16];
+    const float* p = part + ((size_t)st * ks * BM + r) * BN + col;
+    f32x4_v v{0.f, 0.f, 0.f, 0.f}, u{0.f, 0.f, 0.f, 0.f};
+    for (int z = 0; z < ks; z++, p += (size_t)BM * BN) {
+        const f32x4_v a = *reinterpret_cast<const f32x4_v*>(p);
 #pragma unroll
-    for (int j = 0; j < 16; j++) v[j] = 0.f;
-    for (int z = 0; z < ks; z++) {
-        const f32x4_v* p = reinterpret_cast<const f32x4_v*>(part + (((size_t)st * ks + z) * BM + r) * BN + 16 * cb);
+        for (int j = 0; j < 4; j++) v[j] += a[j];
+        if constexpr (GLU) {
+            const f32x4_v b = *reinterpret_cast<const f32x4_v*>(p + 8);
 #pragma unroll
-        for (int q4 = 0; q4 < 4; q4++) {
-            const f32x4_v a = p[q4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[4 * q4 + j] += a[j];
+            for (int j = 0; j < 4; j++) u[j] += b[j];
         }
     }
-    if (out == kOutGLU) {
-        uint16_t* o = reinterpret_cast<uint16_t*>(c) + (size_t)tok * ldc + (n >> 4) * 8;
+    if constexpr (GLU) {
+        uint16_t* o = reinterpret_cast<uint16_t*>(c) + (size_t)tok * ldc + (n >> 4) * 8 + (n & 7);
 #pragma unroll
-        for (int j = 0; j < 8; j++) o[j] = f32_to_bf16(silu_f32(v[j]) * v[j + 8]);
+        for (int j = 0; j < 4; j++) o[j] = f32_to_bf16(silu_f32(v[j]) * u[j]);
     } else if (out == kOutBF16) {
         uint16_t* o = reinterpret_cast<uint16_t*>(c) + (size_t)tok * ldc + n;
+        if (((ldc & 3) | ((uintptr_t)c & 7)) == 0) {
+            *reinterpret_cast<uint2*>(o) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        } else {
 #pragma unroll
-        for (int j = 0; j < 16; j++) o[j] = f32_to_bf16(v[j]);
+            for (int j = 0; j < 4; j++) o[j] = f32_to_bf16(v[j]);
+        }
     } else {
         float* o = reinterpret_cast<float*>(c) + (size_t)tok * ldc + n;
 #pragma unroll
-        for (int j = 0; j < 16; j++) o[j] = v[j];
+        for (int j = 0; j < 4; j++) o[j] = v[j];
     }
 }
 
-// tile configurations: 0 = 256 tokens x 256 rows (WMT 4, WNT 2), 1 = 256 x 128 (4, 1)
-constexpr int kNumCfg = 2;
+// tile configurations: 0 = 256 tokens x 256 rows (WMT 4, WNT 2), 1 = 256 x 128 (4, 1), 2 = 128 x 256 (2, 2),
+// 3 = 128 x 128 (2, 1; two blocks per CU)
+constexpr int kNumCfg = 4;
 template <int CFG>
 struct CfgOf;
 template <>
@@ -500,32 +514,76 @@ template <>
 struct CfgOf<1> {
     static constexpr int WMT = 4, WNT = 1;
 };
+template <>
+struct CfgOf<2> {
+    static constexpr int WMT = 2, WNT = 2;
+};
+template <>
+struct CfgOf<3> {
+    static constexpr int WMT = 2, WNT = 1;
+};
+
+constexpr int kMaxSplit = 16;
 
 struct GemmGeom {
     int nbn, nbt, ntiles, ndirect, nsplit, ks;
     size_t ws_bytes;
 };
+struct CfgDims {
+    int BM, BN, slots;  // tile and how many of its blocks the device holds at once (LDS: one per CU, two of 128 x 128)
+};
+CfgDims cfg_dims(int cfg) {
+    return CfgDims{cfg < 2 ? 256 : 128, (cfg & 1) ? 128 : 256, qe_num_cus() * (cfg == 3 ? 2 : 1)};
+}
+// the most partial-sum workspace a split may take: one 256 x 256 fp32 tile per CU (64 MB)
+size_t max_split_bytes() { return (size_t)qe_num_cus() * 256 * 256 * 4; }
+
 // tiles of configuration cfg and, for ks > 1, the split of the last partial round (stream-K): whole rounds of
-// tiles run directly, the remaining tiles as ks K ranges; false when that split does not apply (no partial round,
-// K steps not divisible into even ranges)
+// tiles run directly, the remaining tiles (all of them when they do not fill one round) as ks K ranges; false when
+// that split does not apply (no partial round, fewer 128-k groups than ranges, too much workspace)
 bool gemm_geom(int cfg, int n, int k, int t, int ks, GemmGeom& g) {
-    const int BM = 256, BN = cfg == 0 ? 256 : 128;
-    g.nbn = (n + BN - 1) / BN;
-    g.nbt = (t + BM - 1) / BM;
+    const CfgDims d = cfg_dims(cfg);
+    g.nbn = (n + d.BN - 1) / d.BN;
+    g.nbt = (t + d.BM - 1) / d.BM;
     g.ntiles = g.nbn * g.nbt;
     g.ks = ks;
     g.ndirect = g.ntiles;
     g.nsplit = 0;
     g.ws_bytes = 0;
     if (ks == 1) return true;
-    const int cus = qe_num_cus(), KT = k / BK;
-    if (KT % (2 * ks) != 0) return false;
-    const int tail = g.ntiles % cus;
-    if (tail == 0 || tail * ks > cus) return false;
+    const int tail = g.ntiles % d.slots;
+    const size_t bytes = (size_t)tail * ks * d.BM * d.BN * 4;
+    if (tail == 0 || k / 128 < ks || bytes > max_split_bytes()) return false;
     g.ndirect = g.ntiles - tail;
     g.nsplit = tail;
-    g.ws_bytes = (size_t)tail * ks * BM * BN * 4;
+    g.ws_bytes = bytes;
     return true;
+}
+
+// Predicted time in us of a choice: the k steps of the fullest CU at a measured cost per step, which falls when only
+// part of the CUs run (clock, shared caches), plus the partial sums written and read again. Fitted to a sweep of
+// every (configuration, ks <= 16) on (n, k) from 1280 x 4224 to 34816 x 5120, t = 70..4000 (MI355X, fp16 scales;
+// 6 % rms): the choice below is within 8 % of the best measured one there for t >= 200, within 25 % for smaller t.
+double gemm_cost_us(int cfg, int n, int k, int t, const GemmGeom& g) {
+    static const double kFull[kNumCfg] = {1.754, 1.074, 1.107, 1.264};  // us per 64-k step, every slot filled
+    static const double kPart[kNumCfg] = {1.233, 0.777, 0.829, 0.678};  // few slots filled
+    const CfgDims d = cfg_dims(cfg);
+    auto phase = [&](int blocks, int steps) {
+        const int full = blocks / d.slots, rem = blocks % d.slots;
+        double us = full * (steps * kFull[cfg] + 0.45);
+        if (rem) {
+            double u = (double)rem / d.slots;
+            if (cfg == 3) u = u < 0.5 ? 0.0 : 2.0 * u - 1.0;  // the share of CUs that hold a second block
+            us += steps * (u * kFull[cfg] + (1.0 - u) * kPart[cfg]) + 0.45;
+        }
+        return us;
+    };
+    double us = phase(g.ndirect, k / BK);
+    if (g.nsplit > 0) {
+        us += phase(g.nsplit * g.ks, 2 * ((k / 128 + g.ks - 1) / g.ks));
+        us += 1.3 + 0.266e-6 * g.nsplit * g.ks * ((double)t / g.nbt) * d.BN * 4;
+    }
+    return us;
 }
 
 }  // namespace
@@ -546,16 +604,59 @@ void launch_cfg(const uint4* q, const uint16_t* s, int n, int k, const uint16_t*
     sp.ks = g.ks;
     sp.part = part;
     const int per = (g.ndirect + 7) / 8;
-    const unsigned blocks = (unsigned)(8 * per + g.nsplit * g.ks);
+    const unsigned blocks = (unsigned)(8 * per + 8 * ((g.nsplit * g.ks + 7) / 8));
     gemm_kernel<FMT, SDT, WMT, WNT><<<dim3(blocks), dim3(NTH), FMT == kFmtW4 ? C::kLdsW4 : 2 * C::kStage, st>>>(
         q, s, n, k, x, ldx, t, c, ldc, out, sdt, g.nbn, g.nbt, sp);
     HIP_CHECK(hipGetLastError());
     if (g.nsplit > 0) {
-        const size_t threads = (size_t)g.nsplit * C::BM * (C::BN / 16);
-        splitk_reduce_kernel<C::BM, C::BN><<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st>>>(
-            part, g.ks, g.ndirect, g.nsplit, g.nbn, t, n, c, ldc, out);
+        const bool glu = out == kOutGLU;
+        const size_t threads = (size_t)g.nsplit * C::BM * (C::BN / (glu ? 8 : 4));
+        const dim3 grid((unsigned)((threads + 255) / 256));
+        if (glu)
+            splitk_reduce_kernel<C::BM, C::BN, true><<<grid, dim3(256), 0, st>>>(part, g.ks, g.ndirect, g.nsplit,
+                                                                                 g.nbn, t, n, c, ldc, out);
+        else
+            splitk_reduce_kernel<C::BM, C::BN, false><<<grid, dim3(256), 0, st>>>(part, g.ks, g.ndirect, g.nsplit,
+                                                                                  g.nbn, t, n, c, ldc, out);
         HIP_CHECK(hipGetLastError());
     }
+}
+
+// untuned choice: 256 x 256 tiles when they fill the CUs at least once (else 256 x 128), with the last partial round
+// split in two K ranges when it is at most half full, unless the cost model puts another choice at least 5 % lower
+// (its error; below that the larger tile stays). maxparts: the largest split allowed (0: any).
+// The last choices of a thread are kept: 64 cost evaluations take about as long as a launch.
+GemmChoice gemm_model_choice(int n, int k, int t, int maxparts) {
+    const int cus = qe_num_cus();
+    struct Kept {
+        int n = 0, k = 0, t = 0, maxparts = 0, cus = 0;
+        GemmChoice ch;
+    };
+    static thread_local Kept kept[64];
+    Kept& slot = kept[((unsigned)n * 31u + (unsigned)k * 17u + (unsigned)t * 7u + (unsigned)maxparts) >> 4 & 63u];
+    if (slot.n == n && slot.k == k && slot.t == t && slot.maxparts == maxparts && slot.cus == cus) return slot.ch;
+    const long tiles_big = (long)((n + 255) / 256) * ((t + 255) / 256);
+    GemmChoice ch{tiles_big >= cus ? 0 : 1, 1};
+    GemmGeom g;
+    if (ch.cfg == 0 && maxparts != 1 && k / BK % 4 == 0 && gemm_geom(0, n, k, t, 2, g) && 2 * g.nsplit <= cus) ch.ks = 2;
+    else if (ch.cfg == 0) {
+        const long rounds = (tiles_big + cus - 1) / cus;
+        if ((double)tiles_big / (rounds * cus) < 0.9) ch.cfg = 1;
+    }
+    gemm_geom(ch.cfg, n, k, t, ch.ks, g);
+    const double base = gemm_cost_us(ch.cfg, n, k, t, g);
+    double best = 0.95 * base;
+    for (int cfg = 0; cfg < kNumCfg; cfg++)
+        for (int ks = 1; ks <= kMaxSplit && (maxparts <= 0 || ks <= maxparts); ks++) {
+            if (!gemm_geom(cfg, n, k, t, ks, g)) continue;
+            const double us = gemm_cost_us(cfg, n, k, t, g);
+            if (us < best) {
+                best = us;
+                ch = GemmChoice{cfg, ks};
+            }
+        }
+    slot = Kept{n, k, t, maxparts, cus, ch};
+    return ch;
 }
 
 template <int FMT, int SDT>
@@ -564,39 +665,38 @@ void run_choice(int cfg, int ks, const uint4* q, const uint16_t* s, int n, int k
     GemmGeom g;
     float* part = nullptr;
     if (ks > 1) {
-        if (!gemm_geom(cfg, n, k, t, ks, g) || (part = static_cast<float*>(stream_ws(kWsSplit, g.ws_bytes, st))) == nullptr) ks = 1;
+        // no such split, or no workspace for it during a graph capture: the best unsplit configuration
+        if (!gemm_geom(cfg, n, k, t, ks, g)) ks = 1;
+        else if ((part = static_cast<float*>(stream_ws(kWsSplit, g.ws_bytes, st))) == nullptr) {
+            ks = 1;
+            cfg = gemm_model_choice(n, k, t, 1).cfg;
+        }
     }
     if (ks == 1) gemm_geom(cfg, n, k, t, 1, g);
     if (cfg == 0) launch_cfg<FMT, SDT, 0>(q, s, n, k, x, ldx, t, c, ldc, out, sdt, g, part, st);
-    else launch_cfg<FMT, SDT, 1>(q, s, n, k, x, ldx, t, c, ldc, out, sdt, g, part, st);
+    else if (cfg == 1) launch_cfg<FMT, SDT, 1>(q, s, n, k, x, ldx, t, c, ldc, out, sdt, g, part, st);
+    else if (cfg == 2) launch_cfg<FMT, SDT, 2>(q, s, n, k, x, ldx, t, c, ldc, out, sdt, g, part, st);
+    else launch_cfg<FMT, SDT, 3>(q, s, n, k, x, ldx, t, c, ldc, out, sdt, g, part, st);
 }
 
-// untuned choice (cost model): 256 x 256 tiles when they fill the CUs at least once (else 256 x 128), with the last
-// partial round split in two K ranges when it is at most half full
-GemmChoice gemm_model_choice(int n, int k, int t) {
-    const int cus = qe_num_cus();
-    const long tiles_big = (long)((n + 255) / 256) * ((t + 255) / 256);
-    GemmChoice ch{tiles_big >= cus ? 0 : 1, 1};
-    GemmGeom g;
-    if (ch.cfg == 0 && gemm_geom(0, n, k, t, 2, g)) ch.ks = 2;
-    else if (ch.cfg == 0) {
-        const long rounds = (tiles_big + cus - 1) / cus;
-        if ((double)tiles_big / (rounds * cus) < 0.9) ch.cfg = 1;
-    }
-    return ch;
-}
-
-// timed choice: every (configuration, split) candidate once untimed, then 5 rounds in rotating order, the median;
-// outside graph capture only (during capture: the cost model)
+// timed choice: the candidates (the eight the cost model puts lowest, beside 256 x 256 and 256 x 128 tiles with splits
+// 1, 2 and 4) once untimed, then 5 rounds in rotating order, the median; outside graph capture only (during capture:
+// the cost model)
 template <int FMT, int SDT>
 GemmChoice gemm_tune_choice(int n, int k, const uint16_t* x, int ldx, int t, void* c, int ldc, int out, int sdt,
                             const uint4* q, const uint16_t* s, hipStream_t st) {
     std::vector<GemmChoice> cl;
+    std::vector<std::pair<double, GemmChoice>> all;
     for (int cfg = 0; cfg < kNumCfg; cfg++)
-        for (int ks : {1, 2, 4}) {
+        for (int ks = 1; ks <= kMaxSplit; ks++) {
             GemmGeom g;
-            if (gemm_geom(cfg, n, k, t, ks, g)) cl.push_back(GemmChoice{cfg, ks});
+            if (gemm_geom(cfg, n, k, t, ks, g)) all.emplace_back(gemm_cost_us(cfg, n, k, t, g), GemmChoice{cfg, ks});
         }
+    std::stable_sort(all.begin(), all.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
+    for (size_t i = 0; i < all.size(); i++) {
+        const GemmChoice& ch = all[i].second;
+        if (i < 8 || (ch.cfg < 2 && (ch.ks == 1 || ch.ks == 2 || ch.ks == 4))) cl.push_back(ch);
+    }
     hipEvent_t e0, e1;
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
@@ -631,7 +731,7 @@ GemmChoice gemm_tune_choice(int n, int k, const uint16_t* x, int ldx, int t, voi
     return cl[best];
 }
 
-// the largest split <= ks that qe_gemm_set_sk_maxparts allows (splits are 1, 2 or 4)
+// a stored or tuned split halved until qe_gemm_set_sk_maxparts allows it
 int capped_split(int ks) {
     const int cap = gemm_sk_maxparts();
     while (cap > 0 && ks > cap) ks /= 2;
@@ -650,7 +750,7 @@ void launch_gemm(const uint4* q, const uint16_t* s, int n, int k, const uint16_t
             ch = gemm_tune_choice<FMT, SDT>(n, k, x, ldx, t, c, ldc, out, sdt, q, s, st);
             gemm_table_add(key, ch);
         } else {
-            ch = gemm_model_choice(n, k, t);
+            ch = gemm_model_choice(n, k, t, gemm_sk_maxparts());
         }
     }
     run_choice<FMT, SDT>(ch.cfg, capped_split(ch.ks), q, s, n, k, x, ldx, t, c, ldc, out, sdt, st);
@@ -680,7 +780,7 @@ void gemm_w4(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, b
 void gemm_w4_choice(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, bool out_bf16, int cfg, int ks,
                     hipStream_t st) {
     gemm_check(w.n, w.k, x, ldx, ldc, t, w.glu);
-    CHECK(cfg >= 0 && cfg < kNumCfg && (ks == 1 || ks == 2 || ks == 4), "gemm choice cfg %d ks %d", cfg, ks);
+    CHECK(cfg >= 0 && cfg < kNumCfg && ks >= 1 && ks <= kMaxSplit, "gemm choice cfg %d ks %d", cfg, ks);
     const int out = w.glu ? kOutGLU : out_bf16 ? kOutBF16 : kOutF32;
     if (w.sdt == kScaleF16) run_choice<kFmtW4, kScaleF16>(cfg, ks, w.q, w.s, w.n, w.k, x, ldx, t, c, ldc, out, w.sdt, st);
     else run_choice<kFmtW4, kScaleBF16>(cfg, ks, w.q, w.s, w.n, w.k, x, ldx, t, c, ldc, out, w.sdt, st);

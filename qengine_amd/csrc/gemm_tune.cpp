@@ -1,5 +1,6 @@
 // GEMM tuning table (see gemm_tune.hpp). File format (text):
-//   qengine_amd gemm tune v1 cfg=256x256,256x128 ks=1,2,4
+//   qengine_amd gemm tune v1 cfg=256x256,256x128,128x256,128x128 ks=1..16
+//   (files whose first line lists the first two tile shapes and ks=1,2,4 are read too: their choices mean the same)
 //   device <pci bus id> <cus>          (a section per device)
 //   <fmt> <n> <k> <bucket> <glu> <cfg> <ks>
 #include "gemm_tune.hpp"
@@ -13,7 +14,8 @@
 
 namespace {
 
-const char* const kHeader = "qengine_amd gemm tune v1 cfg=256x256,256x128 ks=1,2,4";
+const char* const kHeader = "qengine_amd gemm tune v1 cfg=256x256,256x128,128x256,128x128 ks=1..16";
+const char* const kHeaderTwoShapes = "qengine_amd gemm tune v1 cfg=256x256,256x128 ks=1,2,4";
 std::mutex g_mu;
 std::map<std::string, std::map<GemmKey, GemmChoice>> g_tab;  // device line -> choices
 std::string g_path;
@@ -53,7 +55,9 @@ void load_locked() {
     char line[512];
     std::map<std::string, std::map<GemmKey, GemmChoice>> tab;
     std::string cur;
-    bool ok = fgets(line, sizeof(line), f) && strncmp(line, kHeader, strlen(kHeader)) == 0;
+    const bool first = fgets(line, sizeof(line), f) != nullptr;
+    const bool two = first && strncmp(line, kHeaderTwoShapes, strlen(kHeaderTwoShapes)) == 0;
+    bool ok = two || (first && strncmp(line, kHeader, strlen(kHeader)) == 0);
     while (ok && fgets(line, sizeof(line), f)) {
         if (strncmp(line, "device ", 7) == 0) {
             cur = line;
@@ -63,7 +67,8 @@ void load_locked() {
         GemmKey k{};
         GemmChoice c{};
         if (sscanf(line, "%d %d %d %d %d %d %d", &k.fmt, &k.n, &k.k, &k.bucket, &k.glu, &c.cfg, &c.ks) != 7 ||
-            cur.empty() || c.cfg < 0 || c.cfg > 1 || (c.ks != 1 && c.ks != 2 && c.ks != 4)) {
+            cur.empty() || c.cfg < 0 || c.cfg > (two ? 1 : 3) || c.ks < 1 || c.ks > (two ? 4 : 16) ||
+            (two && c.ks == 3)) {
             ok = false;
             break;
         }

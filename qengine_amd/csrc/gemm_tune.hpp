@@ -5,8 +5,8 @@
 #include "qe_api.hpp"
 
 struct GemmChoice {
-    int cfg = 0;  // 0: 256 x 256 tiles, 1: 256 x 128
-    int ks = 1;   // K ranges of the last partial round's tiles (1: no split)
+    int cfg = 0;  // tiles (tokens x rows) 0: 256 x 256, 1: 256 x 128, 2: 128 x 256, 3: 128 x 128
+    int ks = 1;   // K ranges of the last partial round's tiles, 1..16 (1: no split)
 };
 struct GemmKey {
     int fmt, n, k, bucket, glu;

@@ -1,0 +1,98 @@
+"""Prefill GEMM calls whose tiles do not fill the CUs: the four tile shapes and the splits in up to 16 uneven K ranges
+that the cost model picks, against the oracle (1e-4 * rms: the products are the oracle's, only the order of the fp32
+sums differs). K = 1152 and 2176 are 9 and 17 groups (ranges of unequal length), t crosses the 128- and 256-token
+tiles, n leaves ragged row tiles."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from qengine_amd import call, lib, ops, synth
+from test_gemm_gpu import setup
+from test_gemv_gpu import assert_glu_close, err_ratio, glu_act, oracle_ref, out_f32
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,k,t", [(272, 1152, 65), (2976, 2176, 75), (144, 2176, 128), (1040, 1152, 129),
+                                   (528, 2176, 257), (4112, 1152, 300), (2048, 128, 200), (272, 1152, 1100)])
+@pytest.mark.parametrize("glu", [False, True])
+def test_underfilled_prefill(dev, n, k, t, glu):
+    w, q, s = setup(n, k, 1, seed=n + t, glu=glu)
+    xh = synth.x_host(t, k, seed=t)
+    x = synth.to_dev(xh)
+    rows = np.unique(np.r_[0, t // 2, 127 % t, 128 % t, t - 1, np.random.default_rng(t).integers(0, t, 8)])
+    if glu:
+        act = glu_act(oracle_ref(xh[rows], q, s, n, k, 1))
+        y = ops.gemm_w4(w, x)
+        assert_glu_close(out_f32(y)[rows], act, 1e-4)
+        cols = n // 2
+    else:
+        ref = oracle_ref(xh, q, s, n, k, 1)
+        y = ops.gemm_w4(w, x, out_bf16=True)
+        y32 = ops.gemm_w4(w, x)
+        assert err_ratio(out_f32(y32), ref) <= 1e-4
+        assert torch.equal(y32.bfloat16().view(torch.int16), y.view(torch.int16))
+        cols = n
+    # rows of an odd stride at an odd offset (scalar stores, also of the split tiles' sums)
+    big = torch.full((t, cols + 7), float("nan"), dtype=torch.bfloat16, device=dev)
+    got = ops.gemm_w4(w, x, out_bf16=True, y=big[:, 1:1 + cols])
+    assert torch.equal(got.contiguous().view(torch.int16), y.view(torch.int16))
+    assert torch.isnan(big[:, 0]).all() and torch.isnan(big[:, 1 + cols:]).all()
+
+
+@pytest.mark.parametrize("per_channel", [True, False])
+def test_underfilled_prefill_w8(dev, per_channel):
+    from test_gemv_gpu import oracle_ref_w8
+    n, k, t = 272, 1152, 140
+    q, s = synth.w8_host(n, k, seed=3, per_channel=per_channel)
+    w = ops.tile_w8(synth.to_dev(q), synth.to_dev(s, torch.float16), per_channel)
+    xh = synth.x_host(t, k, seed=4)
+    y = ops.gemm_w8(w, synth.to_dev(xh))
+    assert err_ratio(out_f32(y), oracle_ref_w8(xh, q, s, n, k, per_channel)) <= 1e-4
+
+
+def test_capture_without_workspace_runs_unsplit(dev):
+    """a split needs a workspace of its stream: a capture on a stream that has none runs the unsplit GEMM, and every
+    replay gives the eager unsplit bits"""
+    n, k, t = 272, 2176, 100
+    w, q, s = setup(n, k, 1, seed=21)
+    x = synth.to_dev(synth.x_host(t, k, seed=22))
+    call("qe_gemm_set_sk_maxparts", 1)
+    try:
+        want = ops.gemm_w4(w, x)
+    finally:
+        call("qe_gemm_set_sk_maxparts", 0)
+    eager = ops.gemm_w4(w, x)
+    y = torch.empty_like(want)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        ops.gemm_w4(w, x, y=y)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int32), want.view(torch.int32))
+    assert err_ratio(eager.cpu().numpy(), want.cpu().numpy()) <= 1e-5
+
+
+def test_tune_file_with_two_tile_shapes(dev, tmp_path):
+    """a tuning file that lists 256 x 256 and 256 x 128 tiles and splits 1, 2, 4 is still read; a choice outside that
+    list makes it malformed"""
+    lib().qe_gemm_tune_entries.restype = ctypes.c_int
+    p = tmp_path / "tune.txt"
+    head = "qengine_amd gemm tune v1 cfg=256x256,256x128 ks=1,2,4\ndevice 0000:00:00.0 256\n"
+    call("qe_gemm_tune_clear")
+    try:
+        p.write_text(head + "0 2048 1024 512 0 1 2\n")
+        call("qe_gemm_tune_file", ctypes.c_char_p(str(p).encode()))
+        assert lib().qe_gemm_tune_entries() == 1
+        call("qe_gemm_tune_clear")
+        p.write_text(head + "0 2048 1024 512 0 2 2\n")
+        call("qe_gemm_tune_file", ctypes.c_char_p(str(p).encode()))
+        assert lib().qe_gemm_tune_entries() == 0
+    finally:
+        call("qe_gemm_tune_file", ctypes.c_char_p(b""))
+        call("qe_gemm_tune_clear")
