@@ -16,6 +16,7 @@
 //   grid: one block per output tile, tiles ordered so that the 8 XCDs (blockIdx % 8) each sweep a contiguous band
 //        of tiles (their L2 keeps the shared X / W tiles).
 #include "mfma_tile.hpp"
+#include "gemm_split.hpp"
 #include "gemm_tune.hpp"
 
 #include <algorithm>
@@ -29,7 +30,6 @@ using namespace qe_tile;
 constexpr int BK = 64, NTH = 512;
 
 enum Fmt : int { kFmtW4 = 0, kFmtW8G = 1, kFmtW8C = 2, kFmtQ8 = 3 };
-enum Out : int { kOutF32 = 0, kOutBF16 = 1, kOutGLU = 2 };
 
 template <int WMT, int WNT>
 struct Cfg {
@@ -40,15 +40,6 @@ struct Cfg {
     // both double-buffered after the two stages
     static constexpr int kRaw = BN * 32, kSc = BN * 2;
     static constexpr int kLdsW4 = 2 * kStage + 2 * kRaw + 2 * kSc;
-};
-
-// Split tiles: the tiles from `ndirect` on run as `ks` K ranges of whole 128-k groups each (the last, partly filled
-// round, or every tile when they do not fill one round); their fp32 partials go to
-// part [(tile - ndirect) * ks + split][BM][BN] and splitk_reduce_kernel adds them
-struct SplitArgs {
-    int ndirect = 1 << 30;
-    int ks = 1;
-    float* part = nullptr;
 };
 
 template <int FMT, int SDT, int WMT, int WNT>
@@ -77,11 +68,10 @@ __global__ void __launch_bounds__(NTH) gemm_kernel(const uint4* __restrict__ q, 
         tile = (b & 7) * per + (b >> 3);
         if (tile >= sp.ndirect) return;
     } else {
-        // ranges outermost: consecutive items of an XCD's band read the same K range of one X tile
-        const int nsplit = ntiles - sp.ndirect, items = nsplit * sp.ks;
-        const int j = b - 8 * per, it = (j & 7) * ((items + 7) >> 3) + (j >> 3);
-        if (it >= items || (j >> 3) >= ((items + 7) >> 3)) return;
-        const int z = it / nsplit, ts = it - z * nsplit, groups = K >> 7;
+        const int j = b - 8 * per;
+        int ts, z;
+        if (!split_item(j, ntiles - sp.ndirect, sp.ks, ts, z)) return;
+        const int groups = K >> 7;
         tile = sp.ndirect + ts;
         kt0 = 2 * (z * groups / sp.ks);
         KTL = 2 * ((z + 1) * groups / sp.ks) - kt0;
@@ -391,21 +381,21 @@ __global__ void __launch_bounds__(NTH) gemm_kernel(const uint4* __restrict__ q, 
     const int cj = lane & 31, ci = 4 * (lane >> 5);
     if (split_slot >= 0) {
         // raw fp32 partial of the BM x BN tile, [token][row] (rows past N included, tokens past T not)
-        float* pp = sp.part + (size_t)split_slot * BM * BN;
-#pragma unroll
-        for (int a = 0; a < WMT; a++) {
-            const int tl = wm * 32 * WMT + a * 32 + cj;
-            if (t0 + tl >= T) continue;
-#pragma unroll
-            for (int bb = 0; bb < WNT; bb++)
-#pragma unroll
-                for (int rb = 0; rb < 4; rb++) {
-                    const int nl = wn * 32 * WNT + bb * 32 + 8 * rb + ci;
-                    const f32x16_v& v = acc[a][bb];
-                    *reinterpret_cast<f32x4_v*>(pp + (size_t)tl * BN + nl) =
-                        f32x4_v{v[4 * rb], v[4 * rb + 1], v[4 * rb + 2], v[4 * rb + 3]};
-                }
-        }
+        static_assert(NTH / 64 * 32 * out_pitch<kOutF32, WNT>() <= 2 * C::kStage, "one buffer per wave in the stages");
+        store_rows<kOutF32>(acc, lds + wave * 32 * out_pitch<kOutF32, WNT>(), lane, wm * 32 * WMT, T - t0,
+                            wn * 32 * WNT, BN, sp.part + (size_t)split_slot * BM * BN, BN,
+                            [](int bb, int rb) { return 32 * bb + 8 * rb; });
+        return;
+    }
+    if ((ldc & (out == kOutF32 ? 3 : 7)) == 0 && ((uintptr_t)c & 15) == 0) {
+        auto rows = [&](auto o) {
+            constexpr int OUT = decltype(o)::value;
+            store_rows<OUT>(acc, lds + wave * 32 * out_pitch<OUT, WNT>(), lane, t0 + wm * 32 * WMT, T,
+                            n0 + wn * 32 * WNT, N, c, ldc, [](int bb, int rb) { return 32 * bb + 8 * rb; });
+        };
+        if (out == kOutGLU) rows(std::integral_constant<int, kOutGLU>{});
+        else if (out == kOutBF16) rows(std::integral_constant<int, kOutBF16>{});
+        else rows(std::integral_constant<int, kOutF32>{});
         return;
     }
     const bool vec = (ldc & 3) == 0 && ((uintptr_t)c & (out == kOutF32 ? 15u : 7u)) == 0;
@@ -455,52 +445,6 @@ __global__ void __launch_bounds__(NTH) gemm_kernel(const uint4* __restrict__ q, 
         }
 }
 
-// Split tiles' partials -> outputs: one thread per (split tile, token row, 4 input columns; GLU: 4 gate columns and
-// the 4 up columns 8 to the right); the ks partials are added in split order (fixed order: the result does not depend
-// on timing), then the epilogue of the GEMM. Reads are 16 bytes a lane, consecutive lanes consecutive.
-template <int BM, int BN, bool GLU>
-__global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* __restrict__ part, int ks, int ndirect,
-                                                            int nsplit, int nbn, int T, int N, void* __restrict__ c,
-                                                            int ldc, int out) {
-    constexpr int CB = GLU ? BN / 8 : BN / 4;  // threads per row
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (size_t)nsplit * BM * CB) return;
-    const int st = (int)(idx / ((size_t)BM * CB)), r = (int)((idx / CB) % BM), cb = (int)(idx % CB);
-    const int tile = ndirect + st;
-    const int col = GLU ? 16 * (cb >> 1) + 4 * (cb & 1) : 4 * cb;
-    const int tok = (tile / nbn) * BM + r, n = (tile % nbn) * BN + col;
-    if (tok >= T || n >= N) return;
-    const float* p = part + ((size_t)st * ks * BM + r) * BN + col;
-    f32x4_v v{0.f, 0.f, 0.f, 0.f}, u{0.f, 0.f, 0.f, 0.f};
-    for (int z = 0; z < ks; z++, p += (size_t)BM * BN) {
-        const f32x4_v a = *reinterpret_cast<const f32x4_v*>(p);
-#pragma unroll
-        for (int j = 0; j < 4; j++) v[j] += a[j];
-        if constexpr (GLU) {
-            const f32x4_v b = *reinterpret_cast<const f32x4_v*>(p + 8);
-#pragma unroll
-            for (int j = 0; j < 4; j++) u[j] += b[j];
-        }
-    }
-    if constexpr (GLU) {
-        uint16_t* o = reinterpret_cast<uint16_t*>(c) + (size_t)tok * ldc + (n >> 4) * 8 + (n & 7);
-#pragma unroll
-        for (int j = 0; j < 4; j++) o[j] = f32_to_bf16(silu_f32(v[j]) * u[j]);
-    } else if (out == kOutBF16) {
-        uint16_t* o = reinterpret_cast<uint16_t*>(c) + (size_t)tok * ldc + n;
-        if (((ldc & 3) | ((uintptr_t)c & 7)) == 0) {
-            *reinterpret_cast<uint2*>(o) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; j++) o[j] = f32_to_bf16(v[j]);
-        }
-    } else {
-        float* o = reinterpret_cast<float*>(c) + (size_t)tok * ldc + n;
-#pragma unroll
-        for (int j = 0; j < 4; j++) o[j] = v[j];
-    }
-}
-
 // tile configurations: 0 = 256 tokens x 256 rows (WMT 4, WNT 2), 1 = 256 x 128 (4, 1), 2 = 128 x 256 (2, 2),
 // 3 = 128 x 128 (2, 1; two blocks per CU)
 constexpr int kNumCfg = 4;
@@ -523,8 +467,6 @@ struct CfgOf<3> {
     static constexpr int WMT = 2, WNT = 1;
 };
 
-constexpr int kMaxSplit = 16;
-
 struct GemmGeom {
     int nbn, nbt, ntiles, ndirect, nsplit, ks;
     size_t ws_bytes;
@@ -535,9 +477,6 @@ struct CfgDims {
 CfgDims cfg_dims(int cfg) {
     return CfgDims{cfg < 2 ? 256 : 128, (cfg & 1) ? 128 : 256, qe_num_cus() * (cfg == 3 ? 2 : 1)};
 }
-// the most partial-sum workspace a split may take: one 256 x 256 fp32 tile per CU (64 MB)
-size_t max_split_bytes() { return (size_t)qe_num_cus() * 256 * 256 * 4; }
-
 // tiles of configuration cfg and, for ks > 1, the split of the last partial round (stream-K): whole rounds of
 // tiles run directly, the remaining tiles (all of them when they do not fill one round) as ks K ranges; false when
 // that split does not apply (no partial round, fewer 128-k groups than ranges, too much workspace)
@@ -561,27 +500,31 @@ bool gemm_geom(int cfg, int n, int k, int t, int ks, GemmGeom& g) {
 }
 
 // Predicted time in us of a choice: the k steps of the fullest CU at a measured cost per step, which falls when only
-// part of the CUs run (clock, shared caches), plus the partial sums written and read again. Fitted to a sweep of
-// every (configuration, ks <= 16) on (n, k) from 1280 x 4224 to 34816 x 5120, t = 70..4000 (MI355X, fp16 scales;
-// 6 % rms): the choice below is within 8 % of the best measured one there for t >= 200, within 25 % for smaller t.
-double gemm_cost_us(int cfg, int n, int k, int t, const GemmGeom& g) {
-    static const double kFull[kNumCfg] = {1.754, 1.074, 1.107, 1.264};  // us per 64-k step, every slot filled
-    static const double kPart[kNumCfg] = {1.233, 0.777, 0.829, 0.678};  // few slots filled
+// part of the CUs run (clock, shared caches), plus the partial sums written and read again. Fitted to sweeps of every
+// (configuration, ks <= 16) on (n, k) from 1280 x 4224 to 34816 x 5120, t = 70..4000 (MI355X; INT4 26 shapes 5.4 % rms,
+// INT8 15 shapes 5.4 % rms, whose record transpose makes its steps longer): the lowest prediction is within 9 % of
+// the best measured choice at every one of them. What it replaces for shapes whose tiles leave CUs idle (256 x 128
+// tiles, one K range): 5120 x 17408, t = 200 (40 tiles) 240 -> 58 us with 20 tiles of 256 x 256 in 12 ranges;
+// 34816 x 5120 GLU, t = 200 (272 tiles, two rounds) 163 -> 108 us with the last 16 tiles in 10 ranges; 5120 x 17408,
+// t = 1000 272 -> 174 us; 2976 x 7936, t = 75 114 -> 22 us; INT8 1280 x 7168, t = 100 129 -> 22 us.
+double gemm_cost_us(bool w8, int cfg, int n, int k, int t, const GemmGeom& g) {
+    static const double kFull[2][kNumCfg] = {{1.652, 1.014, 1.027, 1.112}, {2.097, 1.360, 1.640, 1.451}};
+    static const double kPart[2][kNumCfg] = {{1.216, 0.797, 0.807, 0.649}, {1.704, 1.026, 1.318, 0.968}};
+    const double full_us = kFull[w8][cfg], part_us = kPart[w8][cfg];  // per 64-k step: every slot filled, few
     const CfgDims d = cfg_dims(cfg);
     auto phase = [&](int blocks, int steps) {
         const int full = blocks / d.slots, rem = blocks % d.slots;
-        double us = full * (steps * kFull[cfg] + 0.45);
+        double us = full * (steps * full_us + 1.2);
         if (rem) {
-            double u = (double)rem / d.slots;
-            if (cfg == 3) u = u < 0.5 ? 0.0 : 2.0 * u - 1.0;  // the share of CUs that hold a second block
-            us += steps * (u * kFull[cfg] + (1.0 - u) * kPart[cfg]) + 0.45;
+            const double u = cfg == 3 ? (2 * rem > d.slots ? 1.0 : 0.0) : (double)rem / d.slots;  // 3: two per CU
+            us += steps * (u * full_us + (1.0 - u) * part_us) + 1.2;
         }
         return us;
     };
-    double us = phase(g.ndirect, k / BK);
+    double us = 4.3 + phase(g.ndirect, k / BK);
     if (g.nsplit > 0) {
         us += phase(g.nsplit * g.ks, 2 * ((k / 128 + g.ks - 1) / g.ks));
-        us += 1.3 + 0.266e-6 * g.nsplit * g.ks * ((double)t / g.nbt) * d.BN * 4;
+        us += 4.0 + 0.245e-6 * g.nsplit * g.ks * ((double)t / g.nbt) * d.BN * 4;
     }
     return us;
 }
@@ -604,37 +547,29 @@ void launch_cfg(const uint4* q, const uint16_t* s, int n, int k, const uint16_t*
     sp.ks = g.ks;
     sp.part = part;
     const int per = (g.ndirect + 7) / 8;
-    const unsigned blocks = (unsigned)(8 * per + 8 * ((g.nsplit * g.ks + 7) / 8));
+    const unsigned blocks = (unsigned)(8 * per) + split_blocks(g.nsplit, g.ks);
     gemm_kernel<FMT, SDT, WMT, WNT><<<dim3(blocks), dim3(NTH), FMT == kFmtW4 ? C::kLdsW4 : 2 * C::kStage, st>>>(
         q, s, n, k, x, ldx, t, c, ldc, out, sdt, g.nbn, g.nbt, sp);
     HIP_CHECK(hipGetLastError());
     if (g.nsplit > 0) {
-        const bool glu = out == kOutGLU;
-        const size_t threads = (size_t)g.nsplit * C::BM * (C::BN / (glu ? 8 : 4));
-        const dim3 grid((unsigned)((threads + 255) / 256));
-        if (glu)
-            splitk_reduce_kernel<C::BM, C::BN, true><<<grid, dim3(256), 0, st>>>(part, g.ks, g.ndirect, g.nsplit,
-                                                                                 g.nbn, t, n, c, ldc, out);
-        else
-            splitk_reduce_kernel<C::BM, C::BN, false><<<grid, dim3(256), 0, st>>>(part, g.ks, g.ndirect, g.nsplit,
-                                                                                  g.nbn, t, n, c, ldc, out);
-        HIP_CHECK(hipGetLastError());
+        launch_splitk_reduce<C::BM, C::BN, 0>(part, g.ks, g.ndirect, g.nsplit, g.nbn, g.nbt, t, n, c, ldc, out, st);
     }
 }
 
 // untuned choice: 256 x 256 tiles when they fill the CUs at least once (else 256 x 128), with the last partial round
-// split in two K ranges when it is at most half full, unless the cost model puts another choice at least 5 % lower
+// split in two K ranges when it is at most half full, unless the cost model puts another choice at least 6 % lower
 // (its error; below that the larger tile stays). maxparts: the largest split allowed (0: any).
 // The last choices of a thread are kept: 64 cost evaluations take about as long as a launch.
-GemmChoice gemm_model_choice(int n, int k, int t, int maxparts) {
+GemmChoice gemm_model_choice(bool w8, int n, int k, int t, int maxparts) {
     const int cus = qe_num_cus();
     struct Kept {
         int n = 0, k = 0, t = 0, maxparts = 0, cus = 0;
+        bool w8 = false;
         GemmChoice ch;
     };
     static thread_local Kept kept[64];
     Kept& slot = kept[((unsigned)n * 31u + (unsigned)k * 17u + (unsigned)t * 7u + (unsigned)maxparts) >> 4 & 63u];
-    if (slot.n == n && slot.k == k && slot.t == t && slot.maxparts == maxparts && slot.cus == cus) return slot.ch;
+    if (slot.n == n && slot.k == k && slot.t == t && slot.maxparts == maxparts && slot.cus == cus && slot.w8 == w8) return slot.ch;
     const long tiles_big = (long)((n + 255) / 256) * ((t + 255) / 256);
     GemmChoice ch{tiles_big >= cus ? 0 : 1, 1};
     GemmGeom g;
@@ -644,18 +579,18 @@ GemmChoice gemm_model_choice(int n, int k, int t, int maxparts) {
         if ((double)tiles_big / (rounds * cus) < 0.9) ch.cfg = 1;
     }
     gemm_geom(ch.cfg, n, k, t, ch.ks, g);
-    const double base = gemm_cost_us(ch.cfg, n, k, t, g);
-    double best = 0.95 * base;
+    const double base = gemm_cost_us(w8, ch.cfg, n, k, t, g);
+    double best = 0.94 * base;
     for (int cfg = 0; cfg < kNumCfg; cfg++)
         for (int ks = 1; ks <= kMaxSplit && (maxparts <= 0 || ks <= maxparts); ks++) {
             if (!gemm_geom(cfg, n, k, t, ks, g)) continue;
-            const double us = gemm_cost_us(cfg, n, k, t, g);
+            const double us = gemm_cost_us(w8, cfg, n, k, t, g);
             if (us < best) {
                 best = us;
                 ch = GemmChoice{cfg, ks};
             }
         }
-    slot = Kept{n, k, t, maxparts, cus, ch};
+    slot = Kept{n, k, t, maxparts, cus, w8, ch};
     return ch;
 }
 
@@ -669,7 +604,7 @@ void run_choice(int cfg, int ks, const uint4* q, const uint16_t* s, int n, int k
         if (!gemm_geom(cfg, n, k, t, ks, g)) ks = 1;
         else if ((part = static_cast<float*>(stream_ws(kWsSplit, g.ws_bytes, st))) == nullptr) {
             ks = 1;
-            cfg = gemm_model_choice(n, k, t, 1).cfg;
+            cfg = gemm_model_choice(FMT != kFmtW4, n, k, t, 1).cfg;
         }
     }
     if (ks == 1) gemm_geom(cfg, n, k, t, 1, g);
@@ -690,7 +625,7 @@ GemmChoice gemm_tune_choice(int n, int k, const uint16_t* x, int ldx, int t, voi
     for (int cfg = 0; cfg < kNumCfg; cfg++)
         for (int ks = 1; ks <= kMaxSplit; ks++) {
             GemmGeom g;
-            if (gemm_geom(cfg, n, k, t, ks, g)) all.emplace_back(gemm_cost_us(cfg, n, k, t, g), GemmChoice{cfg, ks});
+            if (gemm_geom(cfg, n, k, t, ks, g)) all.emplace_back(gemm_cost_us(FMT != kFmtW4, cfg, n, k, t, g), GemmChoice{cfg, ks});
         }
     std::stable_sort(all.begin(), all.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
     for (size_t i = 0; i < all.size(); i++) {
@@ -750,7 +685,7 @@ void launch_gemm(const uint4* q, const uint16_t* s, int n, int k, const uint16_t
             ch = gemm_tune_choice<FMT, SDT>(n, k, x, ldx, t, c, ldc, out, sdt, q, s, st);
             gemm_table_add(key, ch);
         } else {
-            ch = gemm_model_choice(n, k, t, gemm_sk_maxparts());
+            ch = gemm_model_choice(FMT != kFmtW4, n, k, t, gemm_sk_maxparts());
         }
     }
     run_choice<FMT, SDT>(ch.cfg, capped_split(ch.ks), q, s, n, k, x, ldx, t, c, ldc, out, sdt, st);

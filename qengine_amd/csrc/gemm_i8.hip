@@ -22,7 +22,7 @@
 // order k0, k0 + 8, k0 + 1, k0 + 9 (k0 = 2 t, words t = 0..3); the pre-pass stores the activations in that same
 // order, so the dot products pair matching k (the same permutation as the reference's pre-pass, forced by the
 // W4 layout).
-#include "mfma_tile.hpp"
+#include "gemm_split.hpp"
 
 #include <mutex>
 #include <type_traits>
@@ -41,7 +41,6 @@ constexpr int kRaw = BN * 64;                // two 64-k W4 chunks of BN / 16 ti
 constexpr int kSc = BN * 2;                  // [BN / 16][16] weight scales of one group
 constexpr int kSx = BM * 4 * 4;              // [BM][128 / G] activation scales, G >= 32
 constexpr int kLds = 2 * kStage + 2 * kRaw + 2 * kSc + 2 * kSx;
-enum Out : int { kOutF32 = 0, kOutBF16 = 1, kOutGLU = 2 };
 constexpr int kColGroup = 4;  // weight-column tiles per group of the tile order
 
 // byte p of a 16-k block holds k offset kPerm(p) = 2 (p / 4) + {0, 8, 1, 9}[p % 4]
@@ -155,8 +154,6 @@ __global__ void __launch_bounds__(256) x_to_r8_kernel(const uint16_t* __restrict
     if ((j & 3) == 0) sx[(size_t)t * (K / 128) + (j >> 2)] = sc;
 }
 
-// 4 nibbles u (one per byte) -> 4 signed bytes u - 8
-__device__ __forceinline__ uint32_t nib_s8(uint32_t u) { return ((u | 0x80808080u) - 0x08080808u) ^ 0x80808080u; }
 
 // Weight formats (WF):
 // kW4: W4 records, raw chunks by DMA two steps ahead, unpacked to signed int8 between the MFMA rows.
@@ -174,7 +171,7 @@ __device__ __forceinline__ uint32_t nib_s8(uint32_t u) { return ((u | 0x80808080
 //   the same rn(sum sx)), so the result is fixed to the bit.
 enum Wf : int { kW4 = 0, kQ8 = 1, kW8 = 2 };
 
-// Every group's int32 sums start at the bit pattern of M = 1.5 * 2^23: |sum| < 2^22 (at most 128 * 127 * 127), so the
+// Every group's int32 sums start at the bit pattern of M = 1.5 * 2^23: |sum| < 2^22 (at most 128 * 128 * 127), so the
 // accumulator read as fp32 is M + sum exactly, and fma(M + sum, sx, -M sx) = rn(sum * sx) (M sx is exact, sx having 22
 // significant bits): the flush costs 2 VALU per output instead of convert, multiply and fma
 constexpr float kMagicF = 12582912.f;
@@ -186,7 +183,7 @@ template <int G, int SDT, int OUT, int WF, bool PC>
 __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ q, const uint16_t* __restrict__ s,
                                                       int N, int K, const int8_t* __restrict__ xq,
                                                       const float* __restrict__ sxg, int T, void* __restrict__ c,
-                                                      int ldc, int nbn, int ntiles) {
+                                                      int ldc, int nbn, int ntiles, SplitArgs sp) {
     constexpr int NGS = BK / G;   // activation groups per step
     constexpr int KPG = G / 32;   // k32 MFMA steps per activation group
     static_assert(WF != kW8 || G == 128, "W8A8: activation groups of 128");
@@ -195,22 +192,28 @@ __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned lds32 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)lds);
-    const int per = (ntiles + 7) >> 3, b = blockIdx.x;
-    const int tile = (b & 7) * per + (b >> 3);
-    if (tile >= ntiles) return;
+    const int ndirect = min(sp.ndirect, ntiles), per = (ndirect + 7) >> 3, b = blockIdx.x;
+    int tile, kt0 = 0, KT = K / BK;  // this block's 128-k steps [kt0, kt0 + KT)
+    int split_slot = -1;             // >= 0: a split tile's part, stored raw to sp.part
+    if (b < 8 * per) {
+        tile = (b & 7) * per + (b >> 3);
+        if (tile >= ndirect) return;
+    } else {
+        int ts, z;
+        if (!split_item(b - 8 * per, ntiles - ndirect, sp.ks, ts, z)) return;
+        tile = ndirect + ts;
+        kt0 = z * (K / BK) / sp.ks;
+        KT = (z + 1) * (K / BK) / sp.ks - kt0;
+        split_slot = ts * sp.ks + z;
+    }
     // tile order: groups of kColGroup weight-column tiles, token blocks outer and columns inner within a group; each
     // XCD takes a contiguous run of it (blocks b, b + 8, .. run on XCD b % 8), so its 32 resident tiles are 8 token
     // blocks x 4 columns: per step 8 X slices (16 KB) and 4 W slices (32 KB) through its L2 instead of 1 X slice and
     // 32 W slices (4x the HBM fetch: each W tile re-read per token block)
     int tb, cb;
-    {
-        const int nbt = ntiles / nbn, full = nbn / kColGroup, cg = tile / (nbt * kColGroup);
-        const int w = cg < full ? kColGroup : nbn - full * kColGroup, r = tile - cg * nbt * kColGroup;
-        tb = r / w;
-        cb = cg * kColGroup + r % w;
-    }
+    tile_place<kColGroup>(tile, nbn, ntiles / nbn, tb, cb);
     const int n0 = cb * BN, t0 = tb * BM;
-    const int G128 = K >> 7, KT = K / BK;
+    const int G128 = K >> 7;
     const int ntile_last = (N >> 4) - 1;
 
     auto dma_x = [&](int kt, unsigned xt) {  // 8 rows of 128 B per wave instruction
@@ -281,7 +284,8 @@ __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ 
 
     // two stages of X, W and the scales in LDS (a third, the DMA two steps ahead, measured slower for kW8)
     constexpr unsigned kRawOff = 2 * kStage, kScOff = kRawOff + 2 * kRaw, kSxOff = kScOff + 2 * kSc;
-    auto dma_step = [&](int kk, int slot) {  // X, the Q8 / W8 tile and the scales of step kk into stage slot
+    auto dma_step = [&](int kl, int slot) {  // X, the Q8 / W8 tile and the scales of local step kl into stage slot
+        const int kk = kt0 + kl;
         dma_x(kk, slot * kStage);
         if constexpr (WF == kQ8) dma_wq8(kk, slot * kStage + BM * BK);
         if constexpr (WF == kW8) dma_w8(kk, slot * kStage + BM * BK);
@@ -323,8 +327,10 @@ __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ 
     // (row jtr * 16 + jg + 8 h, 16-k block 4 ch + jj) is stored
     uint32_t wd[2][4], ob[4];
     auto unit = [&](char* wtile, int ch, int h, int t) {
-        const uint32_t u = (h ? wd[ch][t] >> 4 : wd[ch][t]) & nib_mask();
-        ob[t] = nib_s8(u);
+        // bytes 16 (u - 8): u ^ 8 is u - 8 as a signed nibble, kept in the byte's high half (4 VALU a word instead of
+        // 9); the sums are 16 times those of u - 8 and sx / 16 takes the factor out. With the activation scales read
+        // at the top of the step: 17408 x 5120, t = 2048, G = 64 401 -> 377 us
+        ob[t] = (h ? wd[ch][t] : wd[ch][t] << 4) & nib_mask_hi();
         if (t == 3) {
             const int row = jtr * 16 + jg + 8 * h;
             *reinterpret_cast<u32x4_v*>(wtile + swz(row, 4 * ch + jj)) = u32x4_v{ob[0], ob[1], ob[2], ob[3]};
@@ -336,14 +342,14 @@ __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ 
             const uint32_t* rw = reinterpret_cast<const uint32_t*>(rawb + ch * BN * 32 + (jtr >> 1) * 1024) +
                                  (8 * (jtr & 1) + jg) * 4 + jj;
 #pragma unroll
-            for (int t = 0; t < 4; t++) wd[ch][t] = rw[64 * t];
+            for (int t = 0; t < 4; t++) wd[ch][t] = rw[64 * t] ^ 0x88888888u;
         }
     };
 
     dma_step(0, 0);
     if constexpr (WF == kW4) {
-        dma_w4(0, kRawOff);
-        if (KT > 1) dma_w4(1, kRawOff + kRaw);
+        dma_w4(kt0, kRawOff);
+        if (KT > 1) dma_w4(kt0 + 1, kRawOff + kRaw);
     }
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     if constexpr (WF == kW4) {
@@ -357,16 +363,60 @@ __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ 
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
 
+    // weight scales of this lane's rows (4 consecutive rows per register quad, one 8-byte read) from a scale buffer
+    auto load_sw = [&](float (&dst)[WNT][16], int slot) {
+        const uint16_t* scb = reinterpret_cast<const uint16_t*>(lds + kScOff + slot * kSc);
+#pragma unroll
+        for (int bb = 0; bb < WNT; bb++)
+#pragma unroll
+            for (int rq = 0; rq < 4; rq++) {
+                const uint2 sp = *reinterpret_cast<const uint2*>(scb + wrow(bb, rq) + 4 * (lane >> 5));
+                dst[bb][4 * rq] = scale_to_f32<SDT>((uint16_t)(sp.x & 0xFFFFu));
+                dst[bb][4 * rq + 1] = scale_to_f32<SDT>((uint16_t)(sp.x >> 16));
+                dst[bb][4 * rq + 2] = scale_to_f32<SDT>((uint16_t)(sp.y & 0xFFFFu));
+                dst[bb][4 * rq + 3] = scale_to_f32<SDT>((uint16_t)(sp.y >> 16));
+            }
+    };
+    // activation scales of the step: this lane's token of each MFMA tile, every group
+    float sxv[WMT][NGS];
+    auto load_sx = [&](int slot) {
+        const float* sxb = reinterpret_cast<const float*>(lds + kSxOff + slot * kSx);
+#pragma unroll
+        for (int a = 0; a < WMT; a++)
+#pragma unroll
+            for (int gi = 0; gi < NGS; gi++) sxv[a][gi] = sxb[(wm * 32 * WMT + a * 32 + (lane & 31)) * NGS + gi];
+    };
+    // flush activation group gi of the step whose activation scales are in sxv: acc += (float(sum) * sx) * sw
+    auto flush = [&](int gi, const float (&swf)[WNT][16]) {
+#pragma unroll
+        for (int a = 0; a < WMT; a++) {
+            // kW4: the operand bytes are 16 (u - 8), the 1 / 16 goes into sx (a power of two: the same rounding)
+            const float sxa = sxv[a][gi] * (WF == kW4 ? 0.0625f : 1.f);
+            const float msx = -kMagicF * sxa;  // exact: sx has 22 significant bits
+#pragma unroll
+            for (int bb = 0; bb < WNT; bb++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    // copied to a scalar first: hipcc lowers a bit_cast of an ext_vector element as element 0
+                    const int d = dsum[a][bb][r];
+                    acc[a][bb][r] = fmaf(fmaf(__builtin_bit_cast(float, d), sxa, msx), swf[bb][r], acc[a][bb][r]);
+                    if (NGS == 4 && (r & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // G = 32: bounds the live temporaries
+                }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
     // step kt: DMA X (kt + 1), the raw W, weight scales and activation scales of kt + 1 / kt + 2; MFMAs of step kt
     // with the unpack of step kt + 1 (two units after each MFMA row); each activation group's sums flushed after its
-    // last k32 step: acc += float(sum) * sx * sw
+    // last k32 step: acc += float(sum) * sx * sw. (Flushing the last group of waves 4..7 at the top of the next step, so
+    // that one wave of a SIMD flushes while the other's MFMAs run, changed nothing for W8A8 and cost W4A8 6 %.)
     auto kstep = [&](int kt, auto more) {
         constexpr bool MORE = decltype(more)::value;
         char* wnext = lds + ((kt + 1) & 1) * kStage + BM * BK;
         const int cur = kt & 1;
         if (MORE) dma_step(kt + 1, (kt + 1) & 1);
         if constexpr (WF == kW4) {
-            if (kt + 2 < KT) dma_w4(kt + 2, kRawOff + (kt & 1) * kRaw);
+            if (kt + 2 < KT) dma_w4(kt0 + kt + 2, kRawOff + (kt & 1) * kRaw);
         }
         const char* xt = lds + cur * kStage;
         const char* wt = xt + BM * BK;
@@ -399,34 +449,12 @@ __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ 
                     bfr[buf][1][2 * e + kb] = (int)__builtin_amdgcn_perm(d1, d0, 0x07060302u);
                 }
         };
+        float swf[WNT][16];
         read_frags(0, 0);
+        load_sx(cur);
         if constexpr (WF == kW8) split_rows(0);
         if constexpr (MORE && WF == kW4) read_words(lds + kRawOff + ((kt + 1) & 1) * kRaw);
-        // weight scales of this lane's rows (4 consecutive rows per register quad, one 8-byte read) for the step
-        const uint16_t* scb = reinterpret_cast<const uint16_t*>(lds + kScOff + cur * kSc);
-        const float* sxb = reinterpret_cast<const float*>(lds + kSxOff + cur * kSx);
-        float swf[WNT][16];
-        auto load_sw = [&](float (&dst)[WNT][16]) {
-#pragma unroll
-            for (int bb = 0; bb < WNT; bb++)
-#pragma unroll
-                for (int rq = 0; rq < 4; rq++) {
-                    const uint2 sp = *reinterpret_cast<const uint2*>(scb + wrow(bb, rq) + 4 * (lane >> 5));
-                    dst[bb][4 * rq] = scale_to_f32<SDT>((uint16_t)(sp.x & 0xFFFFu));
-                    dst[bb][4 * rq + 1] = scale_to_f32<SDT>((uint16_t)(sp.x >> 16));
-                    dst[bb][4 * rq + 2] = scale_to_f32<SDT>((uint16_t)(sp.y & 0xFFFFu));
-                    dst[bb][4 * rq + 3] = scale_to_f32<SDT>((uint16_t)(sp.y >> 16));
-                }
-        };
-        if constexpr (PC) {
-            if (kt == 0) load_sw(swf_pc);
-#pragma unroll
-            for (int bb = 0; bb < WNT; bb++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) swf[bb][r] = swf_pc[bb][r];
-        } else {
-            load_sw(swf);
-        }
+        if constexpr (!PC) load_sw(swf, cur);
         __builtin_amdgcn_sched_barrier(0);
         int slot = 0;
 #pragma unroll
@@ -452,31 +480,33 @@ __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ 
                 slot++;
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (ks % KPG == KPG - 1) {  // flush activation group ks / KPG: acc += (float(sum) * sx) * sw
-                const int gi = ks / KPG;
-#pragma unroll
-                for (int a = 0; a < WMT; a++) {
-                    const float sxa = sxb[(wm * 32 * WMT + a * 32 + (lane & 31)) * NGS + gi];
-                    const float msx = -kMagicF * sxa;  // exact: sx has 22 significant bits
-#pragma unroll
-                    for (int bb = 0; bb < WNT; bb++)
-#pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            // copied to a scalar first: hipcc lowers a bit_cast of an ext_vector element as element 0
-                            const int d = dsum[a][bb][r];
-                            acc[a][bb][r] = fmaf(fmaf(__builtin_bit_cast(float, d), sxa, msx), swf[bb][r], acc[a][bb][r]);
-                        }
-                }
-                __builtin_amdgcn_sched_barrier(0);
+            if (ks % KPG == KPG - 1) {
+                if constexpr (PC) flush(ks / KPG, swf_pc);
+                else flush(ks / KPG, swf);
             }
         }
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     };
     static_assert((BK / 32) * WMT * 2 == 16, "16 unpack units per step, two per MFMA row");
+    if constexpr (PC) load_sw(swf_pc, 0);
     for (int kt = 0; kt + 1 < KT; kt++) kstep(kt, std::true_type{});
     kstep(KT - 1, std::false_type{});
 
     // epilogue: lane = token l % 32, register r = weight row 8 (r / 4) + 4 (l / 32) + r % 4 of its tile
+    auto lcol = [&](int bb, int rq) { return wrow(bb, rq) - wn * 32 * WNT; };  // of the wave's columns
+    if constexpr (WF != kW8) {
+        if (split_slot >= 0) {
+            store_rows<kOutF32>(acc, lds + wave * 32 * out_pitch<kOutF32, WNT>(), lane, wm * 32 * WMT, T - t0, wn * 32 * WNT,
+                                BN, sp.part + (size_t)split_slot * BM * BN, BN, lcol);
+            return;
+        }
+    }
+    if ((ldc & (OUT == kOutF32 ? 3 : 7)) == 0 && ((uintptr_t)c & 15) == 0) {
+        static_assert(NTH / 64 * 32 * out_pitch<kOutF32, WNT>() <= 2 * kStage, "one buffer per wave in the X / W stages");
+        store_rows<OUT>(acc, lds + wave * 32 * out_pitch<OUT, WNT>(), lane, t0 + wm * 32 * WMT, T, n0 + wn * 32 * WNT, N,
+                        c, ldc, lcol);
+        return;
+    }
     const int cj = lane & 31, ci = 4 * (lane >> 5);
     const bool vec = ((ldc & 3) == 0 && ((uintptr_t)c & (OUT == kOutF32 ? 15u : 7u)) == 0);
 #pragma unroll
@@ -538,6 +568,30 @@ void* i8_ws(size_t bytes, hipStream_t st) {
 size_t xq_bytes(int k, int t) { return ((size_t)t * k + 255) / 256 * 256; }
 size_t i8_ws_bytes(int k, int t) { return xq_bytes(k, t) + (size_t)t * (k / 32) * 4; }  // sx sized for G = 32
 
+// K ranges of the last partial round's tiles (W4A8 and the Q8 W8A8; the W8-layout W8A8 keeps its groups in one
+// chain: its result is fixed to the bit): the fewest us of rounds of steps, plus the partials written and read again.
+// us per 128-k step of a full round: 17408 x 5120, t = 2048 (4.25 rounds of 40 steps) unsplit 343 / 412 / 748 us for
+// G = 128 / 64 / 32, with the last 64 tiles split 290 / 358 / 578; partials 0.27 us per MB as in the bf16 GEMM.
+// 5120 x 17408, t = 300, G = 64 (60 tiles on 256 CUs): 239 -> 77 us.
+int i8_split(int ntiles, int kt, int G, double rows) {
+    const int cus = qe_num_cus(), tail = ntiles % cus;
+    if (tail == 0) return 1;
+    const double step = G == 128 ? 1.3 : G == 64 ? 1.9 : 2.9;
+    int best = 1;
+    double best_us = kt * step;
+    const int cap = gemm_sk_maxparts() > 0 ? min(gemm_sk_maxparts(), kMaxSplit) : kMaxSplit;
+    for (int ks = 2; ks <= cap && ks <= kt; ks++) {
+        if ((size_t)tail * ks * BM * BN * 4 > max_split_bytes()) break;
+        const int rounds = (tail * ks + cus - 1) / cus, steps = (kt + ks - 1) / ks;
+        const double us = rounds * (steps * step + 2.0) + 4.0 + 0.27e-6 * tail * ks * rows * BN * 4;
+        if (us < best_us) {
+            best_us = us;
+            best = ks;
+        }
+    }
+    return best;
+}
+
 template <int G, int WF>
 void run_i8(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, int out, hipStream_t st) {
     char* ws = static_cast<char*>(i8_ws(i8_ws_bytes(w.k, t), st));
@@ -548,10 +602,18 @@ void run_i8(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, in
     else x_to_i8_kernel<G, false><<<dim3(pb), dim3(256), 0, st>>>(x, ldx, w.k, t, xq, sx);
     HIP_CHECK(hipGetLastError());
     const int nbn = (w.n + BN - 1) / BN, nbt = (t + BM - 1) / BM, ntiles = nbn * nbt;
-    const unsigned blocks = (unsigned)(8 * ((ntiles + 7) / 8));
+    SplitArgs sp;
+    sp.ks = i8_split(ntiles, w.k / BK, G, (double)t / nbt);
+    const int nsplit = sp.ks > 1 ? ntiles % qe_num_cus() : 0;
+    if (nsplit > 0) {
+        sp.part = static_cast<float*>(stream_ws(kWsSplit, (size_t)nsplit * sp.ks * BM * BN * 4, st));
+        if (sp.part) sp.ndirect = ntiles - nsplit;  // (none during a capture that was not warmed up: unsplit)
+    }
+    const unsigned blocks = 8u * (unsigned)((min(sp.ndirect, ntiles) + 7) / 8) +
+                            (sp.part ? split_blocks(nsplit, sp.ks) : 0u);
 #define QE_GI(SDT_, OUT_)                                                                                            \
     gemm_i8_kernel<G, SDT_, OUT_, WF, false><<<dim3(blocks), dim3(NTH), kLds, st>>>(w.q, w.s, w.n, w.k, xq, sx, t, c, ldc, nbn, \
-                                                                          ntiles)
+                                                                          ntiles, sp)
     if (w.sdt == kScaleF16) {
         if (out == kOutGLU) QE_GI(kScaleF16, kOutGLU);
         else if (out == kOutBF16) QE_GI(kScaleF16, kOutBF16);
@@ -563,6 +625,7 @@ void run_i8(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, in
     }
 #undef QE_GI
     HIP_CHECK(hipGetLastError());
+    if (sp.part) launch_splitk_reduce<BM, BN, kColGroup>(sp.part, sp.ks, sp.ndirect, nsplit, nbn, nbt, t, w.n, c, ldc, out, st);
 }
 
 template <int SDT, bool PC>
@@ -571,10 +634,10 @@ void run_w8a8(const W8& w, const int8_t* xq, const float* sx, void* c, int ldc, 
     const unsigned blocks = (unsigned)(8 * ((ntiles + 7) / 8));
     if (out_bf16)
         gemm_i8_kernel<128, SDT, kOutBF16, kW8, PC><<<dim3(blocks), dim3(NTH), kLds, st>>>(w.q, w.s, w.n, w.k, xq, sx, t,
-                                                                                        c, ldc, nbn, ntiles);
+                                                                                        c, ldc, nbn, ntiles, SplitArgs{});
     else
         gemm_i8_kernel<128, SDT, kOutF32, kW8, PC><<<dim3(blocks), dim3(NTH), kLds, st>>>(w.q, w.s, w.n, w.k, xq, sx, t,
-                                                                                       c, ldc, nbn, ntiles);
+                                                                                       c, ldc, nbn, ntiles, SplitArgs{});
 }
 
 }  // namespace

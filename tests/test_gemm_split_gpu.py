@@ -96,3 +96,44 @@ def test_tune_file_with_two_tile_shapes(dev, tmp_path):
     finally:
         call("qe_gemm_tune_file", ctypes.c_char_p(b""))
         call("qe_gemm_tune_clear")
+
+
+@pytest.mark.parametrize("n,k,t,G", [(272, 1152, 65, 64), (1040, 2176, 129, 32), (4112, 1152, 300, 128), (144, 128, 70, 64)])
+@pytest.mark.parametrize("glu", [False, True])
+def test_underfilled_w4a8(dev, n, k, t, G, glu):
+    """W4A8 tiles split in uneven K ranges: the oracle's INT8 product to 1e-5 relative rms; rows stored through LDS
+    (aligned) and one by one (an odd offset and stride) are the same bits"""
+    w, q, s = setup(n, k, 1, seed=n + G, glu=glu)
+    xh = synth.x_host(t, k, seed=t + 1)
+    x = synth.to_dev(xh)
+    xq, sx = oracle.x_to_i8(xh, G)
+    ref = oracle.gemm_i8(xq, sx, oracle.unpack_w4(q, n, k), oracle.f16_to_f32(s).reshape(n, k // 128), G)
+    y = ops.gemm_w4_i8(w, x, G=G, out_bf16=True)
+    cols = n // 2 if glu else n
+    if glu:
+        assert_glu_close(out_f32(y), glu_act(ref), 1e-4)
+    else:
+        y32 = out_f32(ops.gemm_w4_i8(w, x, G=G)).astype(np.float64)
+        assert np.sqrt(np.mean((y32 - ref) ** 2) / np.mean(ref ** 2)) < 1e-5
+    big = torch.full((t, cols + 7), float("nan"), dtype=torch.bfloat16, device=dev)
+    got = ops.gemm_w4_i8(w, x, G=G, out_bf16=True, y=big[:, 1:1 + cols])
+    assert torch.equal(got.contiguous().view(torch.int16), y.view(torch.int16))
+    assert torch.isnan(big[:, 0]).all() and torch.isnan(big[:, 1 + cols:]).all()
+
+
+@pytest.mark.parametrize("n,t,out_bf16", [(272, 65, True), (272, 300, False), (528, 129, True)])
+def test_w8a8_row_stores(dev, n, t, out_bf16):
+    """W8A8 rows stored through LDS (16-byte aligned) and one by one (odd offset and stride): the same bits, and
+    nothing outside the matrix"""
+    k = 1024
+    q, s = synth.w8_host(n, k, seed=n, per_channel=True)
+    w = ops.tile_w8(synth.to_dev(q), synth.to_dev(s, torch.float16), True)
+    x = synth.to_dev(synth.x_host(t, k, seed=t))
+    dt, iv = (torch.bfloat16, torch.int16) if out_bf16 else (torch.float32, torch.int32)
+    wide = torch.full((t + 1, n + 16), float("nan"), dtype=dt, device=dev)
+    y = ops.gemm_w8a8(w, x, out_bf16=out_bf16, y=wide[:t, :n])
+    odd = torch.full((t, n + 7), float("nan"), dtype=dt, device=dev)
+    z = ops.gemm_w8a8(w, x, out_bf16=out_bf16, y=odd[:, 1:1 + n])
+    assert torch.equal(y.contiguous().view(iv), z.contiguous().view(iv))
+    assert torch.isnan(wide[t]).all() and torch.isnan(wide[:, n:]).all()
+    assert torch.isnan(odd[:, 0]).all() and torch.isnan(odd[:, 1 + n:]).all()
