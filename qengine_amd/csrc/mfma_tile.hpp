@@ -72,29 +72,48 @@ __device__ __forceinline__ void dma4(const void* src, unsigned lds_dst) {  // 4 
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_dst), "v"(src) : "memory", "m0");
 }
 
-// Output of a wave's WMT x WNT MFMA tiles held as C^T (lane l: token l % 32 of a tile, registers 4 rb .. 4 rb + 3 the
-// output columns col(bb, rb) + 4 (l / 32) + 0..3 of the wave's 32 WNT) through a wave-private LDS buffer: one 32-token
-// tile row at a time is written as it lies and read back as whole rows, so that a store instruction writes
-// 32 WNT x esz contiguous bytes a token (128 or 256 B) instead of 16 or 32 B of each of 32 tokens. Stored straight
-// from the registers the W8A8 GEMM (8192 x 2048, t = 4096, fp32) spent 51 of its 163 us on its 134 MB of output.
-// OUT: 0 fp32, 1 bf16, 2 GLU (gate rows rb, up rows rb + 1: half the columns). buf: 32 x out_pitch bytes. Needs c and
-// the row stride 16-byte aligned; N % 16 == 0, so a 16-byte chunk never straddles the last column.
+// Output of a wave's MFMA tiles held as C^T (lane l: token l % 32 of a 32-token tile, registers of 4 consecutive output
+// columns) through a wave-private LDS buffer: one 32-token tile at a time is written as it lies and read back as whole
+// rows, so that a store instruction writes NC ESZ contiguous bytes a token (64 to 256 B) instead of 8 to 32 B of each
+// of 32 tokens. Stored straight from the registers the W8A8 GEMM (8192 x 2048, t = 4096, fp32) spent 51 of its 163 us
+// on its 134 MB of output. write(a, row): token tile a of this lane into its row of the buffer (NC columns of ESZ
+// bytes); buf: 32 rows of out_pitch bytes; c: element (tok0, n0), 16-byte aligned as ldc is; the NC columns end at
+// ncols, a multiple of 16 / ESZ, so a 16-byte chunk never straddles the last column.
+template <int ESZ, int NC>
+constexpr int out_pitch_of() { return NC * ESZ + 16; }
+template <int ESZ, int NC, int NTILES, class Write>
+__device__ __forceinline__ void store_tile_rows(char* buf, int lane, int ntok, int ncols, void* c, int ldc, Write write) {
+    constexpr int PITCH = out_pitch_of<ESZ, NC>();
+    constexpr int LPR = NC * ESZ / 16, RPI = 64 / LPR;  // lanes per row, rows per store instruction
+    const int rr = lane / LPR, ch = lane % LPR;
+    const bool nok = ch * (16 / ESZ) < ncols;
+    char* o = reinterpret_cast<char*>(c) + ((size_t)rr * ldc) * ESZ + ch * 16;
+#pragma unroll
+    for (int a = 0; a < NTILES; a++) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        write(a, buf + (lane & 31) * PITCH);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int i = 0; i < 32 / RPI; i++) {
+            const int row = a * 32 + i * RPI;
+            const u32x4_v v = *reinterpret_cast<const u32x4_v*>(buf + (i * RPI + rr) * PITCH + ch * 16);
+            if (nok && row + rr < ntok) *reinterpret_cast<u32x4_v*>(o + (size_t)row * ldc * ESZ) = v;
+        }
+    }
+}
+
+// the same for a wave's WMT x WNT tiles of a GEMM: registers 4 rb .. 4 rb + 3 of acc[a][bb] are columns
+// col(bb, rb) + 4 (l / 32) + 0..3 of the wave's 32 WNT from n0 on. OUT: 0 fp32, 1 bf16, 2 GLU (gate rows rb, up rows
+// rb + 1: half the columns); N % 16 == 0
 template <int OUT, int WNT>
-constexpr int out_pitch() { return (OUT == 0 ? 128 : OUT == 1 ? 64 : 32) * WNT + 16; }
+constexpr int out_pitch() { return out_pitch_of<OUT == 0 ? 4 : 2, (OUT == 2 ? 16 : 32) * WNT>(); }
 template <int OUT, int WMT, int WNT, class Col>
 __device__ __forceinline__ void store_rows(const f32x16_v (&acc)[WMT][WNT], char* buf, int lane, int tok0, int T, int n0,
                                            int N, void* c, int ldc, Col col) {
-    constexpr int ESZ = OUT == 0 ? 4 : 2, NC = (OUT == 2 ? 16 : 32) * WNT, PITCH = out_pitch<OUT, WNT>();
-    constexpr int LPR = NC * ESZ / 16, RPI = 64 / LPR;  // lanes per row, rows per store instruction
-    const int h4 = 4 * (lane >> 5);
-    char* wr = buf + (lane & 31) * PITCH;
-    const int rr = lane / LPR, ch = lane % LPR;
-    const int nc = (OUT == 2 ? n0 >> 1 : n0) + ch * (16 / ESZ);  // first output column of this lane's chunks
-    const bool nok = nc < (OUT == 2 ? N >> 1 : N);
-    char* o = reinterpret_cast<char*>(c) + ((size_t)(tok0 + rr) * ldc + nc) * ESZ;
-#pragma unroll
-    for (int a = 0; a < WMT; a++) {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    constexpr int ESZ = OUT == 0 ? 4 : 2, NC = (OUT == 2 ? 16 : 32) * WNT;
+    const int h4 = 4 * (lane >> 5), nc0 = OUT == 2 ? n0 >> 1 : n0;
+    char* o = reinterpret_cast<char*>(c) + ((size_t)tok0 * ldc + nc0) * ESZ;
+    store_tile_rows<ESZ, NC, WMT>(buf, lane, T - tok0, (OUT == 2 ? N >> 1 : N) - nc0, o, ldc, [&](int a, char* wr) {
 #pragma unroll
         for (int bb = 0; bb < WNT; bb++)
 #pragma unroll
@@ -115,14 +134,7 @@ __device__ __forceinline__ void store_rows(const f32x16_v (&acc)[WMT][WNT], char
                         uint2{pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3])};
                 }
             }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-        for (int i = 0; i < 32 / RPI; i++) {
-            const int row = a * 32 + i * RPI;
-            const u32x4_v v = *reinterpret_cast<const u32x4_v*>(buf + (i * RPI + rr) * PITCH + ch * 16);
-            if (nok && tok0 + row + rr < T) *reinterpret_cast<u32x4_v*>(o + (size_t)row * ldc * ESZ) = v;
-        }
-    }
+    });
 }
 
 // 32x32 MFMA C fragment: lane l holds column l % 32, rows 8 (r / 4) + 4 (l / 32) + r % 4 for r = 0..15

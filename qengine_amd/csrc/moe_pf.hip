@@ -54,7 +54,6 @@ __device__ __forceinline__ void rw_body(const MoePfArgs& ma, char* lds, int nt, 
     const bool wact = wrow < N;            // wave-uniform: N is a multiple of 64
     const int drow = wact ? wrow : N - 64;  // rows whose records a wave loads (waves past N: loaded, not used)
     const int m = lane & 31, kh = lane >> 5, g = m & 7;
-    const int tl = (wrow >> 4) + (m >> 3);  // the lane's 16-row tile among the expert's N rows
 
     // records of 64-k step kt: DMA d, lane i fetches record (g = i % 8, t = 2 d + i / 32) of wave tile (i / 8) % 4 into
     // LDS slot 64 d + i = 32 t + m (m = i % 32: the row pair of A row m)
@@ -252,38 +251,36 @@ __device__ __forceinline__ void rw_body(const MoePfArgs& ma, char* lds, int nt, 
     }
 
     if (!wact) return;
-    // epilogue: lane l holds token a * 32 + l % 32; register r = 4 q + j is row pair g = 4 (l / 32) + j of tile q
-#pragma unroll
-    for (int a = 0; a < NA; a++) {
-        const int tok = a * 32 + m;
-        if (tok >= T) continue;
-        const int slot = slot0 + tok;
-        if constexpr (MODE == 1) {
-            const float sw = ma.slot_w[slot];
+    // epilogue: lane l holds token a * 32 + l % 32; register r = 4 q + j is row pair g = 4 (l / 32) + j of tile q; the
+    // job's slots are consecutive rows, stored whole (64 B of act, 128 B of a slot row per wave and token) through the
+    // wave's share of the LDS, which every wave has left by the last step's barrier
+    if constexpr (MODE == 1) {
+        store_tile_rows<2, 32, NA>(lds + wave * 32 * out_pitch_of<2, 32>(), lane, T, 32,
+                                   ma.out + (size_t)slot0 * ma.I + (wrow >> 1), ma.I, [&](int a, char* wr) {
+            const int tok = a * 32 + m;
+            const float sw = ma.slot_w[slot0 + (tok < T ? tok : T - 1)];
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 float v[4];
 #pragma unroll
                 for (int j = 0; j < 4; j++)
                     v[j] = silu_f32(acc[a][0][4 * q + j]) * acc[a][1][4 * q + j] * sw * kMoeF16Scale;
-                const int col = ((wrow >> 4) + q) * 8 + 4 * kh;
-                *reinterpret_cast<uint2*>(ma.out + (size_t)slot * ma.I + col) =
-                    uint2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])};
+                *reinterpret_cast<uint2*>(wr + (8 * q + 4 * kh) * 2) = uint2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])};
             }
-        } else {
+        });
+    } else {
+        // the activation is act / 16, so the sums are the slot / 16: stored as is (fp16)
+        store_tile_rows<2, 64, NA>(lds + wave * 32 * out_pitch_of<2, 64>(), lane, T, 64,
+                                   ma.out + (size_t)slot0 * ma.H + wrow, ma.H, [&](int a, char* wr) {
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int n = wrow + 16 * q + 4 * kh;
-                uint16_t* o = ma.out + (size_t)slot * ma.H + n;
-                const f32x16_v& lo = acc[a][0];
-                const f32x16_v& hi = acc[a][1];
-                // the activation is act / 16, so the sums are the slot / 16: stored as is (fp16)
-                *reinterpret_cast<uint2*>(o) =
-                    uint2{pack_f16x2(lo[4 * q], lo[4 * q + 1]), pack_f16x2(lo[4 * q + 2], lo[4 * q + 3])};
-                *reinterpret_cast<uint2*>(o + 8) =
-                    uint2{pack_f16x2(hi[4 * q], hi[4 * q + 1]), pack_f16x2(hi[4 * q + 2], hi[4 * q + 3])};
-            }
-        }
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const f32x16_v& v = acc[a][h];
+                    *reinterpret_cast<uint2*>(wr + (16 * q + 8 * h + 4 * kh) * 2) =
+                        uint2{pack_f16x2(v[4 * q], v[4 * q + 1]), pack_f16x2(v[4 * q + 2], v[4 * q + 3])};
+                }
+        });
     }
 }
 
