@@ -1,5 +1,6 @@
 // Decode GEMM for up to 64 activation rows on the W4 layout, one pass over the weights (the reference's wide decode
-// GEMVs, src/kernels/gemv_x.cu:1-12,902-980, read the matrix once for m 9..64).
+// GEMVs, src/kernels/gemv_x.cu:1-12,902-980, read the matrix once for m 9..64). Up to 32 rows: wdec_kernel, described
+// here; 33..64 rows: wdec2_kernel below.
 //
 // The skinny kernel (skinny.hip) stages every activation row of its K slice per wave and multiplies 16-row weight
 // tiles on 16 x 16 MFMAs; past 16 rows its cost is the activation staging and the B operand reads, which grow with m,
@@ -12,8 +13,7 @@
 // nibbles (shifted down) that of row g + 8. The B operand is chunk c of a token row:
 // one ds_read_b128 of the wave's staged activation tile ([32 rows][64 k] bf16, 16-byte chunks XOR-swizzled).
 //
-// Block = 4 waves = TB token blocks of 32 rows x KP = 4 / TB contiguous K parts, over one 64-row weight slab (N / 64
-// blocks). Every wave stages its own activation rows, records and scales by LDS DMA (global_load_lds) into a ring of
+// Block = 4 waves = KP = 4 contiguous K parts, over one 64-row weight slab (N / 64 blocks). Every wave stages its own activation rows, records and scales by LDS DMA (global_load_lds) into a ring of
 // NBUF buffers, DEPTH = NBUF - 1 steps ahead, so no wave waits for another until the end; per 64-k step a wave issues 7 DMAs
 // (four 1 KB activation pieces, two 1 KB record pieces, one 256-byte scale piece), and every wait is a compile-time
 // vmcnt. The next k16 step's A operands are built between the MFMAs of the current one. After the K loop each
@@ -41,23 +41,23 @@ constexpr int kLds = NBUF * NW * kBuf;        // 76800 B: two blocks per CU
 constexpr int kPart = 68;                     // floats per token row of a wave's partial sums (64 rows + pad)
 static_assert(NW * 32 * kPart * 4 <= kLds, "the partial sums fit the staging buffers");
 
-// TB token blocks of 32 rows (m <= 32 TB), out: 0 fp32, 1 bf16, 2 GLU (bf16 activation, n / 2 columns)
+// up to 32 rows; out: 0 fp32, 1 bf16, 2 GLU (bf16 activation, n / 2 columns)
 // Blocks [0, nmain): one slab each over the whole K. Blocks past nmain: part p = u % P of tail slab nmain + u / P
-// (u = block - nmain), over K steps [p KT / P, (p + 1) KT / P); its sums go to tpart[u] ([TB * 32 tokens][64 rows]
+// (u = block - nmain), over K steps [p KT / P, (p + 1) KT / P); its sums go to tpart[u] ([32 tokens][64 rows]
 // fp32, written through to the device-coherent level), then it adds one to tctr[u / P]; the part that brings the
 // count to P adds the P parts in order p = 0..P-1, stores the outputs and sets the count back to zero (the counters
 // are zero when their buffer is allocated). P = 1: no tail blocks.
-template <int SDT, int TB>
+template <int SDT>
 __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ q, const uint16_t* __restrict__ s,
                                                       int K, const uint16_t* __restrict__ x, int ldx, int M,
                                                       void* __restrict__ y, int ldy, int out, int nmain, int P,
                                                       float* __restrict__ tpart, uint32_t* __restrict__ tctr) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
-    constexpr int KP = NW / TB;
+    constexpr int KP = NW;  // a K part per wave
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned lds32 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)lds);
-    const int tb = wave / KP, kp = wave - tb * KP;
+    const int kp = wave;
     const int b = blockIdx.x, tail = b >= nmain ? b - nmain : -1;  // tail part index u, or -1
     const int slab = tail < 0 ? b : nmain + tail / P, KTb = tail < 0 ? K / BK : K / BK / P;
     const int KTw = KTb / KP, kt0 = (tail < 0 ? 0 : (tail % P) * KTb) + kp * KTw, G = K >> 7;
@@ -72,8 +72,8 @@ __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ 
     const uint16_t* xsrc[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-        const int row = 8 * r + (lane >> 3), tok = 32 * tb + row;
-        xsrc[r] = x + (size_t)(tok < M ? tok : M - 1) * ldx + (((lane & 7) ^ swz_f(row)) << 3);
+        const int row = 8 * r + (lane >> 3);
+        xsrc[r] = x + (size_t)(row < M ? row : M - 1) * ldx + (((lane & 7) ^ swz_f(row)) << 3);
     }
     const int dtl = tile0 + ((lane >> 3) & 3);
     const uint4* wsrc = q + (size_t)dtl * (K >> 6) * 32 + 4 * (lane & 7) + kh;
@@ -225,12 +225,12 @@ __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ 
             *reinterpret_cast<f32x4_v*>(part + (wave * 32 + mr) * kPart + 16 * qq + 8 * op + 4 * kh) =
                 f32x4_v{acc[op][4 * qq], acc[op][4 * qq + 1], acc[op][4 * qq + 2], acc[op][4 * qq + 3]};
     __syncthreads();
-    // the KP parts of a token block added in a fixed tree order (parts i and i + h, h = KP / 2, ..., 1)
-    auto sum4 = [&](int otb, int tok, int r4) {  // rows r4 .. r4 + 3 of the slab
+    // the KP parts added in a fixed tree order (parts i and i + h, h = KP / 2, ..., 1)
+    auto sum4 = [&](int tok, int r4) {  // rows r4 .. r4 + 3 of the slab
         f32x4_v p[KP];
 #pragma unroll
         for (int k = 0; k < KP; k++)
-            p[k] = *reinterpret_cast<const f32x4_v*>(part + ((otb * KP + k) * 32 + tok) * kPart + r4);
+            p[k] = *reinterpret_cast<const f32x4_v*>(part + (k * 32 + tok) * kPart + r4);
 #pragma unroll
         for (int h = KP / 2; h >= 1; h >>= 1)
 #pragma unroll
@@ -238,31 +238,29 @@ __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ 
         return p[0];
     };
     const int n0 = tile0 * 16;
-    // the epilogue of 4 consecutive rows r4 of token otb * 32 + tok, from get4(otb, tok, r4)
+    // the epilogue of 4 consecutive rows r4 of token tok, from get4(tok, r4)
     auto emit = [&](auto&& get4) {
         if (out == 2) {  // thread = (token, tile, row quad of the 8 gate rows): gate rows g, up rows g + 8
-            for (int o = tid; o < TB * 32 * 8; o += NTH) {
-                const int otb = o >> 8, tok = (o >> 3) & 31, qq = (o >> 1) & 3, gq = o & 1;
-                const int t = 32 * otb + tok;
-                if (t >= M) continue;
-                const f32x4_v ga = get4(otb, tok, 16 * qq + 4 * gq), up = get4(otb, tok, 16 * qq + 8 + 4 * gq);
-                uint16_t* p = reinterpret_cast<uint16_t*>(y) + (size_t)t * ldy + (tile0 + qq) * 8 + 4 * gq;
+            for (int o = tid; o < 32 * 8; o += NTH) {
+                const int tok = o >> 3, qq = (o >> 1) & 3, gq = o & 1;
+                if (tok >= M) continue;
+                const f32x4_v ga = get4(tok, 16 * qq + 4 * gq), up = get4(tok, 16 * qq + 8 + 4 * gq);
+                uint16_t* p = reinterpret_cast<uint16_t*>(y) + (size_t)tok * ldy + (tile0 + qq) * 8 + 4 * gq;
 #pragma unroll
                 for (int i = 0; i < 4; i++) p[i] = f32_to_bf16(silu_f32(ga[i]) * up[i]);
             }
             return;
         }
-        for (int o = tid; o < TB * 32 * 16; o += NTH) {  // thread = (token, 4 consecutive rows)
-            const int otb = o >> 9, tok = (o >> 4) & 31, r4 = 4 * (o & 15);
-            const int t = 32 * otb + tok;
-            if (t >= M) continue;
-            const f32x4_v v = get4(otb, tok, r4);
+        for (int o = tid; o < 32 * 16; o += NTH) {  // thread = (token, 4 consecutive rows)
+            const int tok = o >> 4, r4 = 4 * (o & 15);
+            if (tok >= M) continue;
+            const f32x4_v v = get4(tok, r4);
             if (out == 1) {
-                uint16_t* p = reinterpret_cast<uint16_t*>(y) + (size_t)t * ldy + n0 + r4;
+                uint16_t* p = reinterpret_cast<uint16_t*>(y) + (size_t)tok * ldy + n0 + r4;
 #pragma unroll
                 for (int i = 0; i < 4; i++) p[i] = f32_to_bf16(v[i]);
             } else {
-                float* p = reinterpret_cast<float*>(y) + (size_t)t * ldy + n0 + r4;
+                float* p = reinterpret_cast<float*>(y) + (size_t)tok * ldy + n0 + r4;
 #pragma unroll
                 for (int i = 0; i < 4; i++) p[i] = v[i];
             }
@@ -273,14 +271,14 @@ __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ 
         return;
     }
     // a tail part: its sums to tpart[tail] (device-coherent stores), completed before the count
-    constexpr int kPartFloats = TB * 32 * 64;
+    constexpr int kPartFloats = 32 * 64;
     float* mine = tpart + (size_t)tail * kPartFloats;
-    for (int o = tid; o < TB * 32 * 16; o += NTH) {
-        const int otb = o >> 9, tok = (o >> 4) & 31, r4 = 4 * (o & 15);
-        const f32x4_v v = sum4(otb, tok, r4);
+    for (int o = tid; o < 32 * 16; o += NTH) {
+        const int tok = o >> 4, r4 = 4 * (o & 15);
+        const f32x4_v v = sum4(tok, r4);
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            __hip_atomic_store(mine + (otb * 32 + tok) * 64 + r4 + i, v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(mine + tok * 64 + r4 + i, v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __shared__ uint32_t last;
@@ -290,16 +288,311 @@ __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ 
     __syncthreads();
     if (!last) return;
     const float* all = tpart + (size_t)ts * P * kPartFloats;  // parts p = 0..P-1 of this tail slab
-    emit([&](int otb, int tok, int r4) {  // the parts in order p = 0..P-1
+    emit([&](int tok, int r4) {  // the parts in order p = 0..P-1
         f32x4_v v = {0.f, 0.f, 0.f, 0.f};
         for (int pp = 0; pp < P; pp++) {
-            float* src = const_cast<float*>(all) + (size_t)pp * kPartFloats + (otb * 32 + tok) * 64 + r4;
+            float* src = const_cast<float*>(all) + (size_t)pp * kPartFloats + tok * 64 + r4;
 #pragma unroll
             for (int i = 0; i < 4; i++) v[i] += __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         return v;
     });
     if (tid == 0) __hip_atomic_store(&tctr[ts], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ---- 33..64 rows: one wave holds both 32-row token blocks.
+//
+// With a wave per token block two waves would build the same A operands and stage the same records: at 48 rows that
+// ran 34816 x 5120 (GLU, 89 MB) in 58 us and 5120 x 17408 in 44.5 us. This kernel takes 49 and 28 us (1.8 and 1.6
+// TB/s of records). What bounds it (variants that skip one part, 32768 x 5120, 44.5 us): without activation DMAs
+// 35.7, without record DMAs 34.7, without the MFMAs and their operands 30.9, records alone 22.4 us: matrix cores
+// (20 MFMAs a wave and step, 0.6 us of a 1.3 us step), LDS and DMA add up across the step's barrier. Records three
+// steps ahead with 48 staged rows, and whole-record LDS reads, measured the same. Here block = 8 waves = 2 row waves (64 weight rows
+// each, a 128-row slab) x 4 K parts; the two row waves of a K part share one staged activation tile [64][64], so a CU
+// stages half the activations per weight and holds 32 KB of records in flight (2 steps x 8 waves x 2 KB), and every
+// operand feeds two MFMAs. The bias -136 sum x is built once per pair (row wave rw does token block rw) and exchanged
+// through LDS at the group's end, so a k16 step is 5 MFMAs a wave for 4 of product. A step ends with a barrier (the
+// pair shares its tile); the group's flush acc += s (c + b) runs at the top of the next step. K parts are whole
+// groups, uneven where they do not divide; a wave whose part is shorter idles through the last steps' barriers.
+// Slabs past the last whole round of CUs (all of them when they do not fill one) run as P K ranges whose sums
+// wdec2_reduce_kernel adds in order. Rows past m re-read row m - 1 and are not stored.
+namespace two {
+constexpr int NW2 = 8, NTH2 = 64 * NW2, KP = 4, NT = 2, TOK = 32 * NT, ROWS = 128, NBUF2 = 3;
+constexpr int kX2 = TOK * BK * 2;                         // activation tile of a K part and step, swizzled
+constexpr int kW2 = 2048;                                 // a wave's records of a step
+constexpr int kBuf2 = KP * kX2 + NW2 * kW2;               // 48 KB, DMA two steps ahead
+constexpr int kScOff = NBUF2 * kBuf2, kSc2 = 256;         // scales, four deep (a group's are read a step late): [4][wave]
+constexpr int kBiasOff = kScOff + 4 * NW2 * kSc2;         // [KP][NT][32] floats
+constexpr int kLds2 = kBiasOff + KP * NT * 32 * 4;        // 153 KB: one block per CU
+constexpr int kPitch = ROWS + 4;                          // floats per token row of a K part's sums
+static_assert(KP * TOK * kPitch * 4 <= kScOff, "the K parts' sums fit the staging buffers");
+}  // namespace two
+
+// 4 consecutive rows r4 of the slab at n0, token t (< M) from the fp32 sums: out 0 fp32, 1 bf16; GLU (out 2): v gate, u up
+__device__ __forceinline__ void emit4(void* y, int ldy, int out, int t, int n, f32x4_v v, f32x4_v u) {
+    if (out == 0) {
+        float* p = reinterpret_cast<float*>(y) + (size_t)t * ldy + n;
+        if (((ldy & 3) | ((uintptr_t)y & 15)) == 0) {
+            *reinterpret_cast<f32x4_v*>(p) = v;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) p[i] = v[i];
+        }
+        return;
+    }
+    if (out == 2) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = silu_f32(v[i]) * u[i];
+        n = (n >> 4) * 8 + (n & 7);
+    }
+    uint16_t* p = reinterpret_cast<uint16_t*>(y) + (size_t)t * ldy + n;
+    if (((ldy & 3) | ((uintptr_t)y & 7)) == 0) {
+        *reinterpret_cast<uint2*>(p) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) p[i] = f32_to_bf16(v[i]);
+    }
+}
+
+// Blocks [0, nmain): slab b over all groups; block nmain + u: K range u % P of slab nmain + u / P, its sums to
+// tpart[u] ([TOK][ROWS] fp32, rows of tokens below M)
+template <int SDT>
+__global__ void __launch_bounds__(two::NTH2) wdec2_kernel(const uint4* __restrict__ q, const uint16_t* __restrict__ s,
+                                                          int N, int K, const uint16_t* __restrict__ x, int ldx, int M,
+                                                          void* __restrict__ y, int ldy, int out, int nmain, int P,
+                                                          float* __restrict__ tpart) {
+    using namespace two;
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned lds32 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)lds);
+    const int rw = wave & 1, kp = wave >> 1;
+    const int b = blockIdx.x, tail = b >= nmain ? b - nmain : -1;
+    const int slab = tail < 0 ? b : nmain + tail / P, pp = tail < 0 ? 0 : tail % P, np = tail < 0 ? 1 : P;
+    const int G = K >> 7;
+    const int g0 = pp * G / np, gb = (pp + 1) * G / np - g0;  // the block's groups
+    const int ga = g0 + kp * gb / KP, nown = 2 * (g0 + (kp + 1) * gb / KP - ga);  // the wave's first group, its steps
+    const int nst = 2 * ((gb + KP - 1) / KP);                                     // the longest K part's steps
+    const int n0 = slab * ROWS;
+    const int tile0 = min(n0 / 16 + 4 * rw, N / 16 - 4);  // a ragged last slab (N % 128 = 64): rw 1 repeats rw 0's rows
+    const int mr = lane & 31, kh = lane >> 5;
+
+    // DMA sources: as in wdec_kernel; the pair's activation pieces (8 rows each) are split between its waves
+    const uint16_t* xsrc[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int row = 8 * (4 * rw + i) + (lane >> 3);
+        xsrc[i] = x + (size_t)(row < M ? row : M - 1) * ldx + (((lane & 7) ^ swz_f(row)) << 3);
+    }
+    const int dtl = tile0 + ((lane >> 3) & 3);
+    const uint4* wsrc = q + (size_t)dtl * (K >> 6) * 32 + 4 * (lane & 7) + kh;
+    const uint16_t* ssrc = s + (size_t)dtl * G * 16 + 2 * (lane & 7);
+    const int ktmax = 2 * ga + nown - 1 > 0 ? min(2 * ga + max(nown, 1) - 1, 2 * G - 1) : 0;
+    // step j into buffer bj = j % 3: 7 DMAs; steps past the wave's last re-read it
+    auto dma_step = [&](int j, int bj) {
+        const int kt = min(2 * ga + j, ktmax);
+        const unsigned bo = lds32 + bj * kBuf2, wo = bo + KP * kX2 + wave * kW2;
+#pragma unroll
+        for (int i = 0; i < 4; i++) dma16(xsrc[i] + kt * BK, bo + kp * kX2 + (4 * rw + i) * 1024);
+        dma16(wsrc + (size_t)kt * 32, wo);
+        dma16(wsrc + (size_t)kt * 32 + 2, wo + 1024);
+        dma4(ssrc + (kt >> 1) * 16, lds32 + kScOff + ((j & 3) * NW2 + wave) * kSc2);
+    };
+    f32x16_v acc[NT][2], c[NT][2], cb;
+    const f32x16_v zero = {};
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) acc[t][h] = zero;
+    cb = zero;
+    int xo[BK / 16];
+#pragma unroll
+    for (int ks = 0; ks < BK / 16; ks++) xo[ks] = mr * 128 + (((4 * (ks & 1) + 2 * kh + (ks >> 1)) ^ swz_f(mr)) << 4);
+    uint32_t raw[2][4][2];  // words kh, 2 + kh of records t = 0..3, by step parity (masked where they are used)
+    auto load_step = [&](int bj, auto set) {
+        constexpr int S = decltype(set)::value;
+        const uint32_t* rp = reinterpret_cast<const uint32_t*>(lds + bj * kBuf2 + KP * kX2 + wave * kW2) + mr * 4 + kh;
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int w = 0; w < 2; w++) raw[S][t][w] = rp[t * 128 + 2 * w];
+    };
+    auto opnd = [&](const uint32_t (&rv)[4][2], int hi, int ks) {
+        u32x4_v a;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const uint32_t u = (hi ? rv[t][ks & 1] >> 4 : rv[t][ks & 1]) & nib_mask();
+            a[t] = __builtin_amdgcn_perm(0x43434343u, u, (ks >> 1) ? kSel13 : kSel02);
+        }
+        return a;
+    };
+    const u32x4_v bias_w = {0xC308C308u, 0xC308C308u, 0xC308C308u, 0xC308C308u};  // bf16 -136 pairs
+    const bf16x8_v abias = __builtin_bit_cast(bf16x8_v, bias_w);
+    float* biasl = reinterpret_cast<float*>(lds + kBiasOff) + kp * NT * 32;  // the pair's [NT][32]
+    auto flush = [&](int j) {  // the group that ended with step j
+        const uint16_t* sp = reinterpret_cast<const uint16_t*>(lds + kScOff + ((j & 3) * NW2 + wave) * kSc2) + 4 * kh;
+        float bt[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) bt[t] = biasl[(t ^ rw) * 32 + mr];
+#pragma unroll
+        for (int qq = 0; qq < 4; qq++)
+#pragma unroll
+            for (int op = 0; op < 2; op++) {
+                const uint2 sv = *reinterpret_cast<const uint2*>(sp + 16 * qq + 8 * op);
+                const uint16_t sh[4] = {(uint16_t)sv.x, (uint16_t)(sv.x >> 16), (uint16_t)sv.y, (uint16_t)(sv.y >> 16)};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int r = 4 * qq + i;
+#pragma unroll
+                    for (int t = 0; t < NT; t++)
+                        acc[t][op][r] = fmaf(scale_to_f32<SDT>(sh[i]), c[t][op][r] + bt[t], acc[t][op][r]);
+                }
+            }
+    };
+    u32x4_v an[2][2];
+    using P0 = std::integral_constant<int, 0>;
+    using P1 = std::integral_constant<int, 1>;
+    auto wait7 = [] { asm volatile("s_waitcnt vmcnt(7)" ::: "memory"); };  // all DMAs but the newest step's
+    // the MFMAs of a step (set S: its parity, buffer bj), with the next step's records (buffer bn) read at ks = 2 (a
+    // re-read past the last step)
+    auto mfmas = [&](int bj, int bn, auto set) {
+        constexpr int S = decltype(set)::value;
+        using SN = std::integral_constant<int, S ^ 1>;
+        const char* xt = lds + bj * kBuf2 + kp * kX2;  // token block t of the wave: t ^ rw of the tile
+        bf16x8_v xf[2][NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) xf[0][t] = *reinterpret_cast<const bf16x8_v*>(xt + xo[0] + (t ^ rw) * 4096);
+#pragma unroll
+        for (int ks = 0; ks < BK / 16; ks++) {
+            const u32x4_v a0 = an[ks & 1][0], a1 = an[ks & 1][1];
+            const bf16x8_v A0 = __builtin_bit_cast(bf16x8_v, a0);
+            const bf16x8_v A1 = __builtin_bit_cast(bf16x8_v, a1);
+            const bool first = S == 0 && ks == 0;
+            if (ks + 1 < BK / 16) {
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+                    xf[(ks + 1) & 1][t] = *reinterpret_cast<const bf16x8_v*>(xt + xo[ks + 1] + (t ^ rw) * 4096);
+            }
+            if (ks == 2) {
+                wait7();
+                load_step(bn, SN{});
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            c[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A0, xf[ks & 1][0], first ? zero : c[0][0], 0, 0, 0);
+            if (ks + 1 < BK / 16) an[(ks + 1) & 1][0] = opnd(raw[S], 0, ks + 1);
+            else an[0][0] = opnd(raw[S ^ 1], 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            c[1][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A0, xf[ks & 1][1], first ? zero : c[1][0], 0, 0, 0);
+            if (ks + 1 < BK / 16) an[(ks + 1) & 1][1] = opnd(raw[S], 1, ks + 1);
+            else an[0][1] = opnd(raw[S ^ 1], 1, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            c[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A1, xf[ks & 1][0], first ? zero : c[0][1], 0, 0, 0);
+            c[1][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A1, xf[ks & 1][1], first ? zero : c[1][1], 0, 0, 0);
+            cb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(abias, xf[ks & 1][0], first ? zero : cb, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (S == 1 && kh == 0) biasl[rw * 32 + mr] = cb[0];  // every row of cb is the same sum
+    };
+    auto step_end = [] { asm volatile("s_waitcnt vmcnt(7) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+    dma_step(0, 0);
+    dma_step(1, 1);
+    step_end();
+    load_step(0, P0{});
+    an[0][0] = opnd(raw[0], 0, 0);
+    an[0][1] = opnd(raw[0], 1, 0);
+    int b0 = 0, b1 = 1, b2 = 2;  // j % 3, (j + 1) % 3, (j + 2) % 3
+    for (int j = 0; j < nst; j += 2) {
+        dma_step(j + 2, b2);
+        if (j > 0 && j <= nown) flush(j - 1);
+        if (j < nown) mfmas(b0, b1, P0{});
+        step_end();
+        dma_step(j + 3, b0);
+        if (j < nown) mfmas(b1, b2, P1{});
+        step_end();
+        const int t = b1;
+        b1 = b0;
+        b0 = b2;
+        b2 = t;
+    }
+    if (nown == nst) flush(nst - 1);
+
+    // the K parts' sums: lane l holds token 32 (t ^ rw) + mr, register 4 qq + i of operand op is row 64 rw + 16 qq + 8 op +
+    // 4 kh + i of the slab
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the re-read steps' DMAs have landed
+    __syncthreads();
+    float* part = reinterpret_cast<float*>(lds);
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int qq = 0; qq < 4; qq++)
+#pragma unroll
+            for (int op = 0; op < 2; op++) {
+                const f32x16_v& v = acc[t][op];
+                *reinterpret_cast<f32x4_v*>(part + (size_t)(kp * TOK + 32 * (t ^ rw) + mr) * kPitch + 64 * rw + 16 * qq + 8 * op + 4 * kh) =
+                    f32x4_v{v[4 * qq], v[4 * qq + 1], v[4 * qq + 2], v[4 * qq + 3]};
+            }
+    __syncthreads();
+    auto sum4 = [&](int tok, int r4) {  // the four K parts in a fixed tree order
+        f32x4_v p[KP];
+#pragma unroll
+        for (int k = 0; k < KP; k++) p[k] = *reinterpret_cast<const f32x4_v*>(part + (size_t)(k * TOK + tok) * kPitch + r4);
+        return (p[0] + p[2]) + (p[1] + p[3]);
+    };
+    if (tail >= 0) {
+        float* mine = tpart + (size_t)tail * TOK * ROWS;
+        for (int o = tid; o < M * (ROWS / 4); o += NTH2) {
+            const int tok = o / (ROWS / 4), r4 = 4 * (o % (ROWS / 4));
+            *reinterpret_cast<f32x4_v*>(mine + tok * ROWS + r4) = sum4(tok, r4);
+        }
+        return;
+    }
+    if (out == 2) {
+        for (int o = tid; o < M * (ROWS / 8); o += NTH2) {
+            const int tok = o / (ROWS / 8), e = o % (ROWS / 8), r4 = 16 * (e >> 1) + 4 * (e & 1);
+            if (n0 + r4 < N) emit4(y, ldy, out, tok, n0 + r4, sum4(tok, r4), sum4(tok, r4 + 8));
+        }
+    } else {
+        for (int o = tid; o < M * (ROWS / 4); o += NTH2) {
+            const int tok = o / (ROWS / 4), r4 = 4 * (o % (ROWS / 4));
+            if (n0 + r4 < N) emit4(y, ldy, out, tok, n0 + r4, sum4(tok, r4), f32x4_v{});
+        }
+    }
+}
+
+// The P parts of each split slab added in order, then the epilogue: one thread per (slab, token, 4 rows; GLU 4 gate
+// and 4 up rows)
+__global__ void __launch_bounds__(256) wdec2_reduce_kernel(const float* __restrict__ tpart, int P, int slab0, int nslab,
+                                                           int N, int M, void* __restrict__ y, int ldy, int out) {
+    using namespace two;
+    const int CB = out == 2 ? ROWS / 8 : ROWS / 4;
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= nslab * M * CB) return;
+    const int e = idx % CB, tok = (idx / CB) % M, ts = idx / CB / M;
+    const int r4 = out == 2 ? 16 * (e >> 1) + 4 * (e & 1) : 4 * e;
+    const int n = (slab0 + ts) * ROWS + r4;
+    if (n >= N) return;
+    const float* p = tpart + ((size_t)ts * P * TOK + tok) * ROWS + r4;
+    f32x4_v v = {}, u = {};
+    for (int k = 0; k < P; k++, p += TOK * ROWS) {
+        v = v + *reinterpret_cast<const f32x4_v*>(p);
+        if (out == 2) u = u + *reinterpret_cast<const f32x4_v*>(p + 8);
+    }
+    emit4(y, ldy, out, tok, n, v, u);
+}
+
+// K ranges per split slab: the fewest steps of the longest wave with the parts within one round of CUs (then the
+// fewest parts)
+int two_parts(int rem, int G, int ncu) {
+    int best = 1, best_steps = (G + two::KP - 1) / two::KP;
+    for (int p = 2; p <= 16 && p <= G && rem * p <= ncu; p++) {
+        const int steps = ((G + p - 1) / p + two::KP - 1) / two::KP;
+        if (steps < best_steps) {
+            best = p;
+            best_steps = steps;
+        }
+    }
+    return best;
 }
 
 int token_blocks(int m) { return m > 32 ? 2 : 1; }
@@ -331,20 +624,32 @@ namespace qe_gemv {
 int decode_groups(int n, int k);
 }
 
-// Where the one-pass kernel beats the skinny kernel's 32-row launches (measured in one process, bf16 out, us one-pass
-// / skinny): one round of slabs or more (N = 17408, K = 5120, m = 32: 20.7 / 28.9), K without an even skinny slicing
-// (the skinny kernel's uneven slices; N = 3072, K = 9216, m = 32: 14.5 / 20.4), and more than 48 rows from ~26 M
-// weights (N = K = 8192, m = 64: 27.6 / 30.2; N = K = 5120: 20.3 / 21.5). Small matrices keep the skinny launches:
-// N = K = 4096, m = 32: 11.8 / 7.8; N = K = 2048: 9.4 / 5.0; N = 6144, K = 4096, m = 64: 18.9 / 18.2.
+// the 33..64-row kernel's own limits (any whole number of groups)
+static bool two_fits(const W4& w, const uint16_t* x, int ldx, int m) {
+    return m > 32 && m <= 64 && w.n > 0 && w.n % 64 == 0 && w.k > 0 && w.k % 128 == 0 && ((uintptr_t)x & 15) == 0 &&
+           ldx % 8 == 0;
+}
+
+// Where the one-pass kernels beat the skinny kernel's 32-row launches (measured in one process, bf16 out, us one-pass
+// / skinny). 17..32 rows: one round of slabs or more (N = 17408, K = 5120, m = 32: 20.7 / 28.9) and K without an even
+// skinny slicing (the skinny kernel's uneven slices; N = 3072, K = 9216, m = 32: 14.5 / 20.4); small matrices keep the
+// skinny launches: N = K = 4096, m = 32: 11.8 / 7.8; N = K = 2048: 9.4 / 5.0. 33..64 rows (m = 33 / 48 / 64): uneven
+// K (N = 5120, K = 17408: 27 / 28 / 29 against 75 / 88 / 118) and from ~25 M weights (N = K = 5120: 15.3 / 16.3 / 17.0
+// against 16.7 / 18.6 / 21.6; N = 6144, K = 4096: 14.8 / 15.6 / 16.3 against 14.5 / 16.0 / 18.3); smaller ones keep
+// the skinny launches (N = K = 4096: 14.3 / 14.9 / 16.0 against 12.0 / 13.4 / 15.7).
 bool wdec_w4_pick(const W4& w, const uint16_t* x, int ldx, int m) {
     using namespace qe_wdec;
-    if (!wdec_w4_fits(w, x, ldx, m)) return false;
     const int nslabs = w.n / 64, ncu = qe_num_cus();
+    if (token_blocks(m) == 2) {
+        if (!two_fits(w, x, ldx, m)) return false;
+        const long weights = (long)w.n * w.k;
+        return qe_gemv::decode_groups(w.n, w.k) == 0 || weights > (24L << 20) || (m >= 48 && weights >= (23L << 20));
+    }
+    if (!wdec_w4_fits(w, x, ldx, m)) return false;
     // slabs filling at most half the CUs only with K parts (N = 4096, K = 11008, m = 48: 64 slabs, no part count fits
     // 172 steps: 48.4 us against 35.2)
     if (2 * nslabs <= ncu && tail_parts(nslabs, w.k / BK, NW / token_blocks(m), ncu) == 1) return false;
-    if (nslabs >= ncu || qe_gemv::decode_groups(w.n, w.k) == 0) return true;
-    return m > 48 && (long)w.n * w.k >= (26L << 20);
+    return nslabs >= ncu || qe_gemv::decode_groups(w.n, w.k) == 0;
 }
 
 // Slabs past the last whole round of CUs (N / 64 = 272 on 256 CUs: 16) would give 16 CUs two slabs; they run as P
@@ -354,12 +659,39 @@ bool wdec_w4_pick(const W4& w, const uint16_t* x, int ldx, int m) {
 // capture: then P = 1). The last part's in-order sum reads the P parts from the device-coherent level, one part at
 // a time, so fewer parts finish sooner: on C0's matrix (16 tail slabs, 80 K steps) P = 5 measured m = 32 / 64
 // 20.7 / 31.7 us against 22.9 / 36.9 us at P = 10, 23.1 / 33.3 us at P = 2, and 26.7 / 40.0 us with no tail split.
+// (33..64 rows: two_parts, summed by a kernel of their own.)
 void wdec_w4(const W4& w, const uint16_t* x, int ldx, void* y, int ldy, int m, bool out_bf16, hipStream_t st) {
     using namespace qe_wdec;
-    CHECK(wdec_w4_fits(w, x, ldx, m), "wdec_w4: n %d k %d m %d ldx %d", w.n, w.k, m, ldx);
+    CHECK(wdec_w4_fits(w, x, ldx, m) || two_fits(w, x, ldx, m), "wdec_w4: n %d k %d m %d ldx %d", w.n, w.k, m, ldx);
     CHECK(ldy >= (w.glu ? w.n / 2 : w.n), "wdec_w4 ldy %d", ldy);
     const int out = w.glu ? 2 : out_bf16 ? 1 : 0;
-    const int TB = token_blocks(m), KP = NW / TB, KT = w.k / BK, nslabs = w.n / 64, ncu = qe_num_cus();
+    if (token_blocks(m) == 2) {
+        const int ncu = qe_num_cus(), G = w.k >> 7, nsl = (w.n + two::ROWS - 1) / two::ROWS, rem = nsl % ncu;
+        int P = rem > 0 ? two_parts(rem, G, ncu) : 1;
+        float* tpart = nullptr;
+        if (P > 1) {
+            char* ws = dec_tail_ws(st);
+            if (ws) tpart = reinterpret_cast<float*>(ws + dec_tail_ctr_bytes());
+            else P = 1;
+        }
+        const int nmain = P > 1 ? nsl - rem : nsl;
+        const dim3 grid((unsigned)(nmain + (P > 1 ? rem * P : 0)));
+        if (w.sdt == kScaleF16)
+            wdec2_kernel<kScaleF16><<<grid, dim3(two::NTH2), two::kLds2, st>>>(w.q, w.s, w.n, w.k, x, ldx, m, y, ldy, out,
+                                                                               nmain, P, tpart);
+        else
+            wdec2_kernel<kScaleBF16><<<grid, dim3(two::NTH2), two::kLds2, st>>>(w.q, w.s, w.n, w.k, x, ldx, m, y, ldy, out,
+                                                                                nmain, P, tpart);
+        HIP_CHECK(hipGetLastError());
+        if (P > 1) {
+            const int threads = rem * m * (out == 2 ? two::ROWS / 8 : two::ROWS / 4);
+            wdec2_reduce_kernel<<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st>>>(tpart, P, nmain, rem, w.n, m,
+                                                                                               y, ldy, out);
+            HIP_CHECK(hipGetLastError());
+        }
+        return;
+    }
+    const int KP = NW, KT = w.k / BK, nslabs = w.n / 64, ncu = qe_num_cus();
     int nmain = nslabs, P = 1, rem = 0;
     float* tpart = nullptr;
     uint32_t* tctr = nullptr;
@@ -377,16 +709,9 @@ void wdec_w4(const W4& w, const uint16_t* x, int ldx, void* y, int ldy, int m, b
         }
     }
     const dim3 grid((unsigned)(nmain + (P > 1 ? rem * P : 0))), block(NTH);
-#define QE_WDEC(SDT_, TB_)                                                                                    \
-    wdec_kernel<SDT_, TB_><<<grid, block, kLds, st>>>(w.q, w.s, w.k, x, ldx, m, y, ldy, out, nmain, P, tpart, \
-                                                      tctr)
-    if (w.sdt == kScaleF16) {
-        if (token_blocks(m) == 2) QE_WDEC(kScaleF16, 2);
-        else QE_WDEC(kScaleF16, 1);
-    } else {
-        if (token_blocks(m) == 2) QE_WDEC(kScaleBF16, 2);
-        else QE_WDEC(kScaleBF16, 1);
-    }
-#undef QE_WDEC
+    if (w.sdt == kScaleF16)
+        wdec_kernel<kScaleF16><<<grid, block, kLds, st>>>(w.q, w.s, w.k, x, ldx, m, y, ldy, out, nmain, P, tpart, tctr);
+    else
+        wdec_kernel<kScaleBF16><<<grid, block, kLds, st>>>(w.q, w.s, w.k, x, ldx, m, y, ldy, out, nmain, P, tpart, tctr);
     HIP_CHECK(hipGetLastError());
 }

@@ -50,7 +50,7 @@ void* stream_ws(int kind, size_t bytes, hipStream_t st) {
 size_t dec_tail_ctr_bytes() { return ((size_t)qe_num_cus() * 4 + 255) / 256 * 256; }
 
 char* dec_tail_ws(hipStream_t st) {
-    return static_cast<char*>(stream_ws(kWsDec, dec_tail_ctr_bytes() + (size_t)qe_num_cus() * 2 * 32 * 64 * 4, st));
+    return static_cast<char*>(stream_ws(kWsDec, dec_tail_ctr_bytes() + (size_t)qe_num_cus() * 64 * 128 * 4, st));
 }
 
 void stream_ws_reserve(int kind, size_t bytes, hipStream_t st) {

@@ -128,3 +128,26 @@ def test_onepass_tail_parts_deterministic_and_graph(dev):
                 else:
                     rr = err_ratio(out.cpu().numpy(), want.cpu().numpy())
                     assert rr <= 1e-5, (m, r, rr)
+
+
+@pytest.mark.parametrize("n,k", [(64, 128), (192, 384), (4160, 640), (5120, 3712), (33024, 256)])
+@pytest.mark.parametrize("m", [33, 48, 63, 64])
+def test_decode_33_to_64_rows(dev, n, k, m):
+    """the 33..64-row kernel through the row-count dispatch or alone: slabs with a ragged half (n % 128 = 64), K of
+    fewer groups than K parts, uneven K parts, K ranges of split slabs; outputs at an odd offset and stride are the
+    contiguous ones bit for bit; GLU"""
+    w, q, s = setup_w4(n, k, 1, seed=n + m)
+    xh = synth.x_host(m, k, seed=k + m)
+    x = synth.to_dev(xh)
+    y = ops.matmul_w4(w, x)
+    assert err_ratio(out_f32(y), matmul_f64(xh, exact_w4(q, s, n, k, 1))) <= 1e-4
+    big = torch.full((m, n + 7), float("nan"), dtype=torch.float32, device=dev)
+    z = ops.matmul_w4(w, x, y=big[:, 1:1 + n])
+    assert torch.equal(z.contiguous().view(torch.int32), y.view(torch.int32))
+    assert torch.isnan(big[:, 0]).all() and torch.isnan(big[:, 1 + n:]).all()
+    wg, qg, sg = setup_w4(n, k, 1, seed=n + m + 1, glu=True)
+    a = ops.matmul_w4(wg, x)
+    assert_glu_close(out_f32(a), glu_act(matmul_f64(xh, exact_w4(qg, sg, n, k, 1))), 1e-4)
+    if k % 256 == 0:
+        y1 = ops.matmul_w4_onepass(w, x)
+        assert err_ratio(out_f32(y1), matmul_f64(xh, exact_w4(q, s, n, k, 1))) <= 1e-4
