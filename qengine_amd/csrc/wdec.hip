@@ -639,13 +639,13 @@ static bool two_fits(const W4& w, const uint16_t* x, int ldx, int m) {
 // the skinny launches (N = K = 4096: 14.3 / 14.9 / 16.0 against 12.0 / 13.4 / 15.7).
 bool wdec_w4_pick(const W4& w, const uint16_t* x, int ldx, int m) {
     using namespace qe_wdec;
-    const int nslabs = w.n / 64, ncu = qe_num_cus();
     if (token_blocks(m) == 2) {
         if (!two_fits(w, x, ldx, m)) return false;
         const long weights = (long)w.n * w.k;
         return qe_gemv::decode_groups(w.n, w.k) == 0 || weights > (24L << 20) || (m >= 48 && weights >= (23L << 20));
     }
     if (!wdec_w4_fits(w, x, ldx, m)) return false;
+    const int nslabs = w.n / 64, ncu = qe_num_cus();
     // slabs filling at most half the CUs only with K parts (N = 4096, K = 11008, m = 48: 64 slabs, no part count fits
     // 172 steps: 48.4 us against 35.2)
     if (2 * nslabs <= ncu && tail_parts(nslabs, w.k / BK, NW / token_blocks(m), ncu) == 1) return false;

@@ -8,7 +8,7 @@ from dataclasses import dataclass
 
 import torch
 
-from .qe import call
+from .qe import call, typed
 
 SCALE_F16 = 1
 OUT_BF16 = 2
@@ -42,9 +42,31 @@ def set_config(**kw):
     return old
 
 
+def _raw_stream():
+    """the current stream's address (hipStream_t) as an int, without building a Stream object"""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
 def _stream():
     # a pointer-sized argument: an int would be passed as a 32-bit c_int
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(_raw_stream())
+
+
+_TYPED = {}
+
+
+def _typed(name, sig, restype=None):
+    f = _TYPED.get(name)
+    if f is None:
+        f = _TYPED[name] = typed(name, sig, restype)
+    return f
+
+
+def _matmul(name, w, x, y, flags):
+    """the entry points (q, s, n, k, x, ldx, y, ldy, rows, flags, stream)"""
+    _typed(name, "ppiipipiiip")(w.q.data_ptr(), w.s.data_ptr(), w.n, w.k, x.data_ptr(), x.stride(0), y.data_ptr(),
+                                y.stride(0), x.shape[0], flags, _raw_stream())
+    return y
 
 
 def _scale_flag(s):
@@ -121,9 +143,7 @@ def gemv_w4(w: W4, x, out_bf16=False, y=None):
     m = x.shape[0]
     assert x.dtype == torch.bfloat16 and x.shape[1] == w.k and x.stride(1) == 1
     y = _out(m, w.n, out_bf16, w.glu, x.device) if y is None else y
-    call("qe_gemv_w4_ex", w.q, w.s, w.n, w.k, x, x.stride(0), y, y.stride(0), m,
-         w.flags | (OUT_BF16 if out_bf16 else 0), _stream())
-    return y
+    return _matmul("qe_gemv_w4_ex", w, x, y, w.flags | (OUT_BF16 if out_bf16 else 0))
 
 
 def xh_pack(x, ldxh=None):
@@ -164,9 +184,7 @@ def gemm_w4(w: W4, x, out_bf16=False, y=None):
     t = x.shape[0]
     assert x.dtype == torch.bfloat16 and x.shape[1] == w.k and x.stride(1) == 1
     y = _out(t, w.n, out_bf16, w.glu, x.device) if y is None else y
-    call("qe_gemm_w4_ex", w.q, w.s, w.n, w.k, x, x.stride(0), y, y.stride(0), t,
-         w.flags | (OUT_BF16 if out_bf16 else 0), _stream())
-    return y
+    return _matmul("qe_gemm_w4_ex", w, x, y, w.flags | (OUT_BF16 if out_bf16 else 0))
 
 
 def gemm_w4h(w: W4, x, out_bf16=False, y=None):
@@ -174,9 +192,7 @@ def gemm_w4h(w: W4, x, out_bf16=False, y=None):
     t = x.shape[0]
     assert x.dtype == torch.bfloat16 and x.shape[1] == w.k and x.stride(1) == 1
     y = _out(t, w.n, out_bf16, w.glu, x.device) if y is None else y
-    call("qe_gemm_w4h_ex", w.q, w.s, w.n, w.k, x, x.stride(0), y, y.stride(0), t,
-         w.flags | (OUT_BF16 if out_bf16 else 0), _stream())
-    return y
+    return _matmul("qe_gemm_w4h_ex", w, x, y, w.flags | (OUT_BF16 if out_bf16 else 0))
 
 
 def gemm_w4_i8(w: W4, x, G=64, out_bf16=False, y=None):
@@ -184,8 +200,9 @@ def gemm_w4_i8(w: W4, x, G=64, out_bf16=False, y=None):
     t = x.shape[0]
     assert x.dtype == torch.bfloat16 and x.shape[1] == w.k and x.stride(1) == 1
     y = _out(t, w.n, out_bf16, w.glu, x.device) if y is None else y
-    call("qe_gemm_w4_i8_ex", w.q, w.s, w.n, w.k, x, x.stride(0), y, y.stride(0), t, G,
-         w.flags | (OUT_BF16 if out_bf16 else 0), _stream())
+    _typed("qe_gemm_w4_i8_ex", "ppiipipiiiip")(w.q.data_ptr(), w.s.data_ptr(), w.n, w.k, x.data_ptr(), x.stride(0),
+                                               y.data_ptr(), y.stride(0), t, G,
+                                               w.flags | (OUT_BF16 if out_bf16 else 0), _raw_stream())
     return y
 
 
@@ -218,9 +235,7 @@ def matmul_w4(w: W4, x, out_bf16=False, y=None):
     t = x.shape[0]
     assert x.dtype == torch.bfloat16 and x.shape[1] == w.k and x.stride(1) == 1
     y = _out(t, w.n, out_bf16, w.glu, x.device) if y is None else y
-    call("qe_matmul_w4_ex", w.q, w.s, w.n, w.k, x, x.stride(0), y, y.stride(0), t,
-         w.flags | (OUT_BF16 if out_bf16 else 0), _stream())
-    return y
+    return _matmul("qe_matmul_w4_ex", w, x, y, w.flags | (OUT_BF16 if out_bf16 else 0))
 
 
 def tile_w8(q, s, per_channel=True):
@@ -252,18 +267,14 @@ def gemv_w8(w: W8, x, out_bf16=False, y=None):
     m = x.shape[0]
     assert x.dtype == torch.bfloat16 and x.shape[1] == w.k and x.stride(1) == 1
     y = _out(m, w.n, out_bf16, False, x.device) if y is None else y
-    call("qe_gemv_w8_ex", w.q, w.s, w.n, w.k, x, x.stride(0), y, y.stride(0), m,
-         w.flags | (OUT_BF16 if out_bf16 else 0), _stream())
-    return y
+    return _matmul("qe_gemv_w8_ex", w, x, y, w.flags | (OUT_BF16 if out_bf16 else 0))
 
 
 def gemm_w8(w: W8, x, out_bf16=False, y=None):
     t = x.shape[0]
     assert x.dtype == torch.bfloat16 and x.shape[1] == w.k and x.stride(1) == 1
     y = _out(t, w.n, out_bf16, False, x.device) if y is None else y
-    call("qe_gemm_w8_ex", w.q, w.s, w.n, w.k, x, x.stride(0), y, y.stride(0), t,
-         w.flags | (OUT_BF16 if out_bf16 else 0), _stream())
-    return y
+    return _matmul("qe_gemm_w8_ex", w, x, y, w.flags | (OUT_BF16 if out_bf16 else 0))
 
 
 def gemm_w8a8(w: W8, x, out_bf16=False, y=None):
@@ -272,9 +283,7 @@ def gemm_w8a8(w: W8, x, out_bf16=False, y=None):
     t = x.shape[0]
     assert x.dtype == torch.bfloat16 and x.shape[1] == w.k and x.stride(1) == 1
     y = _out(t, w.n, out_bf16, False, x.device) if y is None else y
-    call("qe_gemm_w8a8_ex", w.q, w.s, w.n, w.k, x, x.stride(0), y, y.stride(0), t,
-         w.flags | (OUT_BF16 if out_bf16 else 0), _stream())
-    return y
+    return _matmul("qe_gemm_w8a8_ex", w, x, y, w.flags | (OUT_BF16 if out_bf16 else 0))
 
 
 def rows8(w: W8, x, y=None):
@@ -358,9 +367,7 @@ class MoE:
         return MoE(recs, E, topk, H, I)
 
     def workspace(self, T):
-        from .qe import lib
-        lib().qe_moe_workspace_bytes.restype = ctypes.c_size_t
-        nb = lib().qe_moe_workspace_bytes(T, self.E, self.topk, self.H, self.I)
+        nb = _typed("qe_moe_workspace_bytes", "iiiii", ctypes.c_size_t)(T, self.E, self.topk, self.H, self.I)
         if self._ws is None or self._ws.numel() < nb:
             if self._ws is not None:
                 self._old_ws.append(self._ws)
@@ -373,8 +380,9 @@ class MoE:
         ws, nb = self.workspace(T)
         if out is None:
             out = torch.empty(T, self.H, dtype=torch.bfloat16 if out_bf16 else torch.float32, device=x.device)
-        call("qe_moe_w4", logits, x, self.records, T, self.E, self.topk, self.H, self.I, out,
-             OUT_BF16 if out_bf16 else 0, ws, ctypes.c_size_t(nb), _stream())
+        _typed("qe_moe_w4", "pppiiiiipipzp")(logits.data_ptr(), x.data_ptr(), self.records.data_ptr(), T, self.E, self.topk,
+                                             self.H, self.I, out.data_ptr(), OUT_BF16 if out_bf16 else 0, ws.data_ptr(),
+                                             nb, _raw_stream())
         return out
 
 
