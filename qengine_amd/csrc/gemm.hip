@@ -8,11 +8,10 @@
 //   LDS: two stages of X [BM][64] and W [BN][64] bf16, rows of 128 B with the 16-byte chunks XOR-swizzled by
 //        (row % 8) so the MFMA fragment reads (32 rows x 16 B per half-wave) spread over the banks
 //   pipeline, per k step: the MFMAs of step k read stage k % 2 while the same waves dequantize step k + 1 into the
-//        other stage; the activations of step k + 1 arrive there by LDS DMA issued at the top of step k. INT4: the
-//        raw records of step k + 2 are DMA'd to LDS at the top of step k and dequantized from LDS a step later.
-//        INT8: the records go through two register sets, loaded at the top of step k for step k + 2. Every step
-//        ends with vmcnt(0), lgkmcnt(0) and one barrier: each load gets a step of MFMA time to arrive, and the VALU
-//        dequantization overlaps the matrix pipe.
+//        other stage; the activations of step k + 1 arrive there by LDS DMA issued at the top of step k. The raw
+//        records of step k + 2 are DMA'd to LDS at the top of step k and dequantized from LDS a step later. Every
+//        step ends with vmcnt(0), lgkmcnt(0) and one barrier: each load gets a step of MFMA time to arrive, and the
+//        VALU dequantization overlaps the matrix pipe.
 //   grid: one block per output tile, tiles ordered so that the 8 XCDs (blockIdx % 8) each sweep a contiguous band
 //        of tiles (their L2 keeps the shared X / W tiles).
 #include "mfma_tile.hpp"
@@ -40,6 +39,9 @@ struct Cfg {
     // both double-buffered after the two stages
     static constexpr int kRaw = BN * 32, kSc = BN * 2;
     static constexpr int kLdsW4 = 2 * kStage + 2 * kRaw + 2 * kSc;
+    // INT8: the records of one k step are twice as long; the scales stay in registers (256 x 256 tiles fill the 160 KB)
+    static constexpr int kRaw8 = BN * 64;
+    static constexpr int kLdsW8 = 2 * kStage + 2 * kRaw8;
 };
 
 template <int FMT, int SDT, int WMT, int WNT>
@@ -99,7 +101,7 @@ __global__ void __launch_bounds__(NTH) gemm_kernel(const uint4* __restrict__ q, 
     //      4 full 16-byte chunks of the bf16 tile (rows g and g + 8, chunks 2 j and 2 j + 1).
     constexpr int NJOB = BN * 2;
     const bool jactive = tid < NJOB;
-    const int jj = tid & 3, jg = (tid >> 2) & 7, jtr = tid >> 5;
+    const int jj = tid & 3, jg = (tid >> 2) & 7, jtr = (tid >> 5) & (BN / 16 - 1);  // (threads without a job: another's)
     const int ntile_last = (N >> 4) - 1;
     // record (tile tl, 64-k step kt) and scales (tile tl, group grp)
     auto w_rec = [&](int tl, int kt) -> const uint4* { return q + ((size_t)tl * (K >> 6) + kt) * 32; };
@@ -138,89 +140,44 @@ __global__ void __launch_bounds__(NTH) gemm_kernel(const uint4* __restrict__ q, 
         *reinterpret_cast<u32x4_v*>(wtile + swz(row, 2 * jj + 1)) = u32x4_v{hi[0], hi[1], hi[2], hi[3]};
     };
 
-    // ---- W, INT8 path: two 16-byte records (slabs of 32 k) per (16-row tile, lane), WREC per thread
-    constexpr int NREC = (BN / 16) * 64;
-    constexpr int WREC = NREC >= NTH ? NREC / NTH : 1;
-    const bool wactive = tid < NREC;
-    struct WSet {
-        u32x4_v wr[W4 ? 1 : WREC];
-        uint16_t sr_lo[W4 ? 1 : WREC], sr_hi[W4 ? 1 : WREC];
-    };
-    WSet wsA, wsB;
-    auto rec_of = [&](int e, int& tr, int& slab, int& wl) {
-        const int r = tid + e * NTH;
-        tr = r >> 6, slab = (r >> 5) & 1, wl = r & 31;
-    };
-    auto load_w8 = [&](WSet& ws, int kt) {
-#pragma unroll
-        for (int e = 0; e < WREC; e++) {
-            int tr, slab, wl;
-            rec_of(e, tr, slab, wl);
-            const size_t tl = (size_t)(n0 >> 4) + tr;
-            const bool v = wactive && n0 + tr * 16 < N;
-            const uint4* p = q + (tl * (K >> 5) + 2 * kt + slab) * 32 + wl;
-            ws.wr[e] = v ? __builtin_nontemporal_load(reinterpret_cast<const u32x4_v*>(p)) : u32x4_v{0u, 0u, 0u, 0u};
-            const int wg = wl >> 2;
-            if (FMT == kFmtW8C) {
-                ws.sr_lo[e] = v ? s[n0 + tr * 16 + wg] : 0;
-                ws.sr_hi[e] = v ? s[n0 + tr * 16 + wg + 8] : 0;
-            } else {
-                const uint16_t* sp = s + (tl * G + (kt >> 1)) * 16;
-                ws.sr_lo[e] = v ? sp[wg] : 0;
-                ws.sr_hi[e] = v ? sp[wg + 8] : 0;
-            }
+    // ---- W, INT8 formats: raw records by LDS DMA too. A step holds two slabs of 32 k, a slab 512 B a tile; a 1 KB wave
+    //      load covers two tiles of a slab, lanes placed as above. A job = dword d of the row pair (g, g + 8) of a tile
+    //      in both slabs: that dword of the 4 records (g, t = 0..3) is 2 full 16-byte chunks. W8: dword d = bytes
+    //      (row g: k, k + 1; row g + 8: k, k + 1) at k = 8 d + 2 t: chunk d of rows g and g + 8. Q8: word d = row
+    //      g + 8 (d % 2), bytes at k0 + {0, 8, 1, 9}, k0 = 16 (d / 2) + 2 t: chunks 2 (d / 2) and + 1 of that row.
+    auto dma_w8 = [&](int kt, unsigned raw) {
+        if (wave < BN / 32) {
+            const int tl = min((n0 >> 4) + 2 * wave + ((lane >> 3) & 1), ntile_last);
+            const uint4* p = q + ((size_t)tl * (K >> 5) + 2 * kt) * 32 + 4 * (lane & 7) + (lane >> 4);
+            dma16(p, lds32 + raw + wave * 1024);
+            dma16(p + 32, lds32 + raw + BN * 32 + wave * 1024);
         }
     };
-    // Lanes t = 0..3 of a quad hold the records (g, t) of one 32-k slab. W8: dword d = the k pair 8 d + 2 t of rows
-    // g / g + 8; Q8: word d = row g + 8 (d % 2), bytes at k0 + {0, 8, 1, 9}, k0 = 16 (d / 2) + 2 t. A 4 x 4 transpose
-    // across the quad (two rounds of DPP exchanges with lanes t ^ 2, then t ^ 1) gives lane t dword / word t of all
-    // four, i.e. whole 8-k chunks, stored as 16-byte chunks (instead of eight 4-byte stores). Record e is dequantized
-    // at step ks = e.
-    auto xpose4 = [&](u32x4_v v) {
-        const int t = lane & 3;
-        const bool b = (t & 2) != 0, c = (t & 1) != 0;
-        int r0 = __builtin_amdgcn_mov_dpp((int)(b ? v[0] : v[2]), 0x4E, 0xF, 0xF, false);  // quad_perm [2,3,0,1]
-        int r1 = __builtin_amdgcn_mov_dpp((int)(b ? v[1] : v[3]), 0x4E, 0xF, 0xF, false);
-        v = u32x4_v{b ? (uint32_t)r0 : v[0], b ? (uint32_t)r1 : v[1], b ? v[2] : (uint32_t)r0, b ? v[3] : (uint32_t)r1};
-        r0 = __builtin_amdgcn_mov_dpp((int)(c ? v[0] : v[1]), 0xB1, 0xF, 0xF, false);  // quad_perm [1,0,3,2]
-        r1 = __builtin_amdgcn_mov_dpp((int)(c ? v[2] : v[3]), 0xB1, 0xF, 0xF, false);
-        return u32x4_v{c ? (uint32_t)r0 : v[0], c ? v[1] : (uint32_t)r0, c ? (uint32_t)r1 : v[2], c ? v[3] : (uint32_t)r1};
+    const int jtl = min((n0 >> 4) + jtr, ntile_last);
+    // raw scales of rows g and g + 8 of this thread's tile for global step kt
+    auto load_s8 = [&](int kt, uint16_t (&r)[2]) {
+        const uint16_t* p = FMT == kFmtW8C ? s + (size_t)jtl * 16 : s + ((size_t)jtl * G + (kt >> 1)) * 16;
+        r[0] = p[jg];
+        r[1] = p[jg + 8];
     };
-    auto store_w8x = [&](const WSet& ws, char* wtile, int e) {
-        if (!wactive || e >= WREC) return;
-        int tr, slab, wl;
-        rec_of(e, tr, slab, wl);
-        const int row = tr * 16 + (wl >> 2);
-        const float s_lo = scale_rt<SDT>(ws.sr_lo[e], sdt), s_hi = scale_rt<SDT>(ws.sr_hi[e], sdt);
-        const float b_lo = -1152.f * s_lo, b_hi = -1152.f * s_hi;  // qe_tile::dq_pair's W8 bias
-        const u32x4_v tv = xpose4(ws.wr[e]);  // tv[t'] = dword (lane t) of record (g, t')
+    // unit (slab, t) of the dequantization: word t of the job -> one bf16 pair of either chunk; after t = 3 the stores
+    auto unit_w8 = [&](char* wtile, uint32_t word, const float (&sc)[2], int slab, int t, uint32_t (&lo)[4], uint32_t (&hi)[4]) {
+        const uint32_t x = word ^ 0x80808080u;  // w + 128
         if constexpr (FMT == kFmtQ8) {
-            // Q8 word 2 s + h: row g + 8 h, bytes at k0 + {0, 8, 1, 9}, k0 = 32 slab + 16 s + 2 t: lane t now holds
-            // word t of the quad, i.e. row g + 8 (t % 2) at chunks 4 slab + 2 (t / 2) (bytes 0, 2) and + 1 (bytes 1, 3)
-            const int t = wl & 3;
-            const float sc = (t & 1) ? s_hi : s_lo, bs = -1152.f * sc;
-            uint32_t a[4], b[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const uint32_t x = tv[u] ^ 0x80808080u;  // w + 128
-                a[u] = dq_pair(magic_f16<kSel02>(x), sc, bs);
-                b[u] = dq_pair(magic_f16<kSel13>(x), sc, bs);
-            }
-            const int qrow = row + 8 * (t & 1), ch = 4 * slab + 2 * (t >> 1);
-            *reinterpret_cast<u32x4_v*>(wtile + swz(qrow, ch)) = u32x4_v{a[0], a[1], a[2], a[3]};
-            *reinterpret_cast<u32x4_v*>(wtile + swz(qrow, ch + 1)) = u32x4_v{b[0], b[1], b[2], b[3]};
-            return;
+            const float v = (jj & 1) ? sc[1] : sc[0], bs = -1152.f * v;  // qe_tile::dq_pair's W8 bias
+            lo[t] = dq_pair(magic_f16<kSel02>(x), v, bs);
+            hi[t] = dq_pair(magic_f16<kSel13>(x), v, bs);
+        } else {
+            lo[t] = dq_pair(magic_f16<kSel01>(x), sc[0], -1152.f * sc[0]);
+            hi[t] = dq_pair(magic_f16<kSel23>(x), sc[1], -1152.f * sc[1]);
         }
-        uint32_t lo[4], hi[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const uint32_t x = tv[u] ^ 0x80808080u;  // w + 128
-            lo[u] = dq_pair(magic_f16<kSel01>(x), s_lo, b_lo);
-            hi[u] = dq_pair(magic_f16<kSel23>(x), s_hi, b_hi);
+        if (t == 3 && (NJOB >= NTH || jactive)) {
+            const int row = jtr * 16 + jg, ch = 4 * slab;
+            const int r0 = FMT == kFmtQ8 ? row + 8 * (jj & 1) : row, c0 = FMT == kFmtQ8 ? ch + 2 * (jj >> 1) : ch + jj;
+            const int r1 = FMT == kFmtQ8 ? r0 : row + 8, c1 = FMT == kFmtQ8 ? c0 + 1 : c0;
+            *reinterpret_cast<u32x4_v*>(wtile + swz(r0, c0)) = u32x4_v{lo[0], lo[1], lo[2], lo[3]};
+            *reinterpret_cast<u32x4_v*>(wtile + swz(r1, c1)) = u32x4_v{hi[0], hi[1], hi[2], hi[3]};
         }
-        const int ch = 4 * slab + (wl & 3);
-        *reinterpret_cast<u32x4_v*>(wtile + swz(row, ch)) = u32x4_v{lo[0], lo[1], lo[2], lo[3]};
-        *reinterpret_cast<u32x4_v*>(wtile + swz(row + 8, ch)) = u32x4_v{hi[0], hi[1], hi[2], hi[3]};
     };
 
     // ---- MFMA tiles: wave (wm, wn) owns tokens wm * 32 WMT .. , rows wn * 32 WNT ..
@@ -241,9 +198,7 @@ __global__ void __launch_bounds__(NTH) gemm_kernel(const uint4* __restrict__ q, 
     // pin: nothing is scheduled across those calls, so the work placed in them keeps its place among the MFMAs
     // (the INT4 dequantization: left to the scheduler it clusters into one VALU block per k16 step, during which
     // the wave issues no MFMA).
-    auto mfma_step = [&](int kt, auto&& pre, auto&& between, auto pin) {
-        const char* xt = lds + (kt & 1) * C::kStage;
-        const char* wt = xt + BM * BK * 2;
+    auto mfma_step = [&](const char* xt, const char* wt, auto&& pre, auto&& between, auto pin) {
         // fragments of lane l: row l % 32, k = 16 ks + 8 (l / 32) .. + 8 -> chunk 2 ks + l / 32; the reads of k16
         // step ks + 1 are issued before the MFMAs of step ks
         // (every fragment row block is 32-aligned, so the swizzled offset is a per-lane part + a constant)
@@ -316,7 +271,8 @@ __global__ void __launch_bounds__(NTH) gemm_kernel(const uint4* __restrict__ q, 
             const uint32_t* rw = reinterpret_cast<const uint32_t*>(rnext + (jtr >> 1) * 1024) + (8 * (jtr & 1) + jg) * 4 + jj;
             uint32_t wd[4], lo[2][4], hi[2][4];
             float scl[2];
-            mfma_step(kt, [&] {
+            const char* xt = lds + (kt & 1) * C::kStage;
+            mfma_step(xt, xt + BM * BK * 2, [&] {
                 if constexpr (MORE) {
 #pragma unroll
                     for (int t = 0; t < 4; t++) wd[t] = rw[64 * t];
@@ -345,32 +301,69 @@ __global__ void __launch_bounds__(NTH) gemm_kernel(const uint4* __restrict__ q, 
         for (int kt = 0; kt + 1 < KTL; kt++) kstep(kt, std::true_type{});
         kstep(KTL - 1, std::false_type{});
     } else {
-        // X by LDS DMA (as the INT4 path), INT8 records through two register sets: step kt issues the DMA of X
-        // (kt + 1) and the record loads of kt + 2 at its top, dequantizes the records of kt + 1 (loaded one step
-        // earlier) into the other stage during its MFMAs, and ends with vmcnt(0) + the barrier.
-        dma_x(kt0, 0);
-        load_w8(wsA, kt0);
-        if (KTL > 1) load_w8(wsB, kt0 + 1);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // As the INT4 path: X and the raw records by LDS DMA at the top of a step, a thread's 2 x 4 words read there, its
+        // 8 (slab, word) units pinned after every NSLOT / 8-th MFMA row. The two scales a thread needs are loaded to
+        // registers two steps ahead and converted right after the step's wait (nothing else is in flight there).
+        // Against the records in registers, transposed across quads by DPP, and the units left to the scheduler:
+        // 8192 x 2048, t = 4096 155 -> 137 us, 14176 x 2304, t = 1500 143 -> 124 us, 3760 x 5120, t = 200 30.8 -> 25.2.
+        constexpr unsigned kRawOff = 2 * C::kStage;
+        char* raw = lds + kRawOff;
+        constexpr int NSLOT = (BK / 16) * WMT, STRIDE = NSLOT / 8;
+        static_assert(NSLOT >= 8 && NSLOT % 8 == 0, "eight dequantization units per k step");
+        uint16_t sr[2];
+        float sc[2];
+        auto cvt = [&] {
 #pragma unroll
-        for (int d = 0; d < 4; d++) store_w8x(wsA, lds + BM * BK * 2, d);
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        auto step = [&](int kt, const WSet& cur, WSet& nxt_regs) {
-            char* nxt = lds + ((kt + 1) & 1) * C::kStage;
-            if (kt + 1 < KTL) dma_x(kt0 + kt + 1, ((kt + 1) & 1) * C::kStage);
-            const bool more = kt + 1 < KTL;
-            mfma_step(kt, [] {}, [&](int slot) {
-                if (slot % WMT != WMT - 1) return;  // after the last MFMA row of k16 step ks
-                const int ks = slot / WMT;
-                if (more) store_w8x(cur, nxt + BM * BK * 2, ks);
-                if (ks == 0 && kt + 2 < KTL) load_w8(nxt_regs, kt0 + kt + 2);  // after the first stores free no registers
-            }, std::false_type{});
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            for (int h = 0; h < 2; h++) sc[h] = scale_rt<SDT>(sr[h], sdt);
         };
-        for (int kt = 0; kt < KTL; kt += 2) {
-            step(kt, wsB, wsA);
-            if (kt + 1 < KTL) step(kt + 1, wsA, wsB);
+        dma_x(kt0, 0);
+        dma_w8(kt0, kRawOff);
+        dma_w8(kt0 + 1, kRawOff + C::kRaw8);
+        load_s8(kt0, sr);
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        cvt();
+        auto words = [&](const char* r, uint32_t (&wd)[2][4]) {
+#pragma unroll
+            for (int sl = 0; sl < 2; sl++) {
+                const uint32_t* rw = reinterpret_cast<const uint32_t*>(r + sl * BN * 32 + (jtr >> 1) * 1024) +
+                                     (8 * (jtr & 1) + jg) * 4 + jj;
+#pragma unroll
+                for (int t = 0; t < 4; t++) wd[sl][t] = rw[64 * t];
+            }
+        };
+        {
+            uint32_t wd[2][4], lo[4], hi[4];
+            words(raw, wd);
+#pragma unroll
+            for (int un = 0; un < 8; un++) unit_w8(lds + BM * BK * 2, wd[un >> 2][un & 3], sc, un >> 2, un & 3, lo, hi);
         }
+        if constexpr (FMT != kFmtW8C) load_s8(kt0 + 1, sr);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if constexpr (FMT != kFmtW8C) cvt();
+        auto kstep = [&](int kt, auto more) {
+            constexpr bool MORE = decltype(more)::value;
+            char* wnext = lds + ((kt + 1) & 1) * C::kStage + BM * BK * 2;
+            if (MORE) dma_x(kt0 + kt + 1, ((kt + 1) & 1) * C::kStage);
+            if (kt + 2 < KTL) {
+                dma_w8(kt0 + kt + 2, kRawOff + (kt & 1) * C::kRaw8);
+                if constexpr (FMT != kFmtW8C) load_s8(kt0 + kt + 2, sr);
+            }
+            uint32_t wd[2][4], lo[2][4], hi[2][4];
+            const char* xt = lds + (kt & 1) * C::kStage;
+            mfma_step(xt, xt + BM * BK * 2, [&] {
+                if constexpr (MORE) words(raw + ((kt + 1) & 1) * C::kRaw8, wd);
+            }, [&](int slot) {
+                if constexpr (MORE) {
+                    if (slot % STRIDE != STRIDE - 1) return;
+                    const int un = slot / STRIDE;
+                    unit_w8(wnext, wd[un >> 2][un & 3], sc, un >> 2, un & 3, lo[un >> 2], hi[un >> 2]);
+                }
+            }, std::true_type{});
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if constexpr (FMT != kFmtW8C) cvt();
+        };
+        for (int kt = 0; kt + 1 < KTL; kt++) kstep(kt, std::true_type{});
+        kstep(KTL - 1, std::false_type{});
     }
 
     // ---- epilogue. The MFMAs take the W fragments as A and the X fragments as B, so each 32 x 32 tile holds C^T:
@@ -502,14 +495,14 @@ bool gemm_geom(int cfg, int n, int k, int t, int ks, GemmGeom& g) {
 // Predicted time in us of a choice: the k steps of the fullest CU at a measured cost per step, which falls when only
 // part of the CUs run (clock, shared caches), plus the partial sums written and read again. Fitted to sweeps of every
 // (configuration, ks <= 16) on (n, k) from 1280 x 4224 to 34816 x 5120, t = 70..4000 (MI355X; INT4 26 shapes 5.4 % rms,
-// INT8 15 shapes 5.4 % rms, whose record transpose makes its steps longer): the lowest prediction is within 9 % of
-// the best measured choice at every one of them. What it replaces for shapes whose tiles leave CUs idle (256 x 128
+// INT8, whose dequantization is a little longer, 20 shapes 5.7 % rms): the lowest prediction is within 9 % of the best
+// measured choice at every one of them. What it replaces for shapes whose tiles leave CUs idle (256 x 128
 // tiles, one K range): 5120 x 17408, t = 200 (40 tiles) 240 -> 58 us with 20 tiles of 256 x 256 in 12 ranges;
 // 34816 x 5120 GLU, t = 200 (272 tiles, two rounds) 163 -> 108 us with the last 16 tiles in 10 ranges; 5120 x 17408,
-// t = 1000 272 -> 174 us; 2976 x 7936, t = 75 114 -> 22 us; INT8 1280 x 7168, t = 100 129 -> 22 us.
+// t = 1000 272 -> 174 us; 2976 x 7936, t = 75 114 -> 22 us; INT8 1280 x 7168, t = 100 104 -> 20 us.
 double gemm_cost_us(bool w8, int cfg, int n, int k, int t, const GemmGeom& g) {
-    static const double kFull[2][kNumCfg] = {{1.652, 1.014, 1.027, 1.112}, {2.097, 1.360, 1.640, 1.451}};
-    static const double kPart[2][kNumCfg] = {{1.216, 0.797, 0.807, 0.649}, {1.704, 1.026, 1.318, 0.968}};
+    static const double kFull[2][kNumCfg] = {{1.652, 1.014, 1.027, 1.112}, {1.832, 1.069, 1.128, 1.197}};
+    static const double kPart[2][kNumCfg] = {{1.216, 0.797, 0.807, 0.649}, {1.343, 0.814, 0.824, 0.660}};
     const double full_us = kFull[w8][cfg], part_us = kPart[w8][cfg];  // per 64-k step: every slot filled, few
     const CfgDims d = cfg_dims(cfg);
     auto phase = [&](int blocks, int steps) {
@@ -548,7 +541,7 @@ void launch_cfg(const uint4* q, const uint16_t* s, int n, int k, const uint16_t*
     sp.part = part;
     const int per = (g.ndirect + 7) / 8;
     const unsigned blocks = (unsigned)(8 * per) + split_blocks(g.nsplit, g.ks);
-    gemm_kernel<FMT, SDT, WMT, WNT><<<dim3(blocks), dim3(NTH), FMT == kFmtW4 ? C::kLdsW4 : 2 * C::kStage, st>>>(
+    gemm_kernel<FMT, SDT, WMT, WNT><<<dim3(blocks), dim3(NTH), FMT == kFmtW4 ? C::kLdsW4 : C::kLdsW8, st>>>(
         q, s, n, k, x, ldx, t, c, ldc, out, sdt, g.nbn, g.nbt, sp);
     HIP_CHECK(hipGetLastError());
     if (g.nsplit > 0) {
