@@ -104,7 +104,7 @@ void qe_config_set(const QeConfig& c);
 void gemv_w8(const W8& w, const uint16_t* x, int ldx, void* y, int ldy, int m, bool out_bf16, hipStream_t st);
 
 // ---- library-owned workspaces, one per (kind, device, stream) (workspace.cpp) ----
-enum WsKind : int { kWsSplit = 0, kWsI8 = 1, kWsH = 2, kWsDec = 3, kNumWs = 4 };
+enum WsKind : int { kWsSplit = 0, kWsI8 = 1, kWsH = 2, kWsDec = 3, kWsSkinny = 4, kNumWs = 5 };
 // the buffer of (kind, current device, st), at least `bytes`: grown outside graph capture (the outgrown one kept
 // allocated); nullptr during capture when it is too small. kWsDec buffers (the one-pass decode's tail counters and
 // sums) are zero-filled when allocated; the kernel leaves its counters zero.

@@ -82,12 +82,17 @@ constexpr int skinny_wsz() {  // dwords of LDS per wave: xl [UPX ? NGM : 2][MT][
 // exact integers in fp16 (Q8: w / 16), f16 MFMAs, every 64-k chunk's partial rounded to fp16 and flushed into fp32
 // with the group scale x 16 (Q8 x 256)); W4 and Q8 only
 // UA: activation rows only 4-byte aligned (x or ldx not 16-byte aligned): each 16-byte piece is loaded as 4 dwords
-template <int MT, int SDT, int NG, int RT, int FMT, bool H16 = false, bool UA = false, int D = skinny_d<MT, NG, RT, FMT>(),
-          int WPE = skinny_wpe<MT, NG, RT, FMT>()>
-__global__ void __launch_bounds__(64 * (NG > 0 ? kMaxWaves : kMaxWavesGeneric))
+// PART: a tile's slices run in blocks of kPartWaves waves (block y: slices kPartWaves y ..), each slice's sums go to
+// part [tile][slice][16 tok][16 rows] and skinny_sum_kernel adds them in slice order: the bits of the one-block form
+constexpr int kPartWaves = 4;
+template <int MT, int SDT, int NG, int RT, int FMT, bool H16 = false, bool UA = false, bool PART = false,
+          int D = skinny_d<MT, NG, RT, FMT>(), int WPE = PART ? 4 : skinny_wpe<MT, NG, RT, FMT>()>
+__global__ void __launch_bounds__(64 * (PART ? kPartWaves : NG > 0 ? kMaxWaves : kMaxWavesGeneric))
 __attribute__((amdgpu_waves_per_eu(WPE))) skinny_kernel(
     const uint4* __restrict__ q, const uint16_t* __restrict__ s, int N, int K, const uint16_t* __restrict__ x,
-    int ldx, void* __restrict__ y, int ldy, int m, int out, int sdt, uint16_t* __restrict__ yh = nullptr, int ldyh = 0) {
+    int ldx, void* __restrict__ y, int ldy, int m, int out, int sdt, uint16_t* __restrict__ yh = nullptr, int ldyh = 0,
+    float* __restrict__ part = nullptr, int nslices = 0) {
+    static_assert(!PART || (RT == 1 && MT == 16), "parts of one tile, 16 rows");
     constexpr int NGM = NG > 0 ? NG : kGenericNG;
     constexpr bool UPX = skinny_upx<MT, NG>();
     constexpr int WSZ = skinny_wsz<MT, NG, RT>();
@@ -95,11 +100,13 @@ __attribute__((amdgpu_waves_per_eu(WPE))) skinny_kernel(
     // the same A (weight) operand; every row's arithmetic is that of MT = 16 (MFMA columns are independent)
     constexpr int NB = MT > 16 ? MT / 16 : 1, MTR = MT > 16 ? MT : 16;
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
-    const int S = blockDim.x >> 6, w = threadIdx.x >> 6, L = threadIdx.x & 63;
+    const int S = PART ? nslices : blockDim.x >> 6, lw = threadIdx.x >> 6, L = threadIdx.x & 63;
+    const int w = PART ? (int)blockIdx.y * kPartWaves + lw : lw;  // the wave's slice
+    if (PART && w >= S) return;  // (no block barrier below in this form)
     const int tile0 = blockIdx.x * RT, G = K >> 7;
     const int gb = NG > 0 ? w * NG : w * G / S;
     const int ng = NG > 0 ? NG : (w + 1) * G / S - gb;
-    uint32_t* xl = lds + (size_t)w * WSZ;
+    uint32_t* xl = lds + (size_t)lw * WSZ;
     uint16_t* sl16 = reinterpret_cast<uint16_t*>(xl + (WSZ - RT * NGM * 8));
     float* red = reinterpret_cast<float*>(lds);  // wave w's [RT][16 tok][16 rows] at w * WSZ (its staging area)
 
@@ -390,6 +397,10 @@ __attribute__((amdgpu_waves_per_eu(WPE))) skinny_kernel(
     }
     }
 
+    if constexpr (PART) {
+        *reinterpret_cast<f32x4_v*>(part + ((size_t)tile0 * S + w) * 256 + i * 16 + 4 * qg) = acc[0][0];
+        return;
+    }
     // 2. slices through LDS in a fixed order: wave w's sums over its own staging area (its last LDS reads come
     //    first: a wave's LDS operations complete in order), lane (qg, i) holds rows 4 qg .. + 3 of column i
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -436,6 +447,46 @@ __attribute__((amdgpu_waves_per_eu(WPE))) skinny_kernel(
     }
 }
 
+// PART's second launch: one thread per output of a tile, its S slice sums added in slice order, and the epilogue of
+// skinny_kernel. Reads are consecutive across lanes.
+__global__ void __launch_bounds__(256) skinny_sum_kernel(const float* __restrict__ part, int S, void* __restrict__ y, int ldy,
+                                                         int m, int out) {
+    const float* p = part + (size_t)blockIdx.x * S * 256;
+    auto sum = [&](int tok, int rr) {
+        float b[kMaxWavesGeneric];
+#pragma unroll
+        for (int ws = 0; ws < kMaxWavesGeneric; ws++) b[ws] = p[(ws < S ? ws : S - 1) * 256 + tok * 16 + rr];
+        float v = 0.f;
+#pragma unroll
+        for (int ws = 0; ws < kMaxWavesGeneric; ws++) v = ws < S ? v + b[ws] : v;
+        return v;
+    };
+    if (out == kOutGLU) {
+        const int tok = threadIdx.x >> 3, gg = threadIdx.x & 7;
+        if (tok >= m) return;  // (and every thread past 16 x 8: m <= 16)
+        const float v = silu_f32(sum(tok, gg)) * sum(tok, gg + 8);
+        reinterpret_cast<uint16_t*>(y)[(size_t)tok * ldy + 8 * blockIdx.x + gg] = f32_to_bf16(v);
+    } else {
+        const int tok = threadIdx.x >> 4, rr = threadIdx.x & 15;
+        if (tok >= m) return;
+        const float v = sum(tok, rr);
+        const size_t o = (size_t)tok * ldy + 16 * blockIdx.x + rr;
+        if (out == kOutBF16) reinterpret_cast<uint16_t*>(y)[o] = f32_to_bf16(v);
+        else reinterpret_cast<float*>(y)[o] = v;
+    }
+}
+
+// Whether 16-row launches on uneven slices run in PART form. What bounds the one-block form: its S waves stage 9 KB each
+// (12 waves: 108 KB of the CU's 160), so one block runs per CU and the tiles past the last whole round of CUs run in a
+// round of their own (320 tiles: 64 CUs hold two). Blocks of four waves run four to a CU: up to 4 blocks per CU
+// everything is resident at once. us, one block -> parts, with the second launch, m = 9 / 16: N = 4608, K = 17408 24.1 /
+// 29.2 -> 19.4 / 23.0; N = 5120, K = 17408 24.4 / 29.5 -> 19.5 / 23.2 (m = 12 26.2 -> 20.9, 46 MB at 2.2 TB/s); N = 5120,
+// K = 13824 20.2 / 23.8 -> 16.6 / 19.1; past the line N = 8192 27.1 / 31.0 -> 29.2 / 32.8.
+inline bool part_pays(int tiles, int S) {
+    const int cus = qe_num_cus(), parts = (S + kPartWaves - 1) / kPartWaves;
+    return S > 8 && tiles > cus && tiles * parts <= 4 * cus;
+}
+
 template <int FMT, int SDT, bool H16 = false, bool UA = false>
 void launch(const uint4* q, const uint16_t* s, int n, int k, const uint16_t* x, int ldx, void* y, int ldy, int m,
             int out, int sdt, hipStream_t st, uint16_t* yh = nullptr, int ldyh = 0) {
@@ -446,6 +497,20 @@ void launch(const uint4* q, const uint16_t* s, int n, int k, const uint16_t* x, 
     const int mt = m == 1 ? 1 : m == 2 ? 2 : m <= 4 ? 4 : m <= 8 ? 8 : m <= 16 ? 16 : 32;
     CHECK(mt <= 16 || FMT == qe_gemv::kFmtW4, "skinny: %d rows per launch (32-row launches: INT4 only)", m);
     const dim3 block(64 * sc.S);
+    if constexpr (FMT == kFmtW4 && !H16 && !UA) {
+        if (mt == 16 && sc.ng == 0 && part_pays(n / 16, sc.S)) {
+            // no workspace (a capture that was not warmed up): one block per tile below, the same bits
+            if (float* part = static_cast<float*>(stream_ws(kWsSkinny, (size_t)(n / 16) * sc.S * 256 * 4, st))) {
+                skinny_kernel<16, SDT, 0, 1, FMT, false, false, true>
+                    <<<dim3((unsigned)(n / 16), (unsigned)((sc.S + kPartWaves - 1) / kPartWaves)), dim3(64 * kPartWaves),
+                       (size_t)kPartWaves * skinny_wsz<16, 0, 1>() * 4, st>>>(q, s, n, k, x, ldx, y, ldy, m, out, sdt,
+                                                                              nullptr, 0, part, sc.S);
+                skinny_sum_kernel<<<dim3((unsigned)(n / 16)), dim3(256), 0, st>>>(part, sc.S, y, ldy, m, out);
+                HIP_CHECK(hipGetLastError());
+                return;
+            }
+        }
+    }
     // two tiles per wave (where n / 16 is even) at m >= 5, and for m <= 4 on grids of fewer than 16 waves per CU at
     // one tile per wave. Measured (K = 5120): RT = 2 is 3 % slower at m = 2, 4 on N = 17408 (8704 waves), 3 % faster
     // at m = 8, 13 % faster at m = 16 (two blocks per CU since the partial sums reuse the staging LDS), and 6 to 16 %

@@ -1,5 +1,6 @@
 // Library-owned workspaces of the prefill GEMMs (split-K partial sums, the W4A8 / W8A8 and fp16-accumulate
-// pre-pass buffers) and of the one-pass decode's tail (counters and part sums), one buffer per (kind, device, stream).
+// pre-pass buffers), of the one-pass decode's tail (counters and part sums) and of the skinny kernel's slice sums, one
+// buffer per (kind, device, stream).
 //
 // The reference keeps these buffers thread_local (src/kernels/gemm.cu:3258-3368), so two host threads never share
 // one. Here the key is the stream a call is enqueued on: calls on one stream run in order, so they can share a

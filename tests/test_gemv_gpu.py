@@ -565,3 +565,46 @@ def test_measurement_probes(dev):
     call("qe_read_probe", w.q, n, k, sink, ops._stream())
     torch.cuda.synchronize()
     assert int((sink != 0).sum()) <= 1
+
+
+@pytest.mark.parametrize("n,k,glu", [(4112, 13824, False), (5120, 17408, False), (5440, 17408, False),
+                                     (5120, 17408, True)])
+@pytest.mark.parametrize("m", [9, 12, 16])
+def test_skinny_slices_in_parts(dev, n, k, glu, m):
+    """9..16 rows on K without an even slicing, 257..341 tiles: a tile's slices run in blocks of four waves and a second
+    launch adds them in slice order (257, 320, 340 tiles). Within 1e-4 * rms
+    of the exact product; a row's bits are those of the row in calls of 2 rows (one block per tile, the same slices), of
+    repeated calls, and of a graph captured on a stream without the workspace (one block per tile) or with it"""
+    w, q, s = setup_w4(n, k, 1, seed=n + m, glu=glu)
+    xh = synth.x_host(m, k, seed=k + m)
+    x = synth.to_dev(xh)
+    y = ops.gemv_w4(w, x)
+    yb = y if glu else ops.gemv_w4(w, x, out_bf16=True)
+    pairs = torch.cat([ops.gemv_w4(w, x[i:i + 2].contiguous()) for i in range(m - 1)])
+    torch.cuda.synchronize()
+    exact = matmul_f64(xh, exact_w4(q, s, n, k, 1))
+    if glu:
+        assert_glu_close(out_f32(y), glu_act(exact), 1e-4)
+    else:
+        assert err_ratio(y.cpu().numpy(), exact) <= 1e-4
+        assert torch.equal(yb, y.bfloat16())
+    assert torch.equal(pairs[0::2], y[:-1]) and torch.equal(pairs[-1], y[-1])
+    for warm in (False, True):
+        cs = torch.cuda.Stream()
+        cs.wait_stream(torch.cuda.current_stream())
+        x_in, out = x.clone(), torch.empty_like(y)
+        if warm:
+            with torch.cuda.stream(cs):
+                ops.gemv_w4(w, x_in, y=out)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=cs):
+            ops.gemv_w4(w, x_in, y=out)
+        for r in range(3):
+            xr = synth.to_dev(synth.x_host(m, k, seed=200 + r))
+            want = ops.gemv_w4(w, xr)
+            torch.cuda.synchronize()
+            x_in.copy_(xr)
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), (warm, r)
