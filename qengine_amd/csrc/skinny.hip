@@ -32,7 +32,8 @@ using namespace qe_gemv;
 
 // Tiles per wave RT: the weight tiles of RT consecutive 16-row tiles share one wave's staged activations and B
 // operand reads (the activation traffic per tile halves at RT = 2). Even slices can take RT = 2 (the host picks it
-// in launch()), uneven slices (NG = 0) at MT = 2..8 (16 rows at RT = 2 spill: N = 5120, K = 17408 29.8 -> 55.9 us).
+// in launch()), uneven slices (NG = 0) at MT = 2..8 (16 rows at RT = 2 spill in one block per tile: N = 5120, K = 17408 29.8 -> 55.9
+// us; in parts they do not: part_pays).
 // Measured on uneven slices, RT = 1 -> 2: N = 5120, K = 17408, m = 2 / 4 / 8 15.7 / 16.3 / 21.6 -> 14.8 / 14.8 / 16.0
 // us; K = 13824 13.0 / 13.7 / 17.6 -> 12.2 / 12.2 / 13.1 us; N = 8192, K = 17408, m = 8 24.5 -> 17.5 us. Weight
 // groups in flight per wave D and the occupancy hint WPE, measured on the BASELINE shapes (K = 5120, 5-group slices;
@@ -86,13 +87,13 @@ constexpr int skinny_wsz() {  // dwords of LDS per wave: xl [UPX ? NGM : 2][MT][
 // part [tile][slice][16 tok][16 rows] and skinny_sum_kernel adds them in slice order: the bits of the one-block form
 constexpr int kPartWaves = 4;
 template <int MT, int SDT, int NG, int RT, int FMT, bool H16 = false, bool UA = false, bool PART = false,
-          int D = skinny_d<MT, NG, RT, FMT>(), int WPE = PART ? 4 : skinny_wpe<MT, NG, RT, FMT>()>
+          int D = skinny_d<MT, NG, RT, FMT>(), int WPE = PART ? (RT == 2 ? 2 : 4) : skinny_wpe<MT, NG, RT, FMT>()>
 __global__ void __launch_bounds__(64 * (PART ? kPartWaves : NG > 0 ? kMaxWaves : kMaxWavesGeneric))
 __attribute__((amdgpu_waves_per_eu(WPE))) skinny_kernel(
     const uint4* __restrict__ q, const uint16_t* __restrict__ s, int N, int K, const uint16_t* __restrict__ x,
     int ldx, void* __restrict__ y, int ldy, int m, int out, int sdt, uint16_t* __restrict__ yh = nullptr, int ldyh = 0,
     float* __restrict__ part = nullptr, int nslices = 0) {
-    static_assert(!PART || (RT == 1 && MT == 16), "parts of one tile, 16 rows");
+    static_assert(!PART || MT == 16, "16 rows");
     constexpr int NGM = NG > 0 ? NG : kGenericNG;
     constexpr bool UPX = skinny_upx<MT, NG>();
     constexpr int WSZ = skinny_wsz<MT, NG, RT>();
@@ -398,7 +399,9 @@ __attribute__((amdgpu_waves_per_eu(WPE))) skinny_kernel(
     }
 
     if constexpr (PART) {
-        *reinterpret_cast<f32x4_v*>(part + ((size_t)tile0 * S + w) * 256 + i * 16 + 4 * qg) = acc[0][0];
+#pragma unroll
+        for (int r = 0; r < RT; r++)
+            *reinterpret_cast<f32x4_v*>(part + ((size_t)(tile0 + r) * S + w) * 256 + i * 16 + 4 * qg) = acc[r][0];
         return;
     }
     // 2. slices through LDS in a fixed order: wave w's sums over its own staging area (its last LDS reads come
@@ -476,15 +479,25 @@ __global__ void __launch_bounds__(256) skinny_sum_kernel(const float* __restrict
     }
 }
 
-// Whether 16-row launches on uneven slices run in PART form. What bounds the one-block form: its S waves stage 9 KB each
-// (12 waves: 108 KB of the CU's 160), so one block runs per CU and the tiles past the last whole round of CUs run in a
-// round of their own (320 tiles: 64 CUs hold two). Blocks of four waves run four to a CU: up to 4 blocks per CU
-// everything is resident at once. us, one block -> parts, with the second launch, m = 9 / 16: N = 4608, K = 17408 24.1 /
-// 29.2 -> 19.4 / 23.0; N = 5120, K = 17408 24.4 / 29.5 -> 19.5 / 23.2 (m = 12 26.2 -> 20.9, 46 MB at 2.2 TB/s); N = 5120,
-// K = 13824 20.2 / 23.8 -> 16.6 / 19.1; past the line N = 8192 27.1 / 31.0 -> 29.2 / 32.8.
-inline bool part_pays(int tiles, int S) {
-    const int cus = qe_num_cus(), parts = (S + kPartWaves - 1) / kPartWaves;
-    return S > 8 && tiles > cus && tiles * parts <= 4 * cus;
+// Whether 16-row launches on uneven slices run in PART form, RT tiles per wave. What bounds the one-block form: its S
+// waves stage 9 KB each (12 waves: 108 KB of the CU's 160), so one block runs per CU and the tiles past the last whole
+// round of CUs run in a round of their own (320 tiles: 64 CUs hold two); and with up to 16 waves a block has no
+// registers for two tiles a wave, so every tile stages all activation rows (178 MB at N = 5120, K = 17408 for 45 MB of
+// weights). Blocks of four waves run four to a CU and hold two tiles a wave (135 VGPRs, no spill) where n / 16 is even.
+// us, one block -> RT = 1 -> RT = 2, with the second launch:
+//   N x K           m = 9                 m = 12                m = 16
+//   4608 x 17408    24.4 -> 19.4 -> 17.2  26.0 ->      -> 17.6  29.2 -> 23.0 -> 18.5
+//   5120 x 17408    24.4 -> 19.5 -> 17.7  26.1 -> 20.9 -> 17.8  29.4 -> 23.2 -> 19.1
+//   5120 x 13824    20.7 -> 16.6 -> 15.0  21.2 -> 17.4 -> 15.2  23.8 -> 19.1 -> 16.1
+//   5120 x 28672    35.6 -> 30.4 -> 24.3  39.1 -> 31.7 -> 25.5  44.6 -> 34.1 -> 28.1
+//   8192 x 17408    27.2 -> 29.2 -> 23.1  28.0 ->      -> 23.8  30.9 -> 32.8 -> 26.7
+//  12288 x 13824    31.1 ->      -> 26.6  31.9 ->      -> 27.5  33.6 ->      -> 30.2
+// One tile a wave: only where the parts are all resident (four to a CU). Tiles that fill one round of CUs stay (N =
+// 4096, K = 13824, m = 9 / 16: 12.2 / 13.7 -> 13.0 / 14.6); fewer, shorter K than 12288 and more tiles than three
+// rounds were not measured and stay too (on a short K the second launch, ~2 us, is not paid back).
+inline bool part_pays(int n, int k, int S) {
+    const int cus = qe_num_cus(), tiles = n / 16, parts = (S + kPartWaves - 1) / kPartWaves;
+    return k >= 12288 && tiles > cus && (n % 32 == 0 ? tiles <= 3 * cus : tiles * parts <= 4 * cus);
 }
 
 template <int FMT, int SDT, bool H16 = false, bool UA = false>
@@ -498,13 +511,19 @@ void launch(const uint4* q, const uint16_t* s, int n, int k, const uint16_t* x, 
     CHECK(mt <= 16 || FMT == qe_gemv::kFmtW4, "skinny: %d rows per launch (32-row launches: INT4 only)", m);
     const dim3 block(64 * sc.S);
     if constexpr (FMT == kFmtW4 && !H16 && !UA) {
-        if (mt == 16 && sc.ng == 0 && part_pays(n / 16, sc.S)) {
+        if (mt == 16 && sc.ng == 0 && part_pays(n, k, sc.S)) {
             // no workspace (a capture that was not warmed up): one block per tile below, the same bits
             if (float* part = static_cast<float*>(stream_ws(kWsSkinny, (size_t)(n / 16) * sc.S * 256 * 4, st))) {
-                skinny_kernel<16, SDT, 0, 1, FMT, false, false, true>
-                    <<<dim3((unsigned)(n / 16), (unsigned)((sc.S + kPartWaves - 1) / kPartWaves)), dim3(64 * kPartWaves),
-                       (size_t)kPartWaves * skinny_wsz<16, 0, 1>() * 4, st>>>(q, s, n, k, x, ldx, y, ldy, m, out, sdt,
-                                                                              nullptr, 0, part, sc.S);
+                const dim3 pb(64 * kPartWaves);
+                const unsigned np = (unsigned)((sc.S + kPartWaves - 1) / kPartWaves);
+                if (n % 32 == 0)
+                    skinny_kernel<16, SDT, 0, 2, FMT, false, false, true>
+                        <<<dim3((unsigned)(n / 32), np), pb, (size_t)kPartWaves * skinny_wsz<16, 0, 2>() * 4, st>>>(
+                            q, s, n, k, x, ldx, y, ldy, m, out, sdt, nullptr, 0, part, sc.S);
+                else
+                    skinny_kernel<16, SDT, 0, 1, FMT, false, false, true>
+                        <<<dim3((unsigned)(n / 16), np), pb, (size_t)kPartWaves * skinny_wsz<16, 0, 1>() * 4, st>>>(
+                            q, s, n, k, x, ldx, y, ldy, m, out, sdt, nullptr, 0, part, sc.S);
                 skinny_sum_kernel<<<dim3((unsigned)(n / 16)), dim3(256), 0, st>>>(part, sc.S, y, ldy, m, out);
                 HIP_CHECK(hipGetLastError());
                 return;

@@ -567,12 +567,13 @@ def test_measurement_probes(dev):
     assert int((sink != 0).sum()) <= 1
 
 
-@pytest.mark.parametrize("n,k,glu", [(4112, 13824, False), (5120, 17408, False), (5440, 17408, False),
-                                     (5120, 17408, True)])
+@pytest.mark.parametrize("n,k,glu", [(4112, 13824, False), (5120, 17408, False), (5424, 17408, False),
+                                     (5120, 17408, True), (4128, 28672, False), (12288, 13824, False)])
 @pytest.mark.parametrize("m", [9, 12, 16])
 def test_skinny_slices_in_parts(dev, n, k, glu, m):
-    """9..16 rows on K without an even slicing, 257..341 tiles: a tile's slices run in blocks of four waves and a second
-    launch adds them in slice order (257, 320, 340 tiles). Within 1e-4 * rms
+    """9..16 rows on K without an even slicing, more tiles than CUs: the slices of a tile (an odd number of tiles: 257,
+    339) or of two (258, 320, 768) run in blocks of four waves, the last block short at K = 28672 (14 slices), and a
+    second launch adds them in slice order. Within 1e-4 * rms
     of the exact product; a row's bits are those of the row in calls of 2 rows (one block per tile, the same slices), of
     repeated calls, and of a graph captured on a stream without the workspace (one block per tile) or with it"""
     w, q, s = setup_w4(n, k, 1, seed=n + m, glu=glu)
