@@ -36,7 +36,8 @@ int qe_num_cus() {
     return c;
 }
 
-// The decode GEMV keeps no device workspace (its K slices are reduced in LDS); the entry point stays for the
+// The decode GEMV needs no device workspace (its K slices are reduced in LDS; 9..16 rows on long K without an even
+// slicing keep slice sums in a per-stream buffer that grows by itself); the entry point stays for the
 // reference's calling convention (gemv_workspace_init once per device before any graph capture).
 void gemv_workspace_init() { qe_num_cus(); }
 

@@ -7,8 +7,8 @@
 // buffer, while calls on two streams of one device (or two graphs replayed on two streams) get two buffers and cannot
 // overwrite each other's data. A buffer grows on a call outside graph capture; the outgrown one is kept allocated
 // (retired, never freed: a graph captured earlier may still read it). During capture a buffer that is too small is
-// not grown: stream_ws returns nullptr and the caller either runs without it (the GEMM's split) or aborts with a
-// message (the pre-passes), so callers size it first with an eager call or stream_ws_reserve on that stream.
+// not grown: stream_ws returns nullptr and the caller either runs without it (the GEMM's split, the decode kernels; they
+// do so too when the device has no memory left for it) or aborts with a message (the pre-passes), so callers size it first with an eager call or stream_ws_reserve on that stream.
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -37,7 +37,12 @@ void* stream_ws(int kind, size_t bytes, hipStream_t st) {
     HIP_CHECK(hipStreamIsCapturing(st, &cs));
     if (cs != hipStreamCaptureStatusNone) return nullptr;
     void* np = nullptr;
-    HIP_CHECK(hipMalloc(&np, bytes));
+    const hipError_t e = hipMalloc(&np, bytes);
+    if (e == hipErrorOutOfMemory && kind != kWsI8 && kind != kWsH) {  // every other caller runs without its buffer
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    HIP_CHECK(e);
     if (kind == kWsDec) {  // counters start at zero (the kernel sets them back to zero at the end of every call)
         HIP_CHECK(hipMemsetAsync(np, 0, bytes, st));
         HIP_CHECK(hipStreamSynchronize(st));
