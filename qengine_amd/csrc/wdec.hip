@@ -1,6 +1,6 @@
 // Decode GEMM for up to 64 activation rows on the W4 layout, one pass over the weights (the reference's wide decode
 // GEMVs, src/kernels/gemv_x.cu:1-12,902-980, read the matrix once for m 9..64). Up to 32 rows: wdec_kernel, described
-// here; 33..64 rows: wdec2_kernel below.
+// here; 33..64 rows: wdec2_kernel below, or this one where its smaller slabs fill the CUs better (small_slabs_pay).
 //
 // The skinny kernel (skinny.hip) stages every activation row of its K slice per wave and multiplies 16-row weight
 // tiles on 16 x 16 MFMAs; past 16 rows its cost is the activation staging and the B operand reads, which grow with m,
@@ -13,7 +13,8 @@
 // nibbles (shifted down) that of row g + 8. The B operand is chunk c of a token row:
 // one ds_read_b128 of the wave's staged activation tile ([32 rows][64 k] bf16, 16-byte chunks XOR-swizzled).
 //
-// Block = 4 waves = KP = 4 contiguous K parts, over one 64-row weight slab (N / 64 blocks). Every wave stages its own activation rows, records and scales by LDS DMA (global_load_lds) into a ring of
+// Block = 4 waves = TB token blocks of 32 rows x KP = 4 / TB contiguous K parts, over one 64-row weight slab (N / 64
+// blocks). Every wave stages its own activation rows, records and scales by LDS DMA (global_load_lds) into a ring of
 // NBUF buffers, DEPTH = NBUF - 1 steps ahead, so no wave waits for another until the end; per 64-k step a wave issues 7 DMAs
 // (four 1 KB activation pieces, two 1 KB record pieces, one 256-byte scale piece), and every wait is a compile-time
 // vmcnt. The next k16 step's A operands are built between the MFMAs of the current one. After the K loop each
@@ -41,23 +42,23 @@ constexpr int kLds = NBUF * NW * kBuf;        // 76800 B: two blocks per CU
 constexpr int kPart = 68;                     // floats per token row of a wave's partial sums (64 rows + pad)
 static_assert(NW * 32 * kPart * 4 <= kLds, "the partial sums fit the staging buffers");
 
-// up to 32 rows; out: 0 fp32, 1 bf16, 2 GLU (bf16 activation, n / 2 columns)
+// TB token blocks of 32 rows (m <= 32 TB), out: 0 fp32, 1 bf16, 2 GLU (bf16 activation, n / 2 columns)
 // Blocks [0, nmain): one slab each over the whole K. Blocks past nmain: part p = u % P of tail slab nmain + u / P
-// (u = block - nmain), over K steps [p KT / P, (p + 1) KT / P); its sums go to tpart[u] ([32 tokens][64 rows]
+// (u = block - nmain), over K steps [p KT / P, (p + 1) KT / P); its sums go to tpart[u] ([TB * 32 tokens][64 rows]
 // fp32, written through to the device-coherent level), then it adds one to tctr[u / P]; the part that brings the
 // count to P adds the P parts in order p = 0..P-1, stores the outputs and sets the count back to zero (the counters
 // are zero when their buffer is allocated). P = 1: no tail blocks.
-template <int SDT>
+template <int SDT, int TB>
 __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ q, const uint16_t* __restrict__ s,
                                                       int K, const uint16_t* __restrict__ x, int ldx, int M,
                                                       void* __restrict__ y, int ldy, int out, int nmain, int P,
                                                       float* __restrict__ tpart, uint32_t* __restrict__ tctr) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
-    constexpr int KP = NW;  // a K part per wave
+    constexpr int KP = NW / TB;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned lds32 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)lds);
-    const int kp = wave;
+    const int tb = wave / KP, kp = wave - tb * KP;
     const int b = blockIdx.x, tail = b >= nmain ? b - nmain : -1;  // tail part index u, or -1
     const int slab = tail < 0 ? b : nmain + tail / P, KTb = tail < 0 ? K / BK : K / BK / P;
     const int KTw = KTb / KP, kt0 = (tail < 0 ? 0 : (tail % P) * KTb) + kp * KTw, G = K >> 7;
@@ -72,8 +73,8 @@ __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ 
     const uint16_t* xsrc[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-        const int row = 8 * r + (lane >> 3);
-        xsrc[r] = x + (size_t)(row < M ? row : M - 1) * ldx + (((lane & 7) ^ swz_f(row)) << 3);
+        const int row = 8 * r + (lane >> 3), tok = 32 * tb + row;
+        xsrc[r] = x + (size_t)(tok < M ? tok : M - 1) * ldx + (((lane & 7) ^ swz_f(row)) << 3);
     }
     const int dtl = tile0 + ((lane >> 3) & 3);
     const uint4* wsrc = q + (size_t)dtl * (K >> 6) * 32 + 4 * (lane & 7) + kh;
@@ -225,12 +226,12 @@ __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ 
             *reinterpret_cast<f32x4_v*>(part + (wave * 32 + mr) * kPart + 16 * qq + 8 * op + 4 * kh) =
                 f32x4_v{acc[op][4 * qq], acc[op][4 * qq + 1], acc[op][4 * qq + 2], acc[op][4 * qq + 3]};
     __syncthreads();
-    // the KP parts added in a fixed tree order (parts i and i + h, h = KP / 2, ..., 1)
-    auto sum4 = [&](int tok, int r4) {  // rows r4 .. r4 + 3 of the slab
+    // the KP parts of a token block added in a fixed tree order (parts i and i + h, h = KP / 2, ..., 1)
+    auto sum4 = [&](int otb, int tok, int r4) {  // rows r4 .. r4 + 3 of the slab
         f32x4_v p[KP];
 #pragma unroll
         for (int k = 0; k < KP; k++)
-            p[k] = *reinterpret_cast<const f32x4_v*>(part + (k * 32 + tok) * kPart + r4);
+            p[k] = *reinterpret_cast<const f32x4_v*>(part + ((otb * KP + k) * 32 + tok) * kPart + r4);
 #pragma unroll
         for (int h = KP / 2; h >= 1; h >>= 1)
 #pragma unroll
@@ -238,29 +239,31 @@ __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ 
         return p[0];
     };
     const int n0 = tile0 * 16;
-    // the epilogue of 4 consecutive rows r4 of token tok, from get4(tok, r4)
+    // the epilogue of 4 consecutive rows r4 of token otb * 32 + tok, from get4(otb, tok, r4)
     auto emit = [&](auto&& get4) {
         if (out == 2) {  // thread = (token, tile, row quad of the 8 gate rows): gate rows g, up rows g + 8
-            for (int o = tid; o < 32 * 8; o += NTH) {
-                const int tok = o >> 3, qq = (o >> 1) & 3, gq = o & 1;
-                if (tok >= M) continue;
-                const f32x4_v ga = get4(tok, 16 * qq + 4 * gq), up = get4(tok, 16 * qq + 8 + 4 * gq);
-                uint16_t* p = reinterpret_cast<uint16_t*>(y) + (size_t)tok * ldy + (tile0 + qq) * 8 + 4 * gq;
+            for (int o = tid; o < TB * 32 * 8; o += NTH) {
+                const int otb = o >> 8, tok = (o >> 3) & 31, qq = (o >> 1) & 3, gq = o & 1;
+                const int t = 32 * otb + tok;
+                if (t >= M) continue;
+                const f32x4_v ga = get4(otb, tok, 16 * qq + 4 * gq), up = get4(otb, tok, 16 * qq + 8 + 4 * gq);
+                uint16_t* p = reinterpret_cast<uint16_t*>(y) + (size_t)t * ldy + (tile0 + qq) * 8 + 4 * gq;
 #pragma unroll
                 for (int i = 0; i < 4; i++) p[i] = f32_to_bf16(silu_f32(ga[i]) * up[i]);
             }
             return;
         }
-        for (int o = tid; o < 32 * 16; o += NTH) {  // thread = (token, 4 consecutive rows)
-            const int tok = o >> 4, r4 = 4 * (o & 15);
-            if (tok >= M) continue;
-            const f32x4_v v = get4(tok, r4);
+        for (int o = tid; o < TB * 32 * 16; o += NTH) {  // thread = (token, 4 consecutive rows)
+            const int otb = o >> 9, tok = (o >> 4) & 31, r4 = 4 * (o & 15);
+            const int t = 32 * otb + tok;
+            if (t >= M) continue;
+            const f32x4_v v = get4(otb, tok, r4);
             if (out == 1) {
-                uint16_t* p = reinterpret_cast<uint16_t*>(y) + (size_t)tok * ldy + n0 + r4;
+                uint16_t* p = reinterpret_cast<uint16_t*>(y) + (size_t)t * ldy + n0 + r4;
 #pragma unroll
                 for (int i = 0; i < 4; i++) p[i] = f32_to_bf16(v[i]);
             } else {
-                float* p = reinterpret_cast<float*>(y) + (size_t)tok * ldy + n0 + r4;
+                float* p = reinterpret_cast<float*>(y) + (size_t)t * ldy + n0 + r4;
 #pragma unroll
                 for (int i = 0; i < 4; i++) p[i] = v[i];
             }
@@ -271,14 +274,14 @@ __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ 
         return;
     }
     // a tail part: its sums to tpart[tail] (device-coherent stores), completed before the count
-    constexpr int kPartFloats = 32 * 64;
+    constexpr int kPartFloats = TB * 32 * 64;
     float* mine = tpart + (size_t)tail * kPartFloats;
-    for (int o = tid; o < 32 * 16; o += NTH) {
-        const int tok = o >> 4, r4 = 4 * (o & 15);
-        const f32x4_v v = sum4(tok, r4);
+    for (int o = tid; o < TB * 32 * 16; o += NTH) {
+        const int otb = o >> 9, tok = (o >> 4) & 31, r4 = 4 * (o & 15);
+        const f32x4_v v = sum4(otb, tok, r4);
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            __hip_atomic_store(mine + tok * 64 + r4 + i, v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(mine + (otb * 32 + tok) * 64 + r4 + i, v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __shared__ uint32_t last;
@@ -288,10 +291,10 @@ __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ 
     __syncthreads();
     if (!last) return;
     const float* all = tpart + (size_t)ts * P * kPartFloats;  // parts p = 0..P-1 of this tail slab
-    emit([&](int tok, int r4) {  // the parts in order p = 0..P-1
+    emit([&](int otb, int tok, int r4) {  // the parts in order p = 0..P-1
         f32x4_v v = {0.f, 0.f, 0.f, 0.f};
         for (int pp = 0; pp < P; pp++) {
-            float* src = const_cast<float*>(all) + (size_t)pp * kPartFloats + tok * 64 + r4;
+            float* src = const_cast<float*>(all) + (size_t)pp * kPartFloats + (otb * 32 + tok) * 64 + r4;
 #pragma unroll
             for (int i = 0; i < 4; i++) v[i] += __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
@@ -630,25 +633,61 @@ static bool two_fits(const W4& w, const uint16_t* x, int ldx, int m) {
            ldx % 8 == 0;
 }
 
-// Where the one-pass kernels beat the skinny kernel's 32-row launches (measured in one process, bf16 out, us one-pass
-// / skinny). 17..32 rows: one round of slabs or more (N = 17408, K = 5120, m = 32: 20.7 / 28.9) and K without an even
-// skinny slicing (the skinny kernel's uneven slices; N = 3072, K = 9216, m = 32: 14.5 / 20.4); small matrices keep the
-// skinny launches: N = K = 4096, m = 32: 11.8 / 7.8; N = K = 2048: 9.4 / 5.0. 33..64 rows (m = 33 / 48 / 64): uneven
-// K (N = 5120, K = 17408: 27 / 28 / 29 against 75 / 88 / 118) and from ~25 M weights (N = K = 5120: 15.3 / 16.3 / 17.0
-// against 16.7 / 18.6 / 21.6; N = 6144, K = 4096: 14.8 / 15.6 / 16.3 against 14.5 / 16.0 / 18.3); smaller ones keep
-// the skinny launches (N = K = 4096: 14.3 / 14.9 / 16.0 against 12.0 / 13.4 / 15.7).
-bool wdec_w4_pick(const W4& w, const uint16_t* x, int ldx, int m) {
+// 33..64 rows: wdec_kernel (two token blocks, 64-row slabs, two blocks to a CU) where it was the choice before
+// wdec2_kernel: a round of slabs or more, K without an even skinny slicing, or more than 48 rows of a large matrix
+static bool small_slabs_fit(const W4& w, const uint16_t* x, int ldx, int m) {
     using namespace qe_wdec;
-    if (token_blocks(m) == 2) {
-        if (!two_fits(w, x, ldx, m)) return false;
-        const long weights = (long)w.n * w.k;
-        return qe_gemv::decode_groups(w.n, w.k) == 0 || weights > (24L << 20) || (m >= 48 && weights >= (23L << 20));
-    }
     if (!wdec_w4_fits(w, x, ldx, m)) return false;
     const int nslabs = w.n / 64, ncu = qe_num_cus();
     // slabs filling at most half the CUs only with K parts (N = 4096, K = 11008, m = 48: 64 slabs, no part count fits
     // 172 steps: 48.4 us against 35.2)
-    if (2 * nslabs <= ncu && tail_parts(nslabs, w.k / BK, NW / token_blocks(m), ncu) == 1) return false;
+    if (2 * nslabs <= ncu && tail_parts(nslabs, w.k / BK, NW / 2, ncu) == 1) return false;
+    return nslabs >= ncu || qe_gemv::decode_groups(w.n, w.k) == 0 || (m > 48 && (long)w.n * w.k >= (26L << 20));
+}
+
+// ... and still is. A 128-row slab of wdec2_kernel takes a CU alone, so it needs rounds of 128 ncu rows that are well
+// filled: with at most half of one (0 < r <= ncu slabs of 64 past the whole rounds) it splits K to fill the rest, which
+// short K does not pay back, and just past half it leaves half the CUs idle where 64-row slabs run their few extra ones
+// as tail parts. Tail parts cost wdec_kernel ~5 us, lost on short K. us, wdec_kernel / wdec2_kernel, m = 48:
+//   N      K = 256    512        1024       2048       3072       4096       5120       8192
+//   10240  5.4/8.2    6.5/8.3    8.6/12.5   12.8/15.1  17.0/16.1  21.4/18.3  25.7/20.8  38.2/25.6
+//   16384  5.6/8.3    6.7/8.4    8.8/13.9   13.2/16.0  17.4/18.6  21.9/21.2  26.1/24.1  38.8/32.3
+//   17408  6.6/8.4    11.3/8.5   13.9/10.9  16.7/16.3  19.3/21.0  23.8/25.8  27.8/31.0  40.8/44.6
+//   20480  6.7/8.4    12.4/8.6   15.4/11.0  18.8/16.3  21.1/21.1  25.6/26.4  29.8/31.1  42.9/46.1
+//   24576  6.8/8.5    13.5/8.7   15.2/11.1  19.3/16.5  23.3/21.9  27.5/27.4  31.9/32.3  46.8/46.6
+//   32768  6.9/8.7    8.5/8.8    11.5/12.0  18.6/17.5  25.2/23.3  31.7/29.0  38.4/32.9  58.4/49.9
+//   49152  9.0/14.2   11.3/14.6  16.3/21.6  26.6/30.6  36.5/38.3  46.8/47.8  56.9/53.4  88.3/79.8
+static bool small_slabs_pay(int n, int k) {
+    using namespace qe_wdec;
+    const int s = n / 64, ncu = qe_num_cus(), r = s % (2 * ncu);
+    if (k <= 256) return true;
+    if (tail_parts(s, k / BK, NW / 2, ncu) == 1)
+        return k <= 512 || (r > 0 && r <= ncu ? k <= (16 * s > 11 * ncu ? 3584 : 2560) : k <= 1280);
+    return r > ncu && ((r <= ncu + ncu / 16 && k >= 2560) || (s <= ncu + ncu / 4 && k >= 3072));
+}
+
+// Where the one-pass kernels beat the skinny kernel's 32-row launches (measured in one process, bf16 out, us one-pass
+// / skinny). 17..32 rows: one round of slabs or more (N = 17408, K = 5120, m = 32: 20.7 / 28.9) and K without an even
+// skinny slicing (the skinny kernel's uneven slices; N = 3072, K = 9216, m = 32: 14.5 / 20.4); small matrices keep the
+// skinny launches: N = K = 4096, m = 32: 11.8 / 7.8; N = K = 2048: 9.4 / 5.0. 33..64 rows (m = 33 / 48 / 64): the shapes
+// of small_slabs_fit, uneven K (N = 5120, K = 17408: 27 / 28 / 29 against 75 / 88 / 118) and from ~25 M weights (N = K =
+// 5120: 15.3 / 16.3 / 17.0 against 16.7 / 18.6 / 21.6; N = 6144, K = 4096: 14.8 / 15.6 / 16.3 against 14.5 / 16.0 /
+// 18.3); smaller ones keep the skinny launches (N = K = 4096: 14.3 / 14.9 / 16.0 against 12.0 / 13.4 / 15.7). Skinny
+// blocks of 32 rows that just fill the CUs keep them to ~42 M weights up to 48 rows (N = 8192, m = 33 / 48: K = 3584
+// 15.6 / 16.9 against 14.1 / 15.3, K = 5120 18.2 / 19.5 against 17.9 / 18.4, K = 8192 20.9 against 24.9).
+bool wdec_w4_pick(const W4& w, const uint16_t* x, int ldx, int m) {
+    using namespace qe_wdec;
+    if (token_blocks(m) == 2) {
+        if (small_slabs_fit(w, x, ldx, m)) return true;
+        if (!two_fits(w, x, ldx, m)) return false;
+        const int nb = w.n / 32, ncu = qe_num_cus();
+        const bool full = m <= 48 && 8 * nb > 7 * ncu && nb <= ncu;
+        return qe_gemv::decode_groups(w.n, w.k) == 0 || (long)w.n * w.k > ((full ? 40L : 24L) << 20);
+    }
+    if (!wdec_w4_fits(w, x, ldx, m)) return false;
+    const int nslabs = w.n / 64, ncu = qe_num_cus();
+    // (fewer slabs: as in small_slabs_fit)
+    if (2 * nslabs <= ncu && tail_parts(nslabs, w.k / BK, NW, ncu) == 1) return false;
     return nslabs >= ncu || qe_gemv::decode_groups(w.n, w.k) == 0;
 }
 
@@ -659,13 +698,13 @@ bool wdec_w4_pick(const W4& w, const uint16_t* x, int ldx, int m) {
 // capture: then P = 1). The last part's in-order sum reads the P parts from the device-coherent level, one part at
 // a time, so fewer parts finish sooner: on C0's matrix (16 tail slabs, 80 K steps) P = 5 measured m = 32 / 64
 // 20.7 / 31.7 us against 22.9 / 36.9 us at P = 10, 23.1 / 33.3 us at P = 2, and 26.7 / 40.0 us with no tail split.
-// (33..64 rows: two_parts, summed by a kernel of their own.)
+// (wdec2_kernel: two_parts, summed by a kernel of their own.)
 void wdec_w4(const W4& w, const uint16_t* x, int ldx, void* y, int ldy, int m, bool out_bf16, hipStream_t st) {
     using namespace qe_wdec;
     CHECK(wdec_w4_fits(w, x, ldx, m) || two_fits(w, x, ldx, m), "wdec_w4: n %d k %d m %d ldx %d", w.n, w.k, m, ldx);
     CHECK(ldy >= (w.glu ? w.n / 2 : w.n), "wdec_w4 ldy %d", ldy);
     const int out = w.glu ? 2 : out_bf16 ? 1 : 0;
-    if (token_blocks(m) == 2) {
+    if (m > 32 && !(small_slabs_fit(w, x, ldx, m) && small_slabs_pay(w.n, w.k))) {
         const int ncu = qe_num_cus(), G = w.k >> 7, nsl = (w.n + two::ROWS - 1) / two::ROWS, rem = nsl % ncu;
         int P = rem > 0 ? two_parts(rem, G, ncu) : 1;
         float* tpart = nullptr;
@@ -691,7 +730,7 @@ void wdec_w4(const W4& w, const uint16_t* x, int ldx, void* y, int ldy, int m, b
         }
         return;
     }
-    const int KP = NW, KT = w.k / BK, nslabs = w.n / 64, ncu = qe_num_cus();
+    const int TB = token_blocks(m), KP = NW / TB, KT = w.k / BK, nslabs = w.n / 64, ncu = qe_num_cus();
     int nmain = nslabs, P = 1, rem = 0;
     float* tpart = nullptr;
     uint32_t* tctr = nullptr;
@@ -709,9 +748,16 @@ void wdec_w4(const W4& w, const uint16_t* x, int ldx, void* y, int ldy, int m, b
         }
     }
     const dim3 grid((unsigned)(nmain + (P > 1 ? rem * P : 0))), block(NTH);
-    if (w.sdt == kScaleF16)
-        wdec_kernel<kScaleF16><<<grid, block, kLds, st>>>(w.q, w.s, w.k, x, ldx, m, y, ldy, out, nmain, P, tpart, tctr);
-    else
-        wdec_kernel<kScaleBF16><<<grid, block, kLds, st>>>(w.q, w.s, w.k, x, ldx, m, y, ldy, out, nmain, P, tpart, tctr);
+#define QE_WDEC(SDT_, TB_)                                                                                    \
+    wdec_kernel<SDT_, TB_><<<grid, block, kLds, st>>>(w.q, w.s, w.k, x, ldx, m, y, ldy, out, nmain, P, tpart, \
+                                                      tctr)
+    if (w.sdt == kScaleF16) {
+        if (TB == 2) QE_WDEC(kScaleF16, 2);
+        else QE_WDEC(kScaleF16, 1);
+    } else {
+        if (TB == 2) QE_WDEC(kScaleBF16, 2);
+        else QE_WDEC(kScaleBF16, 1);
+    }
+#undef QE_WDEC
     HIP_CHECK(hipGetLastError());
 }

@@ -151,3 +151,61 @@ def test_decode_33_to_64_rows(dev, n, k, m):
     if k % 256 == 0:
         y1 = ops.matmul_w4_onepass(w, x)
         assert err_ratio(out_f32(y1), matmul_f64(xh, exact_w4(q, s, n, k, 1))) <= 1e-4
+
+
+@pytest.mark.parametrize("n,k", [(16384, 256), (9216, 512), (16384, 1024), (17408, 2560), (20480, 3072), (49152, 512)])
+@pytest.mark.parametrize("m", [33, 48, 64])
+def test_decode_33_to_64_rows_small_slabs(dev, n, k, m):
+    """33..64 rows where the 64-row slabs are the faster ones (one round of them, tail parts just past it, short K) or
+    the skinny launches are still taken (9216 x 512): the exact product, GLU, and outputs at an odd offset and stride"""
+    w, q, s = setup_w4(n, k, 1, seed=n + m)
+    xh = synth.x_host(m, k, seed=k + m)
+    x = synth.to_dev(xh)
+    y = ops.matmul_w4(w, x)
+    assert err_ratio(out_f32(y), matmul_f64(xh, exact_w4(q, s, n, k, 1))) <= 1e-4
+    big = torch.full((m, n + 7), float("nan"), dtype=torch.float32, device=dev)
+    z = ops.matmul_w4(w, x, y=big[:, 1:1 + n])
+    assert torch.equal(z.contiguous().view(torch.int32), y.view(torch.int32))
+    assert torch.isnan(big[:, 0]).all() and torch.isnan(big[:, 1 + n:]).all()
+    wg, qg, sg = setup_w4(n, k, 1, seed=n + m + 1, glu=True)
+    a = ops.matmul_w4(wg, x)
+    assert_glu_close(out_f32(a), glu_act(matmul_f64(xh, exact_w4(qg, sg, n, k, 1))), 1e-4)
+
+
+@pytest.mark.parametrize("n,k", [(16384, 256), (16384, 1024)])
+def test_decode_64_rows_one_pass_of_small_slabs(dev, n, k):
+    """one round of 64-row slabs over a short K: the dispatch takes the one-pass kernel, which needs 0.4 to 0.7 of the
+    time of the skinny launches that batch_invariant takes (MI355X: 5.1 against 13.3 us, 8.2 against 12.3 us). Best of
+    5 replays of a graph of 20 calls each"""
+    w, _, _ = setup_w4(n, k, 1, seed=7)
+    x = synth.to_dev(synth.x_host(64, k, seed=8))
+    y = torch.empty(64, n, dtype=torch.bfloat16, device=dev)
+
+    def us():
+        st = torch.cuda.Stream()
+        st.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(st):
+            ops.matmul_w4(w, x, out_bf16=True, y=y)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            for _ in range(20):
+                ops.matmul_w4(w, x, out_bf16=True, y=y)
+        best = float("inf")
+        for _ in range(5):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            g.replay()
+            e1.record()
+            torch.cuda.synchronize()
+            best = min(best, e0.elapsed_time(e1) * 50)
+        return best
+
+    one = us()
+    old = ops.set_config(batch_invariant=1)
+    try:
+        skinny = us()
+    finally:
+        ops.set_config(**old)
+    print(f"{n} x {k}, m = 64: {one:.2f} us, skinny {skinny:.2f} us", flush=True)
+    assert one < 0.85 * skinny
