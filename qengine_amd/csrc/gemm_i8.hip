@@ -377,7 +377,10 @@ __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ 
                 dst[bb][4 * rq + 3] = scale_to_f32<SDT>((uint16_t)(sp.y >> 16));
             }
     };
-    // activation scales of the step: this lane's token of each MFMA tile, every group
+    // activation scales of the step: this lane's token of each MFMA tile, every group. Read at the top of the step,
+    // except by W8A8 with group scales, whose row split and weight scales already queue there (2048 x 8192, t = 17 / 300 /
+    // 2048: 90.5 / 95.5 / 104.3 us at the top, 87.4 / 91.8 / 100.8 right before the flush)
+    constexpr bool kLateSx = WF == kW8 && !PC;
     float sxv[WMT][NGS];
     auto load_sx = [&](int slot) {
         const float* sxb = reinterpret_cast<const float*>(lds + kSxOff + slot * kSx);
@@ -451,7 +454,7 @@ __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ 
         };
         float swf[WNT][16];
         read_frags(0, 0);
-        load_sx(cur);
+        if constexpr (!kLateSx) load_sx(cur);
         if constexpr (WF == kW8) split_rows(0);
         if constexpr (MORE && WF == kW4) read_words(lds + kRawOff + ((kt + 1) & 1) * kRaw);
         if constexpr (!PC) load_sw(swf, cur);
@@ -481,6 +484,7 @@ __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ 
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (ks % KPG == KPG - 1) {
+                if constexpr (kLateSx) load_sx(cur);
                 if constexpr (PC) flush(ks / KPG, swf_pc);
                 else flush(ks / KPG, swf);
             }
