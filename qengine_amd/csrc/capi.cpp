@@ -87,7 +87,7 @@ void qe_gemm_i8_reserve(int k, int t) { gemm_i8_reserve(k, t, 0); }
 void qe_gemm_reserve_s(size_t bytes, void* stream) { gemm_reserve(bytes, as_stream(stream)); }
 void qe_gemm_h_reserve_s(int k, int t, void* stream) { gemm_h_reserve(k, t, as_stream(stream)); }
 void qe_gemm_i8_reserve_s(int k, int t, void* stream) { gemm_i8_reserve(k, t, as_stream(stream)); }
-int qe_workspace_count(int kind) { return stream_ws_count(kind); }
+int qe_workspace_count(int kind) { return ws_count(kind); }
 
 // W4A8 (reference src/capi.cpp:104-113): ci (tile candidate) and ks (kernel variant) select among the reference's
 // CUDA kernels; this build has one kernel per activation group and ignores them

@@ -19,6 +19,7 @@
 #include "gemm_tune.hpp"
 
 #include <algorithm>
+#include <optional>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -525,7 +526,7 @@ double gemm_cost_us(bool w8, int cfg, int n, int k, int t, const GemmGeom& g) {
 }  // namespace
 
 void gemm_reserve(size_t bytes, hipStream_t st) {
-    stream_ws_reserve(kWsSplit, bytes, st);
+    ws_reserve(kWsSplit, bytes, st);
 }
 
 namespace {
@@ -592,10 +593,11 @@ void run_choice(int cfg, int ks, const uint4* q, const uint16_t* s, int n, int k
                 void* c, int ldc, int out, int sdt, hipStream_t st) {
     GemmGeom g;
     float* part = nullptr;
+    std::optional<WsHold> hold;  // until the sum of the partials is launched
     if (ks > 1) {
         // no such split, or no workspace for it during a graph capture: the best unsplit configuration
         if (!gemm_geom(cfg, n, k, t, ks, g)) ks = 1;
-        else if ((part = static_cast<float*>(stream_ws(kWsSplit, g.ws_bytes, st))) == nullptr) {
+        else if ((part = static_cast<float*>(hold.emplace(st).get(kWsSplit, g.ws_bytes))) == nullptr) {
             ks = 1;
             cfg = gemm_model_choice(FMT != kFmtW4, n, k, t, 1).cfg;
         }

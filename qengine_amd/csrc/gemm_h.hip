@@ -282,8 +282,8 @@ __global__ void __launch_bounds__(NTH) gemm_h_kernel(const uint4* __restrict__ q
 
 // the pre-pass buffer (xh [t][k] fp16, xs [t] fp32) of (device, stream): a capture that needs more than an eager call
 // or gemm_h_reserve on its stream sized aborts with a message
-void* h_ws(size_t bytes, hipStream_t st) {
-    void* p = stream_ws(kWsH, bytes, st);
+void* h_ws(size_t bytes, WsHold& hold) {
+    void* p = hold.get(kWsH, bytes);
     CHECK(p != nullptr,
           "gemm_w4h: the pre-pass buffer (%zu bytes) must be sized by an eager call or qe_gemm_h_reserve(_s) on this "
           "stream before capture",
@@ -296,7 +296,7 @@ size_t h_ws_bytes(int k, int t) { return ((size_t)t * k * 2 + 255) / 256 * 256 +
 }  // namespace
 
 void gemm_h_reserve(int k, int t, hipStream_t st) {
-    if (k > 0 && t > 0) stream_ws_reserve(kWsH, h_ws_bytes(k, t), st);
+    if (k > 0 && t > 0) ws_reserve(kWsH, h_ws_bytes(k, t), st);
 }
 
 // out: 0 fp32, 1 bf16, 2 GLU (bf16 activation [t][n / 2])
@@ -305,7 +305,8 @@ void gemm_w4h(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, 
     CHECK(t > 0, "gemm_w4h: t = %d", t);
     CHECK(ldx >= w.k, "gemm_w4h: ldx = %d < k", ldx);
     CHECK(ldc >= (w.glu ? w.n / 2 : w.n), "gemm_w4h: ldc = %d", ldc);
-    char* ws = static_cast<char*>(h_ws(h_ws_bytes(w.k, t), st));
+    WsHold hold(st);
+    char* ws = static_cast<char*>(h_ws(h_ws_bytes(w.k, t), hold));
     uint16_t* xh = reinterpret_cast<uint16_t*>(ws);
     float* xs = reinterpret_cast<float*>(ws + ((size_t)t * w.k * 2 + 255) / 256 * 256);
     if (((uintptr_t)x & 15) == 0 && ldx % 8 == 0) x_to_h_kernel<true><<<dim3((unsigned)t), dim3(256), 0, st>>>(x, ldx, w.k, xh, xs);

@@ -560,8 +560,8 @@ __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ 
 
 // the pre-pass buffer (xq [t][k] int8, sx [t][k / G] fp32) of (device, stream): a capture that needs more than an
 // eager call or gemm_i8_reserve on its stream sized aborts with a message
-void* i8_ws(size_t bytes, hipStream_t st) {
-    void* p = stream_ws(kWsI8, bytes, st);
+void* i8_ws(size_t bytes, WsHold& hold) {
+    void* p = hold.get(kWsI8, bytes);
     CHECK(p != nullptr,
           "gemm_w4_i8: the pre-pass buffer (%zu bytes) must be sized by an eager call or qe_gemm_i8_reserve(_s) on "
           "this stream before capture",
@@ -598,7 +598,8 @@ int i8_split(int ntiles, int kt, int G, double rows) {
 
 template <int G, int WF>
 void run_i8(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, int out, hipStream_t st) {
-    char* ws = static_cast<char*>(i8_ws(i8_ws_bytes(w.k, t), st));
+    WsHold hold(st);
+    char* ws = static_cast<char*>(i8_ws(i8_ws_bytes(w.k, t), hold));
     int8_t* xq = reinterpret_cast<int8_t*>(ws);
     float* sx = reinterpret_cast<float*>(ws + xq_bytes(w.k, t));
     const unsigned pb = (unsigned)(((long)t * (w.k / 16) + 255) / 256);
@@ -610,7 +611,7 @@ void run_i8(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, in
     sp.ks = i8_split(ntiles, w.k / BK, G, (double)t / nbt);
     const int nsplit = sp.ks > 1 ? ntiles % qe_num_cus() : 0;
     if (nsplit > 0) {
-        sp.part = static_cast<float*>(stream_ws(kWsSplit, (size_t)nsplit * sp.ks * BM * BN * 4, st));
+        sp.part = static_cast<float*>(hold.get(kWsSplit, (size_t)nsplit * sp.ks * BM * BN * 4));
         if (sp.part) sp.ndirect = ntiles - nsplit;  // (none during a capture that was not warmed up: unsplit)
     }
     const unsigned blocks = 8u * (unsigned)((min(sp.ndirect, ntiles) + 7) / 8) +
@@ -652,7 +653,8 @@ void gemm_w8a8(const W8& w, const uint16_t* x, int ldx, void* c, int ldc, int t,
     CHECK(t > 0, "gemm_w8a8: t = %d", t);
     CHECK(ldx >= w.k && ((uintptr_t)x & 1) == 0, "gemm_w8a8: ldx = %d < k", ldx);
     CHECK(ldc >= w.n, "gemm_w8a8: ldc = %d < n", ldc);
-    char* ws = static_cast<char*>(i8_ws(i8_ws_bytes(w.k, t), st));
+    WsHold hold(st);
+    char* ws = static_cast<char*>(i8_ws(i8_ws_bytes(w.k, t), hold));
     int8_t* xq = reinterpret_cast<int8_t*>(ws);
     float* sx = reinterpret_cast<float*>(ws + xq_bytes(w.k, t));
     const unsigned pb = (unsigned)(((long)t * (w.k / 32) + 255) / 256);
@@ -670,7 +672,7 @@ void gemm_w8a8(const W8& w, const uint16_t* x, int ldx, void* c, int ldc, int t,
 }
 
 void gemm_i8_reserve(int k, int t, hipStream_t st) {
-    if (k > 0 && t > 0) stream_ws_reserve(kWsI8, i8_ws_bytes(k, t), st);
+    if (k > 0 && t > 0) ws_reserve(kWsI8, i8_ws_bytes(k, t), st);
 }
 
 void gemm_w4_i8(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, int G, bool out_bf16,

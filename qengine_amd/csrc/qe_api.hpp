@@ -105,17 +105,31 @@ void gemv_w8(const W8& w, const uint16_t* x, int ldx, void* y, int ldy, int m, b
 
 // ---- library-owned workspaces, one per (kind, device, stream) (workspace.cpp) ----
 enum WsKind : int { kWsSplit = 0, kWsI8 = 1, kWsH = 2, kWsDec = 3, kWsSkinny = 4, kNumWs = 5 };
-// the buffer of (kind, current device, st), at least `bytes`: grown outside graph capture (the outgrown one kept
-// allocated); nullptr during capture when it is too small. kWsDec buffers (the one-pass decode's tail counters and
-// sums) are zero-filled when allocated; the kernel leaves its counters zero.
-void* stream_ws(int kind, size_t bytes, hipStream_t st);
-// the stream's tail workspace of the decode kernels (kWsDec, one size for every shape): dec_tail_ctr_bytes() of
-// counters (one per tail tile or slab, at most one per CU), then the tail parts' sums (up to 64 x 128 floats per
-// CU); nullptr during a graph capture on a stream that has none yet
-char* dec_tail_ws(hipStream_t st);
+struct StreamWs;
+// A call's hold on its stream's workspaces: made before the first buffer is asked for and kept until the last launch
+// that uses one, so that no other host thread's launches on the stream come in between.
+class WsHold {
+  public:
+    explicit WsHold(hipStream_t st);
+    ~WsHold();
+    WsHold(const WsHold&) = delete;
+    WsHold& operator=(const WsHold&) = delete;
+    // the buffer of (kind, current device, stream), at least `bytes`: grown outside graph capture (the outgrown one kept
+    // allocated); nullptr during capture when it is too small. kWsDec buffers (the one-pass decode's tail counters and
+    // sums) are zero-filled when allocated; the kernel leaves its counters zero.
+    void* get(int kind, size_t bytes);
+    // the tail workspace of the decode kernels (kWsDec, one size for every shape): dec_tail_ctr_bytes() of counters
+    // (one per tail tile or slab, at most one per CU), then the tail parts' sums (up to 64 x 128 floats per CU);
+    // nullptr during a graph capture on a stream that has none yet
+    char* dec_tail();
+
+  private:
+    hipStream_t st_;
+    StreamWs* s_;
+};
 size_t dec_tail_ctr_bytes();
-void stream_ws_reserve(int kind, size_t bytes, hipStream_t st);
-int stream_ws_count(int kind);  // buffers of that kind allocated so far (all devices and streams)
+void ws_reserve(int kind, size_t bytes, hipStream_t st);
+int ws_count(int kind);  // buffers of that kind allocated so far (all devices and streams)
 
 // ---- prefill GEMM (bf16 MFMA on dequantized tiles staged in LDS) ----
 // tuned: time the candidates on the first call of a (shape, token bucket) outside graph capture (also when the

@@ -28,6 +28,7 @@
 // timing (fixed K parts and sum order). Rows past m re-read row m - 1 and are not stored.
 #include "mfma_tile.hpp"
 
+#include <optional>
 #include <type_traits>
 
 namespace qe_wdec {
@@ -708,8 +709,9 @@ void wdec_w4(const W4& w, const uint16_t* x, int ldx, void* y, int ldy, int m, b
         const int ncu = qe_num_cus(), G = w.k >> 7, nsl = (w.n + two::ROWS - 1) / two::ROWS, rem = nsl % ncu;
         int P = rem > 0 ? two_parts(rem, G, ncu) : 1;
         float* tpart = nullptr;
+        std::optional<WsHold> hold;  // until the sum of the parts is launched
         if (P > 1) {
-            char* ws = dec_tail_ws(st);
+            char* ws = hold.emplace(st).dec_tail();
             if (ws) tpart = reinterpret_cast<float*>(ws + dec_tail_ctr_bytes());
             else P = 1;
         }
@@ -735,10 +737,11 @@ void wdec_w4(const W4& w, const uint16_t* x, int ldx, void* y, int ldy, int m, b
     float* tpart = nullptr;
     uint32_t* tctr = nullptr;
     const int p = qe_wdec::tail_parts(nslabs, KT, KP, ncu);
+    std::optional<WsHold> hold;
     if (p > 1) {
         // one size for every shape (at most ncu tail blocks of two token blocks), so a stream's first call sizes it
         // for all later ones, graph captures included
-        char* ws = dec_tail_ws(st);
+        char* ws = hold.emplace(st).dec_tail();
         if (ws) {
             rem = 2 * nslabs <= ncu ? nslabs : nslabs % ncu;
             P = p;

@@ -5,13 +5,18 @@
 // The reference keeps these buffers thread_local (src/kernels/gemm.cu:3258-3368), so two host threads never share
 // one. Here the key is the stream a call is enqueued on: calls on one stream run in order, so they can share a
 // buffer, while calls on two streams of one device (or two graphs replayed on two streams) get two buffers and cannot
-// overwrite each other's data. A buffer grows on a call outside graph capture; the outgrown one is kept allocated
+// overwrite each other's data. A call's launches that write and read a buffer have to follow each other on the stream
+// without another call's in between, and host threads may call on one stream (torch's threads share the default one),
+// so a call holds the stream's lock (WsHold) from its first buffer to its last launch.
+// A buffer grows on a call outside graph capture; the outgrown one is kept allocated
 // (retired, never freed: a graph captured earlier may still read it). During capture a buffer that is too small is
-// not grown: stream_ws returns nullptr and the caller either runs without it (the GEMM's split, the decode kernels; they
-// do so too when the device has no memory left for it) or aborts with a message (the pre-passes), so callers size it first with an eager call or stream_ws_reserve on that stream.
+// not grown: get returns nullptr and the caller either runs without it (the GEMM's split, the decode kernels; they
+// do so too when the device has no memory left for it) or aborts with a message (the pre-passes), so callers size it
+// first with an eager call or ws_reserve on that stream.
 #include <map>
+#include <memory>
 #include <mutex>
-#include <tuple>
+#include <utility>
 #include <vector>
 
 #include "qe_api.hpp"
@@ -21,20 +26,38 @@ struct Ws {
     void* p = nullptr;
     size_t bytes = 0;
 };
-std::mutex g_mu;
-std::map<std::tuple<int, int, hipStream_t>, Ws> g_ws;  // (kind, device, stream) -> buffer
-std::vector<void*> g_retired;
 }  // namespace
 
-void* stream_ws(int kind, size_t bytes, hipStream_t st) {
-    CHECK(kind >= 0 && kind < kNumWs, "workspace kind %d", kind);
+struct StreamWs {
+    std::mutex mu;  // held by WsHold; guards ws
+    Ws ws[kNumWs];
+};
+
+namespace {
+std::mutex g_mu;  // guards the containers below; never held while a stream's lock is waited for
+std::map<std::pair<int, hipStream_t>, std::unique_ptr<StreamWs>> g_streams;  // (device, stream), never erased
+std::vector<void*> g_retired;
+int g_count[kNumWs];
+
+StreamWs* stream_of(hipStream_t st) {
     int dev = 0;
     HIP_CHECK(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(g_mu);
-    Ws& w = g_ws[std::make_tuple(kind, dev, st)];
+    std::unique_ptr<StreamWs>& s = g_streams[std::make_pair(dev, st)];
+    if (!s) s.reset(new StreamWs);
+    return s.get();
+}
+}  // namespace
+
+WsHold::WsHold(hipStream_t st) : st_(st), s_(stream_of(st)) { s_->mu.lock(); }
+WsHold::~WsHold() { s_->mu.unlock(); }
+
+void* WsHold::get(int kind, size_t bytes) {
+    CHECK(kind >= 0 && kind < kNumWs, "workspace kind %d", kind);
+    Ws& w = s_->ws[kind];
     if (w.bytes >= bytes) return w.p;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    HIP_CHECK(hipStreamIsCapturing(st, &cs));
+    HIP_CHECK(hipStreamIsCapturing(st_, &cs));
     if (cs != hipStreamCaptureStatusNone) return nullptr;
     void* np = nullptr;
     const hipError_t e = hipMalloc(&np, bytes);
@@ -44,10 +67,14 @@ void* stream_ws(int kind, size_t bytes, hipStream_t st) {
     }
     HIP_CHECK(e);
     if (kind == kWsDec) {  // counters start at zero (the kernel sets them back to zero at the end of every call)
-        HIP_CHECK(hipMemsetAsync(np, 0, bytes, st));
-        HIP_CHECK(hipStreamSynchronize(st));
+        HIP_CHECK(hipMemsetAsync(np, 0, bytes, st_));
+        HIP_CHECK(hipStreamSynchronize(st_));
     }
-    if (w.p) g_retired.push_back(w.p);
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        if (w.p) g_retired.push_back(w.p);
+        else g_count[kind]++;
+    }
     w.p = np;
     w.bytes = bytes;
     return np;
@@ -55,18 +82,15 @@ void* stream_ws(int kind, size_t bytes, hipStream_t st) {
 
 size_t dec_tail_ctr_bytes() { return ((size_t)qe_num_cus() * 4 + 255) / 256 * 256; }
 
-char* dec_tail_ws(hipStream_t st) {
-    return static_cast<char*>(stream_ws(kWsDec, dec_tail_ctr_bytes() + (size_t)qe_num_cus() * 64 * 128 * 4, st));
+char* WsHold::dec_tail() {
+    return static_cast<char*>(get(kWsDec, dec_tail_ctr_bytes() + (size_t)qe_num_cus() * 64 * 128 * 4));
 }
 
-void stream_ws_reserve(int kind, size_t bytes, hipStream_t st) {
-    if (bytes > 0) CHECK(stream_ws(kind, bytes, st) != nullptr, "workspace reserve: called during graph capture");
+void ws_reserve(int kind, size_t bytes, hipStream_t st) {
+    if (bytes > 0) CHECK(WsHold(st).get(kind, bytes) != nullptr, "workspace reserve: called during graph capture");
 }
 
-int stream_ws_count(int kind) {
+int ws_count(int kind) {
     std::lock_guard<std::mutex> lk(g_mu);
-    int c = 0;
-    for (const auto& e : g_ws)
-        if (std::get<0>(e.first) == kind && e.second.p) c++;
-    return c;
+    return kind >= 0 && kind < kNumWs ? g_count[kind] : 0;
 }

@@ -1,6 +1,9 @@
 """Library-owned GEMM workspaces are per (device, stream): two streams in flight at once on one GPU each get their own
 split-K partials and pre-pass buffers, so every result equals the same call made serially (the reference keeps these
-buffers thread_local, src/kernels/gemm.cu:3258-3368)."""
+buffers thread_local, src/kernels/gemm.cu:3258-3368). So do two host threads that call on one stream."""
+import sys
+import threading
+
 import pytest
 import torch
 
@@ -43,3 +46,68 @@ def test_two_streams_keep_their_own_workspace(dev, path):
         for r, y in enumerate(got[i]):
             assert torch.equal(y.view(iv), want[i].view(iv)), (path, i, r)
     assert call("qe_workspace_count", KIND[path]) >= 3  # the default stream's and one per stream
+
+
+# one case per buffer: the 9..16-row slice sums, the 33..64-row and 17..32-row tail parts, the split-K partials, the
+# W4A8 and fp16 pre-pass buffers
+PATHS = {"decode_12": (5120, 13824, 12), "decode_48": (5120, 3712, 48), "decode_24": (17408, 2560, 24),
+         "prefill": (1040, 2176, 100), "i8": (1040, 2176, 100), "h16": (1040, 2176, 100)}
+_MADE = {}
+
+
+def _case(path):
+    if path not in _MADE:
+        n, k, m = PATHS[path]
+        w, _, _ = setup(n, k, 1, seed=n + m)
+        f = {"i8": lambda x, y=None: ops.gemm_w4_i8(w, x, G=64, y=y), "h16": lambda x, y=None: ops.gemm_w4h(w, x, y=y)}
+        _MADE[path] = f.get(path, lambda x, y=None: ops.matmul_w4(w, x, y=y)), \
+            [synth.to_dev(synth.x_host(m, k, seed=s)) for s in (1, 2)]
+    return _MADE[path]
+
+
+@pytest.mark.parametrize("path", list(PATHS))
+def test_two_threads_on_one_stream(dev, path):
+    """a call's launches stay together on the stream: no other thread's launch writes its buffer in between"""
+    run, xs = _case(path)
+    want = [run(x) for x in xs]
+    torch.cuda.synchronize()
+    got = [[torch.empty_like(want[i]) for _ in range(60)] for i in range(2)]
+    gate = threading.Barrier(2)
+
+    def calls(i):
+        gate.wait()
+        for y in got[i]:
+            run(xs[i], y)
+
+    threads = [threading.Thread(target=calls, args=(i,)) for i in range(2)]
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)
+    try:
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(interval)
+    torch.cuda.synchronize()
+    for i in range(2):
+        for r, y in enumerate(got[i]):
+            assert torch.equal(y, want[i]), (path, i, r)
+
+
+@pytest.mark.parametrize("path", list(PATHS))
+def test_two_streams_in_flight(dev, path):
+    """calls of two streams interleaved, nothing waits in between: each the bits of the serial call"""
+    run, xs = _case(path)
+    want = [run(x) for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    got = [[torch.empty_like(want[i]) for _ in range(20)] for i in range(2)]
+    for r in range(20):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                run(xs[i], got[i][r])
+    torch.cuda.synchronize()
+    for i in range(2):
+        for r, y in enumerate(got[i]):
+            assert torch.equal(y, want[i]), (path, i, r)
