@@ -62,17 +62,22 @@ void qe_set_config(const qe_config_t* cfg);
 void qe_gemm_tune_file(const char* path);
 void qe_gemm_tune_clear(void);
 int qe_gemm_tune_entries(void);
-/* Library-owned workspaces of the prefill GEMMs (the split-K partial sums, the fp16-accumulate and W4A8 / W8A8
- * pre-pass buffers) are kept per (device, stream): calls on one stream share a buffer (they run in order), calls on
- * two streams of a device use two, so concurrent streams (or graphs replayed on two streams) never overwrite each
- * other's workspace (the reference keeps them thread_local, src/kernels/gemm.cu:3258-3368). A buffer grows on a call
- * outside graph capture; during capture it is not grown (the GEMM then runs unsplit; a pre-pass aborts with a message).
- * qe_gemm_reserve sizes the split-K workspace of the current device's default stream before capturing (the
- * reference's gemm_reserve_ws); qe_gemm_reserve_s that of `stream`. */
+/* Library-owned workspaces (the prefill GEMMs' split-K partial sums, the fp16-accumulate and W4A8 / W8A8 pre-pass
+ * buffers, the part sums of 9..64-row decode) are kept per (device, stream): calls on one stream share a buffer (a
+ * call's launches stay together, also with several host threads on the stream), calls on two streams of a device use
+ * two, so concurrent streams never overwrite each other's workspace (the reference keeps them thread_local,
+ * src/kernels/gemm.cu:3258-3368). A buffer grows on a call outside graph capture. Captured calls use buffers that their
+ * graph holds (a HIP user object), so graphs may replay on any streams, beside each other and eager calls; destroying
+ * the graph and its executables gives them back for later captures. (An executable that was updated from another graph
+ * by hipGraphExecUpdate uses that graph's buffers: keep it.) A capture of a prefill GEMM wants its stream sized before,
+ * by an eager call there or a reserve: the GEMM then runs unsplit else; a pre-pass aborts with a message. Decode needs
+ * no preparation. qe_gemm_reserve sizes the split-K workspace of the current device's default stream before capturing
+ * (the reference's gemm_reserve_ws); qe_gemm_reserve_s that of `stream`. */
 void qe_gemm_reserve(size_t bytes);
 void qe_gemm_reserve_s(size_t bytes, void* stream);
-/* test hook: how many workspace buffers of a kind (0 split-K, 1 W4A8 / W8A8 pre-pass, 2 fp16-accumulate pre-pass)
- * the library holds, over all devices and streams. No counterpart in the reference. */
+/* test hook: how many workspace buffers of a kind (0 split-K, 1 W4A8 / W8A8 pre-pass, 2 fp16-accumulate pre-pass, 3 part
+ * sums of 17..64-row decode, 4 slice sums of 9..16-row decode) the library's streams and live graphs hold, over all
+ * devices. No counterpart in the reference. */
 int qe_workspace_count(int kind);
 /* Prefill GEMM with the reference's fp16-accumulate numerics (gemm_h_kernel + x_to_h_kernel,
  * src/kernels/gemm.cu:236-461): activations scaled per token to |x| <= 16 (xs = amax / 16) and rounded to fp16,

@@ -595,7 +595,8 @@ void run_choice(int cfg, int ks, const uint4* q, const uint16_t* s, int n, int k
     float* part = nullptr;
     std::optional<WsHold> hold;  // until the sum of the partials is launched
     if (ks > 1) {
-        // no such split, or no workspace for it during a graph capture: the best unsplit configuration
+        // no such split, or no workspace for it (memory; a graph capture on a stream that was not sized before): the
+        // best unsplit configuration
         if (!gemm_geom(cfg, n, k, t, ks, g)) ks = 1;
         else if ((part = static_cast<float*>(hold.emplace(st).get(kWsSplit, g.ws_bytes))) == nullptr) {
             ks = 1;

@@ -612,7 +612,7 @@ void run_i8(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, in
     const int nsplit = sp.ks > 1 ? ntiles % qe_num_cus() : 0;
     if (nsplit > 0) {
         sp.part = static_cast<float*>(hold.get(kWsSplit, (size_t)nsplit * sp.ks * BM * BN * 4));
-        if (sp.part) sp.ndirect = ntiles - nsplit;  // (none during a capture that was not warmed up: unsplit)
+        if (sp.part) sp.ndirect = ntiles - nsplit;  // (none: no memory, or a capture on a stream not sized: unsplit)
     }
     const unsigned blocks = 8u * (unsigned)((min(sp.ndirect, ntiles) + 7) / 8) +
                             (sp.part ? split_blocks(nsplit, sp.ks) : 0u);

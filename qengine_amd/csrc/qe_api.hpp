@@ -114,14 +114,15 @@ class WsHold {
     ~WsHold();
     WsHold(const WsHold&) = delete;
     WsHold& operator=(const WsHold&) = delete;
-    // the buffer of (kind, current device, stream), at least `bytes`: grown outside graph capture (the outgrown one kept
-    // allocated); nullptr during capture when it is too small. kWsDec buffers (the one-pass decode's tail counters and
-    // sums) are zero-filled when allocated; the kernel leaves its counters zero.
+    // the buffer of (kind, current device, stream), at least `bytes`, grown on a call outside graph capture. During
+    // capture: a buffer that the graph holds; nullptr for kWsSplit, kWsI8 and kWsH where the stream's own has not that
+    // size. nullptr too where the device has no memory for a kWsSplit, kWsDec or kWsSkinny buffer. kWsDec buffers
+    // (the one-pass decode's tail counters and sums) are zero-filled when allocated; the kernel leaves its counters zero.
     void* get(int kind, size_t bytes);
     // the tail workspace of the decode kernels (kWsDec, one size for every shape): dec_tail_ctr_bytes() of counters
-    // (one per tail tile or slab, at most one per CU), then the tail parts' sums (up to 64 x 128 floats per CU);
-    // nullptr during a graph capture on a stream that has none yet
+    // (one per tail tile or slab, at most one per CU), then the tail parts' sums (up to 64 x 128 floats per CU)
     char* dec_tail();
+    size_t sized(int kind) const;  // bytes of the stream's own buffer
 
   private:
     hipStream_t st_;
@@ -129,7 +130,7 @@ class WsHold {
 };
 size_t dec_tail_ctr_bytes();
 void ws_reserve(int kind, size_t bytes, hipStream_t st);
-int ws_count(int kind);  // buffers of that kind allocated so far (all devices and streams)
+int ws_count(int kind);  // buffers of that kind that streams (all devices) and graphs hold
 
 // ---- prefill GEMM (bf16 MFMA on dequantized tiles staged in LDS) ----
 // tuned: time the candidates on the first call of a (shape, token bucket) outside graph capture (also when the
@@ -154,7 +155,7 @@ void gemm_i8_reserve(int k, int t, hipStream_t st);
 // the reference's W8A8 row GEMM of a W8 matrix (k_x_to_r8 + k_rows_qt), on the same pre-pass buffer
 void gemm_w8a8(const W8& w, const uint16_t* x, int ldx, void* c, int ldc, int t, bool out_bf16, hipStream_t st);
 void gemm_set_out_bf16(bool on);
-// reserve the split-K workspace of (the current device, st) (grown on demand otherwise, never during graph capture)
+// reserve the split-K workspace of (the current device, st) (grown on demand otherwise; a capture wants it sized before)
 void gemm_reserve(size_t bytes, hipStream_t st);
 bool gemm_out_bf16();
 // run-time cap of the split count of the prefill GEMMs' last partial round (0 or less: no cap, i.e. up to 4)

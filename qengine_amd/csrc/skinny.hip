@@ -512,7 +512,7 @@ void launch(const uint4* q, const uint16_t* s, int n, int k, const uint16_t* x, 
     const dim3 block(64 * sc.S);
     if constexpr (FMT == kFmtW4 && !H16 && !UA) {
         if (mt == 16 && sc.ng == 0 && part_pays(n, k, sc.S)) {
-            // no workspace (a capture that was not warmed up): one block per tile below, the same bits
+            // no workspace (out of memory): one block per tile below, the same bits
             WsHold hold(st);
             if (float* part = static_cast<float*>(hold.get(kWsSkinny, (size_t)(n / 16) * sc.S * 256 * 4))) {
                 const dim3 pb(64 * kPartWaves);

@@ -695,8 +695,7 @@ bool wdec_w4_pick(const W4& w, const uint16_t* x, int ldx, int m) {
 // Slabs past the last whole round of CUs (N / 64 = 272 on 256 CUs: 16) would give 16 CUs two slabs; they run as P
 // K parts each instead (tail blocks, sharing CUs with the whole slabs), so no CU gets two slabs' work: P the first
 // of 5, 4, 8, 10, 2 with the tail blocks at most one round and an even number of steps per wave, if the stream's
-// zero-initialised workspace (kWsDec: counters, then the parts' sums) is at hand (not allocated during graph
-// capture: then P = 1). The last part's in-order sum reads the P parts from the device-coherent level, one part at
+// zero-initialised workspace (kWsDec: counters, then the parts' sums) is at hand (without memory for it P = 1). The last part's in-order sum reads the P parts from the device-coherent level, one part at
 // a time, so fewer parts finish sooner: on C0's matrix (16 tail slabs, 80 K steps) P = 5 measured m = 32 / 64
 // 20.7 / 31.7 us against 22.9 / 36.9 us at P = 10, 23.1 / 33.3 us at P = 2, and 26.7 / 40.0 us with no tail split.
 // (wdec2_kernel: two_parts, summed by a kernel of their own.)

@@ -575,7 +575,7 @@ def test_skinny_slices_in_parts(dev, n, k, glu, m):
     339) or of two (258, 320, 768) run in blocks of four waves, the last block short at K = 28672 (14 slices), and a
     second launch adds them in slice order. Within 1e-4 * rms
     of the exact product; a row's bits are those of the row in calls of 2 rows (one block per tile, the same slices), of
-    repeated calls, and of a graph captured on a stream without the workspace (one block per tile) or with it"""
+    repeated calls, and of a graph captured on a stream that never ran the call or one that did"""
     w, q, s = setup_w4(n, k, 1, seed=n + m, glu=glu)
     xh = synth.x_host(m, k, seed=k + m)
     x = synth.to_dev(xh)

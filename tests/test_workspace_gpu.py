@@ -111,3 +111,65 @@ def test_two_streams_in_flight(dev, path):
     for i in range(2):
         for r, y in enumerate(got[i]):
             assert torch.equal(y, want[i]), (path, i, r)
+
+
+def _graph(run, x, y, stream):
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream):
+        run(x, y)
+    return g
+
+
+@pytest.mark.parametrize("path", list(PATHS))
+def test_two_graphs_of_one_stream_replayed_at_once(dev, path):
+    """a graph's calls use buffers of the graph's own: two captured on one stream and replayed on two, beside eager calls
+    on the stream of the capture, nothing waiting in between, all give the eager bits"""
+    run, xs = _case(path)
+    want = [run(x) for x in xs]
+    cap = torch.cuda.Stream()
+    cap.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(cap):
+        run(xs[0])  # (the split and the pre-passes need their stream sized before a capture)
+    outs = [torch.empty_like(want[i]) for i in range(2)]
+    graphs = [_graph(run, xs[i], outs[i], cap) for i in range(2)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    got, eager = [[], []], []
+    for _ in range(20):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                graphs[i].replay()
+                got[i].append(outs[i].clone())
+        with torch.cuda.stream(cap):
+            eager.append(run(xs[1]))
+    torch.cuda.synchronize()
+    for r in range(20):
+        assert torch.equal(eager[r], want[1]), (path, r)
+        for i in range(2):
+            assert torch.equal(got[i][r], want[i]), (path, i, r)
+
+
+@pytest.mark.parametrize("path,kind", [("decode_12", 4), ("decode_48", 3), ("decode_24", 3)])
+def test_decode_captured_without_preparation(dev, path, kind):
+    """decode under capture on a stream that never ran it: the kernels of the eager call, hence its bits; the graph's
+    buffer goes back with the graph and serves the next one"""
+    run, xs = _case(path)
+    want = run(xs[0])
+    y = torch.empty_like(want)
+    torch.cuda.synchronize()
+    counts = []
+    for _ in range(3):
+        before = call("qe_workspace_count", kind)
+        g = _graph(run, xs[0], y, torch.cuda.Stream())
+        counts.append(call("qe_workspace_count", kind) - before)
+        for _ in range(3):
+            y.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want), path
+        g.reset()
+        del g
+        torch.cuda.synchronize()
+        counts.append(call("qe_workspace_count", kind) - before)
+    assert counts == [1, 0] * 3, counts

@@ -5,7 +5,7 @@
 #include <chrono>
 #include <cstring>
 #include <map>
-#include <set>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -21,7 +21,32 @@
     } while (0)
 
 namespace {
-std::set<void*> g_live;  // allocations not freed
+struct Graph {
+    int refs = 1;  // the graph and its executables
+    std::vector<std::pair<hipHostFn_t, void*>> held;
+};
+struct Capture {
+    unsigned long long id;
+    Graph* graph;
+};
+std::mutex g_model;
+std::map<hipStream_t, Capture> g_captures;  // streams being captured
+unsigned long long g_next_id = 0;
+size_t g_allocs = 0;
+bool g_oom = false;
+thread_local hipStreamCaptureMode t_mode = hipStreamCaptureModeGlobal;
+
+Graph* begin_capture(hipStream_t st) {
+    Graph* g = new Graph;
+    g_captures[st] = Capture{++g_next_id, g};
+    return g;
+}
+void end_capture(hipStream_t st) { g_captures.erase(st); }
+void unref(Graph* g) {  // the graph or an executable of it is destroyed
+    if (--g->refs) return;
+    for (auto& h : g->held) h.first(h.second);
+    delete g;
+}
 }  // namespace
 
 // ---- the HIP calls ----
@@ -32,15 +57,45 @@ hipError_t hipGetDevice(int* d) {
 }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "model"; }
-hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) {
-    *s = hipStreamCaptureStatusNone;
+hipError_t hipStreamGetCaptureInfo_v2(hipStream_t st, hipStreamCaptureStatus* s, unsigned long long* id, hipGraph_t* g,
+                                      const hipGraphNode_t**, size_t*) {
+    std::lock_guard<std::mutex> lk(g_model);
+    auto it = g_captures.find(st);
+    *s = it == g_captures.end() ? hipStreamCaptureStatusNone : hipStreamCaptureStatusActive;
+    if (it != g_captures.end()) {
+        *id = it->second.id;
+        *g = reinterpret_cast<hipGraph_t>(it->second.graph);
+    }
     return hipSuccess;
 }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {
+    std::swap(*m, t_mode);
+    return hipSuccess;
+}
+hipError_t hipUserObjectCreate(hipUserObject_t* o, void* p, hipHostFn_t f, unsigned, unsigned) {
+    *o = reinterpret_cast<hipUserObject_t>(new std::pair<hipHostFn_t, void*>(f, p));
+    return hipSuccess;
+}
+hipError_t hipGraphRetainUserObject(hipGraph_t g, hipUserObject_t o, unsigned, unsigned) {
+    auto* h = reinterpret_cast<std::pair<hipHostFn_t, void*>*>(o);
+    reinterpret_cast<Graph*>(g)->held.push_back(*h);
+    delete h;
+    return hipSuccess;
+}
+// memory calls fail in a thread of the global mode while any stream is being captured, as HIP's do
 hipError_t hipMalloc(void** p, size_t n) {
+    std::lock_guard<std::mutex> lk(g_model);
+    if (t_mode == hipStreamCaptureModeGlobal && !g_captures.empty()) return hipErrorStreamCaptureUnsupported;
+    if (g_oom) return hipErrorOutOfMemory;
+    g_allocs++;
     *p = malloc(n);
-    g_live.insert(*p);
     return hipSuccess;
 }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+    *s = reinterpret_cast<hipStream_t>(8);
+    return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) {
     memset(p, v, n);
     return hipSuccess;
@@ -92,9 +147,79 @@ static void another_stream_runs() {
     EXPECT(ws_count(kWsSplit) == 2);
 }
 
+// every kind under capture: not the stream's buffer, the same one again in that capture, another for another capture and
+// another stream; the kinds that need sizing get none before
+static void captures_have_their_own() {
+    for (int kind = 0; kind < kNumWs; kind++) {
+        hipStream_t st = stream(10 + kind), other = stream(100 + kind);
+        const bool sizing = kind == kWsSplit || kind == kWsI8 || kind == kWsH;
+        Graph* g0 = begin_capture(st);
+        EXPECT((WsHold(st).get(kind, 1 << 20) == nullptr) == sizing);
+        end_capture(st);
+        unref(g0);
+        void* own = WsHold(st).get(kind, 1 << 20);
+        EXPECT(own && WsHold(other).get(kind, 1 << 20));
+        Graph* g1 = begin_capture(st);
+        void* a = WsHold(st).get(kind, 1 << 20);
+        EXPECT(a && a != own && WsHold(st).get(kind, 1000) == a);
+        EXPECT((WsHold(st).get(kind, 64 << 20) == nullptr) == sizing);
+        end_capture(st);
+        EXPECT(WsHold(st).get(kind, 1 << 20) == own);
+        Graph* g2 = begin_capture(st);
+        Graph* g3 = begin_capture(other);
+        void *b = WsHold(st).get(kind, 1 << 20), *c = WsHold(other).get(kind, 1 << 20);
+        EXPECT(b && c && b != c && b != a && c != a && b != own);
+        end_capture(st);
+        end_capture(other);
+        unref(g1), unref(g2), unref(g3);
+    }
+}
+
+// a graph's buffer serves no other capture while the graph or an executable of it lives, and the next one after that
+static void graphs_give_back() {
+    hipStream_t st = stream(1);
+    const int before = ws_count(kWsDec);
+    Graph* g1 = begin_capture(st);
+    void* a = WsHold(st).get(kWsDec, 1 << 20);
+    end_capture(st);
+    g1->refs++;  // instantiated
+    unref(g1);   // the graph is destroyed, the executable lives
+    Graph* g2 = begin_capture(st);
+    void* b = WsHold(st).get(kWsDec, 1 << 20);
+    end_capture(st);
+    EXPECT(a != b && ws_count(kWsDec) == before + 2);
+    unref(g1);
+    EXPECT(ws_count(kWsDec) == before + 1);
+    const size_t allocs = g_allocs;
+    for (int i = 0; i < 5; i++) {
+        Graph* g = begin_capture(st);
+        EXPECT(WsHold(st).get(kWsDec, 1 << 20) == a);
+        end_capture(st);
+        unref(g);
+    }
+    EXPECT(g_allocs == allocs);
+    unref(g2);
+    EXPECT(ws_count(kWsDec) == before);
+}
+
+// no memory under capture: no buffer, and the capture goes on
+static void capture_without_memory() {
+    hipStream_t st = stream(1);
+    Graph* g = begin_capture(st);
+    g_oom = true;
+    EXPECT(WsHold(st).get(kWsSkinny, 1 << 20) == nullptr);
+    g_oom = false;
+    EXPECT(WsHold(st).get(kWsSkinny, 1 << 20) != nullptr);
+    end_capture(st);
+    unref(g);
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> all = {{"threads_on_one_stream", threads_on_one_stream},
-                                                   {"another_stream_runs", another_stream_runs}};
+                                                   {"another_stream_runs", another_stream_runs},
+                                                   {"captures_have_their_own", captures_have_their_own},
+                                                   {"graphs_give_back", graphs_give_back},
+                                                   {"capture_without_memory", capture_without_memory}};
     EXPECT(argc == 2 && all.count(argv[1]));
     all.at(argv[1])();
     printf("OK\n");
