@@ -98,8 +98,8 @@ void give_back(void* arg) {
     state().pool.emplace(std::make_pair(b->dev, b->kind), b);
 }
 
-// device memory inside a capture, which its default (global) mode forbids: the allocation is not part of the graph, so
-// this thread leaves that mode for it
+// device memory inside a capture or beside one of another thread, which the default (global) mode forbids: the allocation
+// is not part of any graph, so this thread leaves that mode for it
 struct RelaxedCapture {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     RelaxedCapture() { HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode)); }
@@ -169,6 +169,7 @@ void* WsHold::get(int kind, size_t bytes) {
     hipGraph_t graph = nullptr;
     if (capturing(st_, &id, &graph)) return needs_sizing(kind) && w.bytes < bytes ? nullptr : capture_buf(s_, kind, bytes, id, graph);
     if (w.bytes >= bytes) return w.p;
+    RelaxedCapture relaxed;
     void* np = nullptr;
     const hipError_t e = hipMalloc(&np, bytes);
     if (e == hipErrorOutOfMemory && kind != kWsI8 && kind != kWsH) {  // every other caller runs without its buffer

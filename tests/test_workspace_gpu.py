@@ -1,6 +1,7 @@
 """Library-owned GEMM workspaces are per (device, stream): two streams in flight at once on one GPU each get their own
 split-K partials and pre-pass buffers, so every result equals the same call made serially (the reference keeps these
 buffers thread_local, src/kernels/gemm.cu:3258-3368). So do two host threads that call on one stream."""
+import ctypes
 import sys
 import threading
 
@@ -173,3 +174,43 @@ def test_decode_captured_without_preparation(dev, path, kind):
         torch.cuda.synchronize()
         counts.append(call("qe_workspace_count", kind) - before)
     assert counts == [1, 0] * 3, counts
+
+
+@pytest.mark.parametrize("path", list(PATHS))
+def test_first_call_beside_a_capture(dev, path):
+    """a stream's first call, which allocates its buffer, while another thread captures in the default (global) mode: both
+    give the eager bits"""
+    run, xs = _case(path)
+    want = [run(x) for x in xs]
+    y, z = torch.empty_like(want[0]), torch.empty_like(want[1])
+    hip = ctypes.CDLL("libamdhip64.so")
+    raw = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(raw), 1) == 0  # non-blocking, no call made on it yet
+    fresh = torch.cuda.ExternalStream(raw.value)
+    failed = []
+
+    def first_call():
+        try:
+            with torch.cuda.stream(fresh):
+                run(xs[1], z)
+        except Exception as e:  # noqa: BLE001  (reported by the main thread, whose capture has to end first)
+            failed.append(e)
+
+    cap = torch.cuda.Stream()
+    with torch.cuda.stream(cap):
+        run(xs[0], y)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=cap):
+        t = threading.Thread(target=first_call)
+        t.start()
+        t.join()
+        run(xs[0], y)
+    torch.cuda.synchronize()
+    assert not failed, failed
+    assert torch.equal(z, want[1]), path
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want[0]), path

@@ -202,6 +202,20 @@ static void graphs_give_back() {
     EXPECT(ws_count(kWsDec) == before);
 }
 
+// a stream's first call while another thread captures on another stream in the global mode
+static void allocate_beside_a_capture() {
+    Graph* g = begin_capture(stream(1));
+    std::thread([] {
+        for (int kind = 0; kind < kNumWs; kind++) {
+            EXPECT(WsHold(stream(2)).get(kind, 1 << 20) != nullptr);
+            EXPECT(WsHold(nullptr).get(kind, 1 << 20) != nullptr);
+        }
+        EXPECT(t_mode == hipStreamCaptureModeGlobal);
+    }).join();
+    end_capture(stream(1));
+    unref(g);
+}
+
 // no memory under capture: no buffer, and the capture goes on
 static void capture_without_memory() {
     hipStream_t st = stream(1);
@@ -219,6 +233,7 @@ int main(int argc, char** argv) {
                                                    {"another_stream_runs", another_stream_runs},
                                                    {"captures_have_their_own", captures_have_their_own},
                                                    {"graphs_give_back", graphs_give_back},
+                                                   {"allocate_beside_a_capture", allocate_beside_a_capture},
                                                    {"capture_without_memory", capture_without_memory}};
     EXPECT(argc == 2 && all.count(argv[1]));
     all.at(argv[1])();
