@@ -8,7 +8,7 @@
 // overwrite each other's data. A call's launches that write and read a buffer have to follow each other on the stream
 // without another call's in between, and host threads may call on one stream (torch's threads share the default one),
 // so a call holds the stream's lock (WsHold) from its first buffer to its last launch.
-// A buffer grows on a call outside graph capture; the outgrown one is kept allocated (retired).
+// A buffer grows on a call outside graph capture; the outgrown one is freed when the stream's work on it is done.
 //
 // Calls under graph capture never get the stream's buffer: a graph replays on whatever stream it is launched on, beside
 // eager calls on the stream it was captured on or another graph captured there. The calls of one capture on one stream
@@ -22,7 +22,6 @@
 #include <memory>
 #include <mutex>
 #include <utility>
-#include <vector>
 
 #include "qe_api.hpp"
 
@@ -50,7 +49,6 @@ namespace {
 struct State {
     std::mutex mu;  // guards the rest; never held over a HIP call or while a stream's lock is waited for
     std::map<std::pair<int, hipStream_t>, std::unique_ptr<StreamWs>> streams;  // (device, stream), never erased
-    std::vector<void*> retired;
     std::multimap<std::pair<int, int>, CapBuf*> pool;  // (device, kind)
     int count[kNumWs] = {};
 };
@@ -178,10 +176,12 @@ void* WsHold::get(int kind, size_t bytes) {
     }
     HIP_CHECK(e);
     if (kind == kWsDec) zero_fill(np, bytes);
-    {
+    if (w.p) {  // only this stream's calls use it, and they are all enqueued (the lock)
+        HIP_CHECK(hipStreamSynchronize(st_));
+        HIP_CHECK(hipFree(w.p));
+    } else {
         std::lock_guard<std::mutex> lk(state().mu);
-        if (w.p) state().retired.push_back(w.p);
-        else state().count[kind]++;
+        state().count[kind]++;
     }
     w.p = np;
     w.bytes = bytes;

@@ -19,7 +19,7 @@ def model(tmp_path_factory):
 
 
 @pytest.mark.parametrize("scenario", ["threads_on_one_stream", "another_stream_runs", "captures_have_their_own",
-                                      "graphs_give_back", "allocate_beside_a_capture", "capture_without_memory"])
+                                      "graphs_give_back", "allocate_beside_a_capture", "capture_without_memory", "growth_frees"])
 def test_workspace(model, scenario):
     r = subprocess.run([model, scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.endswith("OK\n"), r.stdout + r.stderr

@@ -32,8 +32,10 @@ struct Capture {
 std::mutex g_model;
 std::map<hipStream_t, Capture> g_captures;  // streams being captured
 unsigned long long g_next_id = 0;
-size_t g_allocs = 0;
-bool g_oom = false;
+size_t g_allocs = 0, g_tries = 0, g_held = 0;  // allocations, attempts, bytes held
+std::map<void*, size_t> g_sizes;
+std::atomic<bool> g_oom{false};
+std::map<hipStream_t, int> g_synced;  // synchronizations by stream
 thread_local hipStreamCaptureMode t_mode = hipStreamCaptureModeGlobal;
 
 Graph* begin_capture(hipStream_t st) {
@@ -86,9 +88,20 @@ hipError_t hipGraphRetainUserObject(hipGraph_t g, hipUserObject_t o, unsigned, u
 hipError_t hipMalloc(void** p, size_t n) {
     std::lock_guard<std::mutex> lk(g_model);
     if (t_mode == hipStreamCaptureModeGlobal && !g_captures.empty()) return hipErrorStreamCaptureUnsupported;
+    g_tries++;
     if (g_oom) return hipErrorOutOfMemory;
     g_allocs++;
+    g_held += n;
     *p = malloc(n);
+    g_sizes[*p] = n;
+    return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+    std::lock_guard<std::mutex> lk(g_model);
+    if (t_mode == hipStreamCaptureModeGlobal && !g_captures.empty()) return hipErrorStreamCaptureUnsupported;
+    g_held -= g_sizes.at(p);
+    g_sizes.erase(p);
+    free(p);
     return hipSuccess;
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
@@ -100,7 +113,11 @@ hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) {
     memset(p, v, n);
     return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t st) {
+    std::lock_guard<std::mutex> lk(g_model);
+    g_synced[st]++;
+    return hipSuccess;
+}
 }
 int qe_num_cus() { return 4; }
 [[noreturn]] void qe_fatal_check() {
@@ -228,13 +245,68 @@ static void capture_without_memory() {
     unref(g);
 }
 
+static void* get(hipStream_t st, int kind, size_t bytes) { return WsHold(st).get(kind, bytes); }
+static size_t sized(hipStream_t st, int kind) { return WsHold(st).sized(kind); }
+
+// a growing call gives the outgrown buffer back once the stream's work on it is done
+static void growth_frees() {
+    hipStream_t st = stream(1);
+    Graph* g = begin_capture(stream(2));  // (freeing beside a capture, too)
+    for (int kind = 0; kind < kNumWs; kind++)
+        for (size_t mb = 1; mb <= 40; mb++) {
+            const size_t held = g_held, own = sized(st, kind);
+            const int synced = g_synced[st];
+            EXPECT(get(st, kind, mb << 20) && sized(st, kind) == mb << 20);
+            EXPECT(g_held == held - own + (mb << 20) && g_synced[st] == synced + (mb > 1));
+            EXPECT(get(st, kind, 1 << 20) && g_held == held - own + (mb << 20));
+        }
+    end_capture(stream(2));
+    unref(g);
+}
+
+// no memory: the calls that can run without a buffer are told so and do not ask the device each time; they get one later
+static void without_memory() {
+    for (int kind : {kWsSplit, kWsDec, kWsSkinny}) {
+        hipStream_t st = stream(1);
+        g_oom = true;
+        const size_t tries = g_tries;
+        for (int i = 0; i < 1000; i++) EXPECT(get(st, kind, 2 << 20) == nullptr);
+        EXPECT(g_tries - tries >= 2 && g_tries - tries <= 10);
+        EXPECT(get(st, kind, 1 << 20) == nullptr);
+        EXPECT(g_tries - tries <= 11);  // a smaller size is asked for
+        g_oom = false;
+        int i = 0;
+        while (get(st, kind, 2 << 20) == nullptr) EXPECT(++i < 1000);
+        EXPECT(get(st, kind, 1 << 20) != nullptr);
+        g_oom = true;  // growing fails: the smaller buffer stays
+        EXPECT(get(st, kind, 4 << 20) == nullptr && get(st, kind, 2 << 20) != nullptr);
+        g_oom = false;
+    }
+}
+
+// what a reserve that cannot be met reports
+static void reserve_in_capture() {
+    ws_reserve(kWsSplit, 1 << 20, stream(1));
+    begin_capture(stream(1));
+    ws_reserve(kWsSplit, 1 << 20, stream(1));
+    ws_reserve(kWsSplit, 2 << 20, stream(1));
+}
+static void reserve_without_memory() {
+    g_oom = true;
+    ws_reserve(kWsSplit, 1 << 20, stream(1));
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> all = {{"threads_on_one_stream", threads_on_one_stream},
                                                    {"another_stream_runs", another_stream_runs},
                                                    {"captures_have_their_own", captures_have_their_own},
                                                    {"graphs_give_back", graphs_give_back},
                                                    {"allocate_beside_a_capture", allocate_beside_a_capture},
-                                                   {"capture_without_memory", capture_without_memory}};
+                                                   {"capture_without_memory", capture_without_memory},
+                                                   {"growth_frees", growth_frees},
+                                                   {"without_memory", without_memory},
+                                                   {"reserve_in_capture", reserve_in_capture},
+                                                   {"reserve_without_memory", reserve_without_memory}};
     EXPECT(argc == 2 && all.count(argv[1]));
     all.at(argv[1])();
     printf("OK\n");
