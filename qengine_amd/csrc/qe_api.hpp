@@ -118,7 +118,8 @@ class WsHold {
     // capture: a buffer that the graph holds; nullptr for kWsSplit, kWsI8 and kWsH where the stream's own has not that
     // size. nullptr too where the device has no memory for a kWsSplit, kWsDec or kWsSkinny buffer. kWsDec buffers
     // (the one-pass decode's tail counters and sums) are zero-filled when allocated; the kernel leaves its counters zero.
-    void* get(int kind, size_t bytes);
+    // retry: ask the device also shortly after it had no memory.
+    void* get(int kind, size_t bytes, bool retry = false);
     // the tail workspace of the decode kernels (kWsDec, one size for every shape): dec_tail_ctr_bytes() of counters
     // (one per tail tile or slab, at most one per CU), then the tail parts' sums (up to 64 x 128 floats per CU)
     char* dec_tail();

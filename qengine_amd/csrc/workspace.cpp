@@ -17,7 +17,8 @@
 // that lived at one time needed. The pre-passes and the GEMM's split keep the rule that a capture needs its stream
 // sized first (an eager call or ws_reserve there): get returns nullptr else, and the caller runs without the buffer (the
 // split) or aborts with a message (the pre-passes). The decode kernels' buffers need no preparation. They and the split
-// also run without a buffer when the device has no memory left for it.
+// also run without a buffer when the device has no memory left for it; a failed hipMalloc takes longer than the call,
+// so the next kRetry calls do not try again.
 #include <map>
 #include <memory>
 #include <mutex>
@@ -26,9 +27,12 @@
 #include "qe_api.hpp"
 
 namespace {
+constexpr int kRetry = 256;  // calls that do without a buffer after the device had no memory for it, before it is asked again
 struct Ws {
     void* p = nullptr;
     size_t bytes = 0;
+    size_t refused = 0;  // the size it had no memory for, and the calls of at least that size left to do without
+    int wait = 0;
 };
 struct CapBuf {  // a buffer that a graph holds, or one in the pool (owner 0)
     int dev, kind;
@@ -160,18 +164,25 @@ bool needs_sizing(int kind) { return kind == kWsSplit || kind == kWsI8 || kind =
 WsHold::WsHold(hipStream_t st) : st_(st), s_(stream_of(st)) { s_->mu.lock(); }
 WsHold::~WsHold() { s_->mu.unlock(); }
 
-void* WsHold::get(int kind, size_t bytes) {
+void* WsHold::get(int kind, size_t bytes, bool retry) {
     CHECK(kind >= 0 && kind < kNumWs, "workspace kind %d", kind);
     Ws& w = s_->ws[kind];
     unsigned long long id = 0;
     hipGraph_t graph = nullptr;
     if (capturing(st_, &id, &graph)) return needs_sizing(kind) && w.bytes < bytes ? nullptr : capture_buf(s_, kind, bytes, id, graph);
     if (w.bytes >= bytes) return w.p;
+    const bool optional = kind != kWsI8 && kind != kWsH;  // the caller runs without it
+    if (optional && !retry && w.wait > 0 && bytes >= w.refused) {
+        w.wait--;
+        return nullptr;
+    }
     RelaxedCapture relaxed;
     void* np = nullptr;
     const hipError_t e = hipMalloc(&np, bytes);
-    if (e == hipErrorOutOfMemory && kind != kWsI8 && kind != kWsH) {  // every other caller runs without its buffer
+    if (e == hipErrorOutOfMemory && optional) {
         (void)hipGetLastError();
+        w.refused = bytes;
+        w.wait = kRetry;
         return nullptr;
     }
     HIP_CHECK(e);
@@ -185,6 +196,7 @@ void* WsHold::get(int kind, size_t bytes) {
     }
     w.p = np;
     w.bytes = bytes;
+    w.wait = 0;
     return np;
 }
 
@@ -202,7 +214,7 @@ void ws_reserve(int kind, size_t bytes, hipStream_t st) {
     hipGraph_t graph = nullptr;
     WsHold hold(st);
     if (capturing(st, &id, &graph)) CHECK(hold.sized(kind) >= bytes, "workspace reserve: called during graph capture");
-    else CHECK(hold.get(kind, bytes) != nullptr, "workspace reserve: no memory for %zu bytes", bytes);
+    else CHECK(hold.get(kind, bytes, true) != nullptr, "workspace reserve: no memory for %zu bytes", bytes);
 }
 
 int ws_count(int kind) {

@@ -19,7 +19,15 @@ def model(tmp_path_factory):
 
 
 @pytest.mark.parametrize("scenario", ["threads_on_one_stream", "another_stream_runs", "captures_have_their_own",
-                                      "graphs_give_back", "allocate_beside_a_capture", "capture_without_memory", "growth_frees"])
+                                      "graphs_give_back", "allocate_beside_a_capture", "capture_without_memory", "growth_frees",
+                                      "without_memory"])
 def test_workspace(model, scenario):
     r = subprocess.run([model, scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.endswith("OK\n"), r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("scenario,msg", [("reserve_in_capture", "called during graph capture"),
+                                          ("reserve_without_memory", "no memory for 1048576 bytes")])
+def test_reserve_that_cannot_be_met(model, scenario, msg):
+    r = subprocess.run([model, scenario], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 3 and "FATAL" in r.stdout and msg in r.stderr, r.stdout + r.stderr

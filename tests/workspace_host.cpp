@@ -278,8 +278,12 @@ static void without_memory() {
         int i = 0;
         while (get(st, kind, 2 << 20) == nullptr) EXPECT(++i < 1000);
         EXPECT(get(st, kind, 1 << 20) != nullptr);
+        g_oom = true;
+        EXPECT(get(st, kind, 3 << 20) == nullptr);
+        g_oom = false;
+        ws_reserve(kind, 3 << 20, st);  // a reserve asks at once
         g_oom = true;  // growing fails: the smaller buffer stays
-        EXPECT(get(st, kind, 4 << 20) == nullptr && get(st, kind, 2 << 20) != nullptr);
+        EXPECT(get(st, kind, 4 << 20) == nullptr && get(st, kind, 3 << 20) != nullptr);
         g_oom = false;
     }
 }
