@@ -101,7 +101,10 @@ void qe_gemm_h_reserve_s(int k, int t, void* stream);
  * src/capi.cpp:109 (act bf16 [t][n/2] of a GLU matrix); ci / ks (the reference's tile candidate and kernel variant)
  * are accepted and ignored. qe_gemm_w4_i8_ex: strides, stream, flags QE_SCALE_F16 / QE_OUT_BF16 / QE_GLU. The
  * pre-pass buffer (t * (k + k / 8) bytes) is the library's, one per (device, stream), grown on first use;
- * qe_gemm_i8_reserve(k, t) sizes the default stream's, qe_gemm_i8_reserve_s that of `stream`, before graph capture. */
+ * qe_gemm_i8_reserve(k, t) sizes the default stream's, qe_gemm_i8_reserve_s that of `stream`, before graph capture, and
+ * with it the split-K workspace (64 MB: calls whose tiles do not fill the CUs run the last round of tiles in K ranges).
+ * A row's fp32 sum over the groups is therefore taken in ranges or not depending on the tile it falls in, i.e. on t;
+ * qe_gemm_set_sk_maxparts(1) keeps every row in one chain over k, whose bits do not depend on t. */
 void qe_gemm_w4_i8(const void* q, const void* s, int n, int k, const uint16_t* x, float* y, int t, int G, int ci,
                    int ks);
 void qe_gemm_w4_i8_glu(const void* q, const void* s, int n, int k, const uint16_t* x, void* act, int t, int G, int ci,
@@ -195,11 +198,11 @@ void qe_gemm_w4_s(const void* q, const void* s, int n, int k, const uint16_t* x,
 /* on != 0: later non-GLU GEMM calls write bf16 (round to nearest even) into y viewed as bf16 [t][n].
  * Replaces reference src/capi.cpp:114 (gemm_set_out_bf16, gemm.cu:4363-4375). */
 void qe_gemm_set_out_bf16(int on);
-/* run-time cap of the stream-K split: later prefill GEMM calls (W4, W8 / Q8 bf16-activation GEMMs) split the tiles
- * of their last partial round into at most n K ranges (n <= 0: no cap, the default; splits here are 1..16, n = 1
- * turns the split off). Applies to the cost model's, the tuner's and a stored choice alike (the cost model picks among
- * the allowed ones; a stored split above the cap is halved until it fits). Replaces reference src/capi.cpp:115
- * (gemm_set_sk_maxparts, gemm.cu:3485-3496,4359). */
+/* run-time cap of the stream-K split: later prefill GEMM calls (W4, W8 / Q8 bf16-activation GEMMs, W4A8 and Q8 W8A8;
+ * the W8-layout W8A8 and the fp16-accumulate GEMM do not split) split the tiles of their last partial round into at most
+ * n K ranges (n <= 0: no cap, the default; splits here are 1..16, n = 1 turns the split off). Applies to the cost
+ * model's, the tuner's and a stored choice alike (the cost model picks among the allowed ones; a stored split above the
+ * cap is halved until it fits). Replaces reference src/capi.cpp:115 (gemm_set_sk_maxparts, gemm.cu:3485-3496,4359). */
 void qe_gemm_set_sk_maxparts(int n);
 
 /* RTN INT8 group-128 quantization of a row-major bf16 [n][k] into the W8 layout: scale = bf16(amax/127),

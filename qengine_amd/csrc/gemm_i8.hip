@@ -672,7 +672,10 @@ void gemm_w8a8(const W8& w, const uint16_t* x, int ldx, void* c, int ldc, int t,
 }
 
 void gemm_i8_reserve(int k, int t, hipStream_t st) {
-    if (k > 0 && t > 0) ws_reserve(kWsI8, i8_ws_bytes(k, t), st);
+    if (k <= 0 || t <= 0) return;
+    ws_reserve(kWsI8, i8_ws_bytes(k, t), st);
+    // n is not known here: the most that a split may take, if there is memory for it (the calls run unsplit else)
+    (void)WsHold(st).get(kWsSplit, max_split_bytes(), true);
 }
 
 void gemm_w4_i8(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, int G, bool out_bf16,

@@ -176,6 +176,38 @@ def test_decode_captured_without_preparation(dev, path, kind):
     assert counts == [1, 0] * 3, counts
 
 
+def _fresh_stream():
+    """a non-blocking stream that no call was made on (torch hands out 32 of its own in turn)"""
+    hip = ctypes.CDLL("libamdhip64.so")
+    raw = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(raw), 1) == 0
+    return torch.cuda.ExternalStream(raw.value)
+
+
+@pytest.mark.parametrize("G", [32, 64, 128])
+def test_w4a8_captured_after_its_reserve(dev, G):
+    """qe_gemm_i8_reserve_s is all that a W4A8 capture needs: the split of the eager call, hence its bits"""
+    n, k, t = 1040, 2176, 100
+    w, _, _ = setup(n, k, 1, seed=n + t)
+    x = synth.to_dev(synth.x_host(t, k, seed=1))
+    want = ops.gemm_w4_i8(w, x, G=G)
+    call("qe_gemm_set_sk_maxparts", 1)
+    try:
+        unsplit = ops.gemm_w4_i8(w, x, G=G)
+    finally:
+        call("qe_gemm_set_sk_maxparts", 0)
+    assert not torch.equal(unsplit, want)  # (the eager call splits)
+    st = _fresh_stream()
+    call("qe_gemm_i8_reserve_s", k, t, ctypes.c_void_p(st.cuda_stream))
+    y = torch.empty_like(want)
+    g = _graph(lambda a, b: ops.gemm_w4_i8(w, a, G=G, y=b), x, y, st)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+
+
 @pytest.mark.parametrize("path", list(PATHS))
 def test_first_call_beside_a_capture(dev, path):
     """a stream's first call, which allocates its buffer, while another thread captures in the default (global) mode: both
@@ -183,10 +215,7 @@ def test_first_call_beside_a_capture(dev, path):
     run, xs = _case(path)
     want = [run(x) for x in xs]
     y, z = torch.empty_like(want[0]), torch.empty_like(want[1])
-    hip = ctypes.CDLL("libamdhip64.so")
-    raw = ctypes.c_void_p()
-    assert hip.hipStreamCreateWithFlags(ctypes.byref(raw), 1) == 0  # non-blocking, no call made on it yet
-    fresh = torch.cuda.ExternalStream(raw.value)
+    fresh = _fresh_stream()
     failed = []
 
     def first_call():
