@@ -121,8 +121,8 @@ int qe_gemm_w4_choice(const void* q, const void* s, int n, int k, const uint16_t
 /* test hook: the one-pass decode GEMM of qe_matmul_w4_ex for m = 1..64 rows whatever the dispatch would pick (the
  * weights read once for all rows, as the reference's wide decode GEMVs, src/kernels/gemv_x.cu:902-980; this build's
  * decode numerics: the exact products (u - 8) x summed in fp32 and scaled once per 128-k group). Returns 0 without
- * running when the shape does not fit it (n % 64, x not 16-byte aligned or ldx % 8, K / 64 not an even number of
- * steps per wave), else 1. */
+ * running when the shape does not fit it (n % 64, x not 16-byte aligned or ldx % 8; up to 32 rows also K not a
+ * multiple of 512), else 1. */
 int qe_matmul_w4_onepass_ex(const void* q, const void* s, int n, int k, const uint16_t* x, int ldx, void* y, int ldy,
                             int m, int flags, void* stream);
 

@@ -56,7 +56,7 @@ void skinny_w4_wide(const W4& w, const uint16_t* x, int ldx, void* y, int ldy, i
 bool skinny_w4_wide_fits(const W4& w, const uint16_t* x, int ldx);
 // one pass over the weights for 1..64 rows (wdec.hip): the decode numerics (exact (u - 8) x products, group scale on
 // the fp32 sums) on the 32 x 32 matrix cores, K split over the waves of a block, fixed-order sums; n % 64 == 0, x
-// 16-byte aligned, ldx % 8 == 0 and the K steps even per wave (wdec_w4_fits)
+// 16-byte aligned, ldx % 8 == 0 and up to 32 rows K % 512 == 0 (wdec_w4_fits)
 bool wdec_w4_fits(const W4& w, const uint16_t* x, int ldx, int m);
 // the dispatch's choice for 17..64 rows outside batch_invariant: fits, and faster than the skinny kernel's launches
 bool wdec_w4_pick(const W4& w, const uint16_t* x, int ldx, int m);

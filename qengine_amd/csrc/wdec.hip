@@ -617,7 +617,8 @@ int tail_parts(int nslabs, int KT, int KP, int ncu) {
 }
 }  // namespace qe_wdec
 
-bool wdec_w4_fits(const W4& w, const uint16_t* x, int ldx, int m) {
+// wdec_kernel's limits
+static bool one_fits(const W4& w, const uint16_t* x, int ldx, int m) {
     using namespace qe_wdec;
     if (m < 1 || m > 64 || w.n % 64 != 0 || w.k % BK != 0 || ((uintptr_t)x & 15) != 0 || ldx % 8 != 0) return false;
     const int KP = NW / token_blocks(m), KT = w.k / BK;
@@ -634,11 +635,15 @@ static bool two_fits(const W4& w, const uint16_t* x, int ldx, int m) {
            ldx % 8 == 0;
 }
 
+bool wdec_w4_fits(const W4& w, const uint16_t* x, int ldx, int m) {
+    return m > 32 ? two_fits(w, x, ldx, m) : one_fits(w, x, ldx, m);  // (two_fits covers one_fits)
+}
+
 // 33..64 rows: wdec_kernel (two token blocks, 64-row slabs, two blocks to a CU) where it was the choice before
 // wdec2_kernel: a round of slabs or more, K without an even skinny slicing, or more than 48 rows of a large matrix
 static bool small_slabs_fit(const W4& w, const uint16_t* x, int ldx, int m) {
     using namespace qe_wdec;
-    if (!wdec_w4_fits(w, x, ldx, m)) return false;
+    if (!one_fits(w, x, ldx, m)) return false;
     const int nslabs = w.n / 64, ncu = qe_num_cus();
     // slabs filling at most half the CUs only with K parts (N = 4096, K = 11008, m = 48: 64 slabs, no part count fits
     // 172 steps: 48.4 us against 35.2)
@@ -701,7 +706,7 @@ bool wdec_w4_pick(const W4& w, const uint16_t* x, int ldx, int m) {
 // (wdec2_kernel: two_parts, summed by a kernel of their own.)
 void wdec_w4(const W4& w, const uint16_t* x, int ldx, void* y, int ldy, int m, bool out_bf16, hipStream_t st) {
     using namespace qe_wdec;
-    CHECK(wdec_w4_fits(w, x, ldx, m) || two_fits(w, x, ldx, m), "wdec_w4: n %d k %d m %d ldx %d", w.n, w.k, m, ldx);
+    CHECK(wdec_w4_fits(w, x, ldx, m), "wdec_w4: n %d k %d m %d ldx %d", w.n, w.k, m, ldx);
     CHECK(ldy >= (w.glu ? w.n / 2 : w.n), "wdec_w4 ldy %d", ldy);
     const int out = w.glu ? 2 : out_bf16 ? 1 : 0;
     if (m > 32 && !(small_slabs_fit(w, x, ldx, m) && small_slabs_pay(w.n, w.k))) {

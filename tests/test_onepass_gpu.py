@@ -83,6 +83,22 @@ def test_onepass_shape_checks(dev):
     assert ops.matmul_w4_onepass(w3, xb) is None
 
 
+@pytest.mark.parametrize("n,k", [(64, 128), (192, 384), (1024, 1280), (4160, 640)])
+def test_onepass_33_rows_take_any_groups(dev, n, k):
+    """33..64 rows: any whole number of 128-k groups is taken (up to 32 rows K % 512 == 0), other shapes are declined"""
+    w, q, s = setup_w4(n, k, 1, seed=n)
+    xh = synth.x_host(40, k, seed=k)
+    x = synth.to_dev(xh)
+    y = ops.matmul_w4_onepass(w, x)
+    assert y is not None
+    assert err_ratio(out_f32(y), matmul_f64(xh, exact_w4(q, s, n, k, 1))) <= 1e-4
+    assert ops.matmul_w4_onepass(w, x[:32]) is None
+    odd, _, _ = setup_w4(n + 16, k, 1, seed=n)
+    assert ops.matmul_w4_onepass(odd, x) is None
+    xb = torch.zeros(40 * k + 1, dtype=torch.bfloat16, device=dev)[1:].view(40, k)
+    assert ops.matmul_w4_onepass(w, xb) is None
+
+
 def test_onepass_tail_parts_deterministic_and_graph(dev):
     """N = 17408 has 272 slabs of 64 rows: the 16 past the last whole round of 256 CUs run as K parts added by the
     last part to finish (a device-side count per tail slab, zero again after every call). Repeated calls, calls of
