@@ -595,8 +595,8 @@ void run_choice(int cfg, int ks, const uint4* q, const uint16_t* s, int n, int k
     float* part = nullptr;
     std::optional<WsHold> hold;  // until the sum of the partials is launched
     if (ks > 1) {
-        // no such split, or no workspace for it (memory; a graph capture on a stream that was not sized before): the
-        // best unsplit configuration
+        // no such split: these tiles unsplit; no workspace for it (memory; a graph capture on a stream that was not
+        // sized before): the best unsplit configuration
         if (!gemm_geom(cfg, n, k, t, ks, g)) ks = 1;
         else if ((part = static_cast<float*>(hold.emplace(st).get(kWsSplit, g.ws_bytes))) == nullptr) {
             ks = 1;
@@ -662,7 +662,7 @@ GemmChoice gemm_tune_choice(int n, int k, const uint16_t* x, int ldx, int t, voi
     return cl[best];
 }
 
-// a stored or tuned split halved until qe_gemm_set_sk_maxparts allows it
+// a stored or tuned split, halved until qe_gemm_set_sk_maxparts allows it
 int capped_split(int ks) {
     const int cap = gemm_sk_maxparts();
     while (cap > 0 && ks > cap) ks /= 2;
@@ -674,7 +674,13 @@ void launch_gemm(const uint4* q, const uint16_t* s, int n, int k, const uint16_t
                  int out, int sdt, bool tuned, hipStream_t st) {
     GemmChoice ch;
     const GemmKey key{FMT, n, k, gemm_bucket(t), out == kOutGLU ? 1 : 0};
-    if (!gemm_table_find(key, ch)) {
+    if (gemm_table_find(key, ch)) {
+        // a stored split that the cap takes away, or that does not apply at this t of its bucket, leaves large tiles that
+        // fill few CUs (1280 x 8192, t = 200: 173 us unsplit at 256 x 256, 94 at 128 x 128): the model's choice instead
+        GemmGeom g;
+        if (ch.ks > 1 && (capped_split(ch.ks) == 1 || !gemm_geom(ch.cfg, n, k, t, capped_split(ch.ks), g)))
+            ch = gemm_model_choice(FMT != kFmtW4, n, k, t, gemm_sk_maxparts());
+    } else {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         HIP_CHECK(hipStreamIsCapturing(st, &cs));
         if ((tuned || qe_config().gemm_tune) && cs == hipStreamCaptureStatusNone) {

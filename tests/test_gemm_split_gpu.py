@@ -98,6 +98,71 @@ def test_tune_file_with_two_tile_shapes(dev, tmp_path):
         call("qe_gemm_tune_clear")
 
 
+@pytest.fixture
+def stored(tmp_path):
+    """stored((fmt, n, k, bucket, glu, cfg, ks), ..): a tuning file of these choices for this device is loaded (fmt 0 W4,
+    1 W8 group scales, 2 W8 per channel, 3 Q8)"""
+    p = tmp_path / "tune.txt"
+
+    def load(*entries):
+        call("qe_gemm_tune_clear")
+        call("qe_gemm_tune_file", ctypes.c_char_p(str(p).encode()))
+        w, _, _ = setup(64, 128, 0, seed=1)
+        y = torch.empty(70, 64, device="cuda")
+        call("qe_gemm_w4_t", w.q, w.s, 64, 128, synth.to_dev(synth.x_host(70, 128, seed=1)), y, 70)  # writes the file
+        head = p.read_text().splitlines()[:2]  # format and device
+        p.write_text("\n".join(head + [" ".join(map(str, e)) for e in entries]) + "\n")
+        call("qe_gemm_tune_clear")
+        call("qe_gemm_tune_file", ctypes.c_char_p(str(p).encode()))
+        lib().qe_gemm_tune_entries.restype = ctypes.c_int
+        assert lib().qe_gemm_tune_entries() == len(entries)
+
+    yield load
+    call("qe_gemm_tune_file", ctypes.c_char_p(b""))
+    call("qe_gemm_tune_clear")
+
+
+def _us(f, calls=10):
+    best = float("inf")
+    f()
+    for _ in range(5):
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        e0.record()
+        for _ in range(calls):
+            f()
+        e1.record()
+        torch.cuda.synchronize()
+        best = min(best, e0.elapsed_time(e1) * 1e3 / calls)
+    return best
+
+
+def test_stored_split_that_does_not_apply(dev, stored):
+    """a stored choice serves every token count of its bucket. Where its split would take more than the workspace bound
+    (80 tiles of 256 x 256 in 4 ranges), the call runs the untuned choice; where qe_gemm_set_sk_maxparts leaves no split,
+    the best unsplit tiles, not the stored ones (5 blocks of 256 x 256 take about twice as long as 20 of 128 x 128)"""
+    n, k, t = 5120, 4352, 1000
+    w, _, _ = setup(n, k, 1, seed=31)
+    x = synth.to_dev(synth.x_host(t, k, seed=32))
+    assert not ops.gemm_w4_choice(w, x, cfg=0, ks=4)[1]
+    want = ops.gemm_w4(w, x)
+    assert not torch.equal(want, ops.gemm_w4_choice(w, x, cfg=0, ks=1)[0])  # (the untuned choice splits)
+    stored((0, n, k, 1024, 0, 0, 4))
+    assert torch.equal(ops.gemm_w4(w, x), want)
+
+    n, k, t = 1280, 8192, 200
+    w, _, _ = setup(n, k, 1, seed=33)
+    x = synth.to_dev(synth.x_host(t, k, seed=34))
+    big = _us(lambda: ops.gemm_w4_choice(w, x, cfg=0, ks=1))
+    stored((0, n, k, 256, 0, 0, 12))
+    call("qe_gemm_set_sk_maxparts", 1)
+    try:
+        us = _us(lambda: ops.gemm_w4(w, x))
+    finally:
+        call("qe_gemm_set_sk_maxparts", 0)
+    print(f"1280 x 8192, t = 200 unsplit: 256 x 256 tiles {big:.1f} us, stored choice capped {us:.1f} us", flush=True)
+    assert us < 0.8 * big
+
+
 @pytest.mark.parametrize("n,k,t,G", [(272, 1152, 65, 64), (1040, 2176, 129, 32), (4112, 1152, 300, 128), (144, 128, 70, 64)])
 @pytest.mark.parametrize("glu", [False, True])
 def test_underfilled_w4a8(dev, n, k, t, G, glu):
