@@ -113,9 +113,9 @@ void qe_gemm_w4_i8_ex(const void* q, const void* s, int n, int k, const uint16_t
                       int G, int flags, void* stream);
 void qe_gemm_i8_reserve(int k, int t);
 void qe_gemm_i8_reserve_s(int k, int t, void* stream);
-/* test hook: qe_gemm_w4_ex with a given choice instead of the tuner's (cfg 0: 256 x 256 tiles, 1: 256 x 128; ks: K
- * ranges of the last partial round's tiles, 1 / 2 / 4); returns 1 if that split applies to the shape (else it runs
- * unsplit and returns 0). The reference's QE_GEMM_FORCE (src/kernels/gemm.cu:4376-4394). */
+/* test hook: qe_gemm_w4_ex with a given choice instead of the tuner's (cfg: tokens x rows of a tile, 0: 256 x 256,
+ * 1: 256 x 128, 2: 128 x 256, 3: 128 x 128; ks: K ranges of the last partial round's tiles, 1..16); returns 1 if that
+ * split applies to the shape (else it runs unsplit and returns 0). The reference's QE_GEMM_FORCE (src/kernels/gemm.cu:4376-4394). */
 int qe_gemm_w4_choice(const void* q, const void* s, int n, int k, const uint16_t* x, int ldx, void* y, int ldy, int t,
                       int flags, int cfg, int ks, void* stream);
 /* test hook: the one-pass decode GEMM of qe_matmul_w4_ex for m = 1..64 rows whatever the dispatch would pick (the

@@ -119,7 +119,6 @@ int qe_matmul_w4_onepass_ex(const void* q, const void* s, int n, int k, const ui
 
 int qe_gemm_w4_choice(const void* q, const void* s, int n, int k, const uint16_t* x, int ldx, void* y, int ldy, int t,
                       int flags, int cfg, int ks, void* stream) {
-    CHECK(cfg >= 0 && cfg < 2 && (ks == 1 || ks == 2 || ks == 4), "gemm choice cfg %d ks %d", cfg, ks);
     const W4 w = mk_w4(q, s, n, k, (flags & QE_GLU) != 0, (flags & QE_SCALE_F16) ? kScaleF16 : kScaleBF16);
     gemm_w4_choice(w, x, ldx, y, ldy, t, (flags & QE_OUT_BF16) != 0, cfg, ks, as_stream(stream));
     return ks > 1 && gemm_split_applies(cfg, n, k, t, ks) ? 1 : 0;

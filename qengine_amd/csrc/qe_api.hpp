@@ -140,7 +140,7 @@ void gemm_w4(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, b
              bool tuned = false);
 void gemm_w8(const W8& w, const uint16_t* x, int ldx, void* c, int ldc, int t, bool out_bf16, hipStream_t st,
              bool tuned = false);
-// a given choice (tile configuration 0: 256 x 256, 1: 256 x 128; ks K ranges of the last partial round, 1 = none);
+// a given choice (tile configuration 0..3 as GemmChoice; ks K ranges of the last partial round, 1..16, 1 = none);
 // falls back to ks = 1 where the split does not apply (gemm_split_applies false) or has no workspace
 void gemm_w4_choice(const W4& w, const uint16_t* x, int ldx, void* c, int ldc, int t, bool out_bf16, int cfg, int ks,
                     hipStream_t st);
@@ -159,7 +159,7 @@ void gemm_set_out_bf16(bool on);
 // reserve the split-K workspace of (the current device, st) (grown on demand otherwise; a capture wants it sized before)
 void gemm_reserve(size_t bytes, hipStream_t st);
 bool gemm_out_bf16();
-// run-time cap of the split count of the prefill GEMMs' last partial round (0 or less: no cap, i.e. up to 4)
+// run-time cap of the split count of the prefill GEMMs' last partial round (0 or less: no cap, i.e. up to 16)
 void gemm_set_sk_maxparts(int n);
 int gemm_sk_maxparts();
 

@@ -1,7 +1,7 @@
-"""Prefill GEMM calls whose tiles do not fill the CUs: the four tile shapes and the splits in up to 16 uneven K ranges
-that the cost model picks, against the oracle (1e-4 * rms: the products are the oracle's, only the order of the fp32
-sums differs). K = 1152 and 2176 are 9 and 17 groups (ranges of unequal length), t crosses the 128- and 256-token
-tiles, n leaves ragged row tiles."""
+"""Prefill GEMM calls whose tiles do not fill the CUs, against the oracle (1e-4 * rms: the products are the oracle's, only
+the order of the fp32 sums differs): what the cost model picks there (mostly 128 x 128 tiles in 9, 5 or 1 ranges at these
+sizes), and each of the four tile shapes with 1, 3, 10 and 16 ranges for every weight format. K = 1152 and 2176 are 9
+and 17 groups (ranges of unequal length), t crosses the 128- and 256-token tiles, n leaves ragged row tiles."""
 import ctypes
 
 import numpy as np
@@ -11,7 +11,8 @@ import torch
 import oracle
 from qengine_amd import call, lib, ops, synth
 from test_gemm_gpu import setup
-from test_gemv_gpu import assert_glu_close, err_ratio, glu_act, oracle_ref, out_f32
+from test_gemv_gpu import assert_glu_close, err_ratio, glu_act, matmul_f64, oracle_ref, oracle_ref_w8, out_f32
+from test_q8_gpu import q8_host
 
 pytestmark = pytest.mark.gpu
 
@@ -45,7 +46,6 @@ def test_underfilled_prefill(dev, n, k, t, glu):
 
 @pytest.mark.parametrize("per_channel", [True, False])
 def test_underfilled_prefill_w8(dev, per_channel):
-    from test_gemv_gpu import oracle_ref_w8
     n, k, t = 272, 1152, 140
     q, s = synth.w8_host(n, k, seed=3, per_channel=per_channel)
     w = ops.tile_w8(synth.to_dev(q), synth.to_dev(s, torch.float16), per_channel)
@@ -134,6 +134,71 @@ def _us(f, calls=10):
         torch.cuda.synchronize()
         best = min(best, e0.elapsed_time(e1) * 1e3 / calls)
     return best
+
+
+TILE = (1040, 2176, 270)  # 10 to 27 tiles: every one split
+_FMT = {}
+
+
+def _format(fmt):
+    """(run(x), the oracle's product or GLU activation of the inputs, format number) of a weight format at TILE"""
+    if fmt not in _FMT:
+        n, k, t = TILE
+        xh = synth.x_host(t, k, seed=41)
+        glu = fmt.endswith("glu")
+        if fmt.startswith("w4"):
+            w, q, s = setup(n, k, 1, seed=42, glu=glu)
+            run, ref, num = None, oracle_ref(xh, q, s, n, k, 1), 0
+        elif fmt.startswith("q8"):
+            q, s, _ = q8_host(n, k, 43)
+            w = ops.repack_q8(synth.to_dev(q), synth.to_dev(s), glu=glu)
+            if glu:
+                q, s = oracle.glu_rows(q, s, n, k, bits=8)
+            run, ref, num = ops.gemm_q8, matmul_f64(xh, oracle.bf16_to_f32(oracle.dequant_q8(q, s, n, k))), 3
+        else:
+            pc = fmt == "w8c"
+            q, s = synth.w8_host(n, k, seed=44, per_channel=pc)
+            w = ops.tile_w8(synth.to_dev(q), synth.to_dev(s, torch.float16), pc)
+            run, ref, num = ops.gemm_w8, oracle_ref_w8(xh, q, s, n, k, pc), 2 if pc else 1
+        _FMT[fmt] = w, run, glu_act(ref) if glu else ref, num, synth.to_dev(xh)
+    return _FMT[fmt]
+
+
+@pytest.mark.parametrize("ks", [1, 3, 10, 16])
+@pytest.mark.parametrize("cfg", [0, 1, 2, 3])
+@pytest.mark.parametrize("fmt", ["w4", "w4glu", "w8g", "w8c", "q8", "q8glu"])
+def test_every_tile_shape_and_split(dev, stored, fmt, cfg, ks):
+    """a given tile shape and split (INT4 by the hook, the others by a tuning file): the oracle's product, and where it is
+    split other bits than unsplit"""
+    n, k, t = TILE
+    w, run, ref, num, x = _format(fmt)
+    glu = fmt.endswith("glu")
+    if run is None:
+        y, applied = ops.gemm_w4_choice(w, x, cfg, ks)
+        one, _ = ops.gemm_w4_choice(w, x, cfg, 1)
+        assert applied == (ks > 1)
+    else:
+        stored((num, n, k, 512, int(glu), cfg, ks))
+        y = run(w, x)
+        stored((num, n, k, 512, int(glu), cfg, 1))
+        one = run(w, x)
+    if glu:
+        assert_glu_close(out_f32(y), ref, 1e-3 if fmt == "q8glu" else 1e-4)
+    else:
+        assert err_ratio(out_f32(y), ref) <= 1e-4
+    assert torch.equal(y, one) == (ks == 1)
+
+
+@pytest.mark.parametrize("cfg", [1, 2, 3])
+def test_whole_rounds_and_split_tiles(dev, cfg):
+    """256 (128 x 128: 512) whole tiles and 33 to 49 of three ranges of 9 groups in one launch"""
+    n, k, t = 4112, 1152, 2100
+    w, q, s = setup(n, k, 1, seed=45)
+    xh = synth.x_host(t, k, seed=46)
+    y, applied = ops.gemm_w4_choice(w, synth.to_dev(xh), cfg, 3)
+    assert applied
+    rows = np.unique(np.r_[0, 127, 128, 255, 256, 1900, 1920, 2047, 2048, 2099, np.random.default_rng(1).integers(0, t, 30)])
+    assert err_ratio(out_f32(y)[rows], oracle_ref(xh[rows], q, s, n, k, 1)) <= 1e-4
 
 
 def test_stored_split_that_does_not_apply(dev, stored):
