@@ -584,6 +584,8 @@ def test_skinny_slices_in_parts(dev, n, k, glu, m):
     pairs = torch.cat([ops.gemv_w4(w, x[i:i + 2].contiguous()) for i in range(m - 1)])
     torch.cuda.synchronize()
     exact = matmul_f64(xh, exact_w4(q, s, n, k, 1))
+    for _ in range(3):
+        assert torch.equal(ops.gemv_w4(w, x), y)
     if glu:
         assert_glu_close(out_f32(y), glu_act(exact), 1e-4)
     else:
@@ -609,3 +611,23 @@ def test_skinny_slices_in_parts(dev, n, k, glu, m):
             g.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, want), (warm, r)
+
+
+@pytest.mark.parametrize("n,k", [(4112, 13824), (5120, 17408)])
+@pytest.mark.parametrize("m", [9, 16])
+def test_skinny_slices_in_parts_forms(dev, n, k, m):
+    """the parts with bf16 scales: outputs at an odd offset and stride, fp32 and bf16, are the contiguous ones bit for bit
+    and write nothing else; activation rows that are 4-byte aligned only take one block per tile: the same bits"""
+    w, q, s = setup_w4(n, k, 0, seed=n + m)
+    xh = synth.x_host(m, k, seed=k + m)
+    x = synth.to_dev(xh)
+    y = ops.gemv_w4(w, x)
+    assert err_ratio(y.cpu().numpy(), matmul_f64(xh, exact_w4(q, s, n, k, 0))) <= 1e-4
+    for dt in (torch.float32, torch.bfloat16):
+        big = torch.full((m, n + 7), float("nan"), dtype=dt, device=dev)
+        z = ops.gemv_w4(w, x, out_bf16=dt == torch.bfloat16, y=big[:, 1:1 + n])
+        assert torch.equal(z, y.to(dt))
+        assert torch.isnan(big[:, 0]).all() and torch.isnan(big[:, 1 + n:]).all()
+    xu = torch.zeros(m, k + 10, dtype=torch.bfloat16, device=dev)[:, 2:2 + k]
+    xu.copy_(x)
+    assert torch.equal(ops.gemv_w4(w, xu), y)

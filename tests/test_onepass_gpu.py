@@ -100,8 +100,8 @@ def test_onepass_33_rows_take_any_groups(dev, n, k):
 
 
 def test_onepass_tail_parts_deterministic_and_graph(dev):
-    """N = 17408 has 272 slabs of 64 rows: the 16 past the last whole round of 256 CUs run as K parts added by the
-    last part to finish (a device-side count per tail slab, zero again after every call). Repeated calls, calls of
+    """N = 17408 has 272 slabs of 64 rows (40 rows take these too, two token blocks): the 16 past the last whole round of
+    256 CUs run as K parts added by the last part to finish (a device-side count per tail slab, zero again after every call). Repeated calls, calls of
     other shapes in between, and a HIP graph captured on a stream that ran the kernel eagerly all give the same bits;
     a capture on a stream that never ran it within 1e-5 * rms (test_workspace_gpu.py: the same bits)"""
     n, k = 17408, 5120
@@ -145,12 +145,14 @@ def test_onepass_tail_parts_deterministic_and_graph(dev):
                     assert rr <= 1e-5, (m, r, rr)
 
 
-@pytest.mark.parametrize("n,k", [(64, 128), (192, 384), (4160, 640), (5120, 3712), (33024, 256)])
+@pytest.mark.parametrize("n,k", [(64, 128), (192, 384), (4160, 640), (5120, 3712), (33024, 256), (4160, 3712),
+                                 (32896, 896), (33088, 896)])
 @pytest.mark.parametrize("m", [33, 48, 63, 64])
 def test_decode_33_to_64_rows(dev, n, k, m):
-    """the 33..64-row kernel through the row-count dispatch or alone: slabs with a ragged half (n % 128 = 64), K of
-    fewer groups than K parts, uneven K parts, K ranges of split slabs; outputs at an odd offset and stride are the
-    contiguous ones bit for bit; GLU"""
+    """the 33..64-row kernels through the row-count dispatch (skinny launches at 4160 x 640, 64-row slabs at 33024 x 256,
+    else 128-row slabs) and alone: slabs with a ragged half (n % 128 = 64), K of fewer groups than K parts, uneven K
+    parts, every slab split in K ranges (5120 and 4160 x 3712, the last ragged there), 256 whole slabs and 1 or 3 split
+    ones (896, the last ragged at 33088); outputs at an odd offset and stride are the contiguous ones bit for bit; GLU"""
     w, q, s = setup_w4(n, k, 1, seed=n + m)
     xh = synth.x_host(m, k, seed=k + m)
     x = synth.to_dev(xh)
@@ -163,9 +165,9 @@ def test_decode_33_to_64_rows(dev, n, k, m):
     wg, qg, sg = setup_w4(n, k, 1, seed=n + m + 1, glu=True)
     a = ops.matmul_w4(wg, x)
     assert_glu_close(out_f32(a), glu_act(matmul_f64(xh, exact_w4(qg, sg, n, k, 1))), 1e-4)
-    if k % 256 == 0:
-        y1 = ops.matmul_w4_onepass(w, x)
-        assert err_ratio(out_f32(y1), matmul_f64(xh, exact_w4(q, s, n, k, 1))) <= 1e-4
+    y1 = ops.matmul_w4_onepass(w, x)
+    assert err_ratio(out_f32(y1), matmul_f64(xh, exact_w4(q, s, n, k, 1))) <= 1e-4
+    assert torch.equal(ops.matmul_w4_onepass(w, x), y1)
 
 
 @pytest.mark.parametrize("n,k", [(16384, 256), (9216, 512), (16384, 1024), (17408, 2560), (20480, 3072), (49152, 512)])
