@@ -148,7 +148,7 @@ void qe_repack_w4(const int32_t* q, const uint16_t* s, int n, int k, void* dq, v
 
 /* y[m][n] (fp32, stride n) = x[m][k] (bf16, stride k) . W^T; any m (1..16 rows: the decode GEMV; 17..64: the
  * one-pass decode GEMM where the shape fits it and it is the faster choice (K without an even slicing of the skinny
- * kernel, up to 32 rows N >= 64 x the CU count, from 33 rows matrices of more than ~25 M weights), else the skinny
+ * kernel, N >= 64 x the CU count, from 33 rows matrices of more than ~25 M weights), else the skinny
  * kernel's 32- and 16-row launches, which batch_invariant always takes; the prefill GEMM above, as qe_matmul_w4_ex).
  * Replaces reference src/capi.cpp:47 (gemv_w4, gemv.cu:1585). */
 void qe_gemv_w4(const void* q, const void* s, int n, int k, const uint16_t* x, float* y, int m);

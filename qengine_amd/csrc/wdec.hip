@@ -654,22 +654,23 @@ static bool small_slabs_fit(const W4& w, const uint16_t* x, int ldx, int m) {
 // ... and still is. A 128-row slab of wdec2_kernel takes a CU alone, so it needs rounds of 128 ncu rows that are well
 // filled: with at most half of one (0 < r <= ncu slabs of 64 past the whole rounds) it splits K to fill the rest, which
 // short K does not pay back, and just past half it leaves half the CUs idle where 64-row slabs run their few extra ones
-// as tail parts. Tail parts cost wdec_kernel ~5 us, lost on short K. us, wdec_kernel / wdec2_kernel, m = 48:
-//   N      K = 256    512        1024       2048       3072       4096       5120       8192
-//   10240  5.4/8.2    6.5/8.3    8.6/12.5   12.8/15.1  17.0/16.1  21.4/18.3  25.7/20.8  38.2/25.6
-//   16384  5.6/8.3    6.7/8.4    8.8/13.9   13.2/16.0  17.4/18.6  21.9/21.2  26.1/24.1  38.8/32.3
-//   17408  6.6/8.4    11.3/8.5   13.9/10.9  16.7/16.3  19.3/21.0  23.8/25.8  27.8/31.0  40.8/44.6
-//   20480  6.7/8.4    12.4/8.6   15.4/11.0  18.8/16.3  21.1/21.1  25.6/26.4  29.8/31.1  42.9/46.1
-//   24576  6.8/8.5    13.5/8.7   15.2/11.1  19.3/16.5  23.3/21.9  27.5/27.4  31.9/32.3  46.8/46.6
-//   32768  6.9/8.7    8.5/8.8    11.5/12.0  18.6/17.5  25.2/23.3  31.7/29.0  38.4/32.9  58.4/49.9
-//   49152  9.0/14.2   11.3/14.6  16.3/21.6  26.6/30.6  36.5/38.3  46.8/47.8  56.9/53.4  88.3/79.8
-static bool small_slabs_pay(int n, int k) {
+// as tail parts. Tail parts cost wdec_kernel ~5 us, lost on short K; at 49..64 rows and from ncu / 16 extra slabs on
+// wdec2_kernel is the faster one (K = 5120: 17408 at 64 rows 32.7/31.5, 20480 at 48 rows 35.0/31.1). us, wdec_kernel /
+// wdec2_kernel, m = 48, weights rotating past the Infinity Cache, where the choice is near or was measured:
+//   N      K = 256       512       1024      2048      2560      3072      3584      4096      5120      8192
+//   16384      5.0/7.8   6.2/8.4   8.4/13.9  12.9/16.9 15.1/20.0 17.7/20.3 19.7/22.7
+//   17408      6.0/7.9                                 19.7/18.5 20.8/20.9 23.1/23.2 24.8/25.6 30.3/31.0 43.2/45.1
+//   18432      6.1/7.9                                           21.8/20.8 23.8/23.3 25.9/25.7 31.9/30.8 44.6/45.6
+//   20480      6.2/7.9                                           24.4/21.1 25.3/23.4 28.5/26.0 34.9/31.1 48.9/45.8
+//   43008      8.7/14.1  11.6/15.2 17.7/22.7 28.5/31.0 34.5/35.8 40.3/38.5 45.6/44.3
+//   49152      8.9/14.3  11.9/15.4 18.1/23.7 29.5/33.3 35.2/39.3 40.8/43.2 46.4/49.7
+static bool small_slabs_pay(int n, int k, int m) {
     using namespace qe_wdec;
     const int s = n / 64, ncu = qe_num_cus(), r = s % (2 * ncu);
     if (k <= 256) return true;
     if (tail_parts(s, k / BK, NW / 2, ncu) == 1)
-        return k <= 512 || (r > 0 && r <= ncu ? k <= (16 * s > 11 * ncu ? 3584 : 2560) : k <= 1280);
-    return r > ncu && ((r <= ncu + ncu / 16 && k >= 2560) || (s <= ncu + ncu / 4 && k >= 3072));
+        return k <= 512 || (r > 0 && r <= ncu ? k <= (16 * r > 11 * ncu ? 3584 : 2560) : k <= 1280);
+    return m <= 48 && r > ncu && r <= ncu + ncu / 16 && k >= 3072;
 }
 
 // Where the one-pass kernels beat the skinny kernel's 32-row launches (measured in one process, bf16 out, us one-pass
@@ -709,7 +710,7 @@ void wdec_w4(const W4& w, const uint16_t* x, int ldx, void* y, int ldy, int m, b
     CHECK(wdec_w4_fits(w, x, ldx, m), "wdec_w4: n %d k %d m %d ldx %d", w.n, w.k, m, ldx);
     CHECK(ldy >= (w.glu ? w.n / 2 : w.n), "wdec_w4 ldy %d", ldy);
     const int out = w.glu ? 2 : out_bf16 ? 1 : 0;
-    if (m > 32 && !(small_slabs_fit(w, x, ldx, m) && small_slabs_pay(w.n, w.k))) {
+    if (m > 32 && !(small_slabs_fit(w, x, ldx, m) && small_slabs_pay(w.n, w.k, m))) {
         const int ncu = qe_num_cus(), G = w.k >> 7, nsl = (w.n + two::ROWS - 1) / two::ROWS, rem = nsl % ncu;
         int P = rem > 0 ? two_parts(rem, G, ncu) : 1;
         float* tpart = nullptr;
