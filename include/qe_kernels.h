@@ -253,7 +253,7 @@ void qe_dequant_w4(const void* q, const void* s, int n, int k, int flags, uint16
  * m = 2..16 the matrix-core skinny kernel, whose rows are bit-identical for every m in 2..16 (a row does not depend
  * on the other rows of the batch); the two kernels agree to ~1e-6 relative (fp32 sums in another order), and with
  * qe_config_t.batch_invariant set m = 1 takes the skinny kernel too. Activation rows that are not 16-byte aligned
- * (x, or ldx not a multiple of 8) take the VALU decode kernel for every m. */
+ * (x, or ldx not a multiple of 8) take the skinny kernel's 4-dword loads (the same bits), at m = 1 the VALU kernel. */
 void qe_gemv_w4_ex(const void* q, const void* s, int n, int k, const uint16_t* x, int ldx, void* y, int ldy, int m,
                    int flags, void* stream);
 
@@ -261,9 +261,9 @@ void qe_gemv_w4_ex(const void* q, const void* s, int n, int k, const uint16_t* x
 void qe_gemm_w4_ex(const void* q, const void* s, int n, int k, const uint16_t* x, int ldx, void* y, int ldy, int t,
                    int flags, void* stream);
 
-/* GEMV for m <= 64 (row blocks of 16), GEMM above: the reference's matmul() dispatch (gemv.cuh:187-190) with the
- * decode range widened from 32 to 64 rows (measured faster on MI355X; every row of a 1..64-row call has the bits it
- * has alone). */
+/* GEMV for m <= 64, GEMM above: the reference's matmul() dispatch (gemv.cuh:187-190) with the decode range widened
+ * from 32 to 64 rows (measured faster on MI355X). 17..64 rows take the kernels of qe_gemv_w4; a row does not depend on
+ * the other rows of its call, and with batch_invariant every row of a 1..64-row call has the bits it has alone. */
 void qe_matmul_w4_ex(const void* q, const void* s, int n, int k, const uint16_t* x, int ldx, void* y, int ldy, int m,
                      int flags, void* stream);
 

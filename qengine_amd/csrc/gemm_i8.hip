@@ -393,7 +393,8 @@ __global__ void __launch_bounds__(NTH) gemm_i8_kernel(const uint4* __restrict__ 
     auto flush = [&](int gi, const float (&swf)[WNT][16]) {
 #pragma unroll
         for (int a = 0; a < WMT; a++) {
-            // kW4: the operand bytes are 16 (u - 8), the 1 / 16 goes into sx (a power of two: the same rounding)
+            // kW4: the operand bytes are 16 (u - 8), the 1 / 16 goes into sx (a power of two: the same rounding; where
+            // sx / 16 is subnormal, |x| below 2e-35 in the whole group, it loses the low bits of sx: to 4e-6 relative)
             const float sxa = sxv[a][gi] * (WF == kW4 ? 0.0625f : 1.f);
             const float msx = -kMagicF * sxa;  // exact: sx has 22 significant bits
 #pragma unroll

@@ -32,8 +32,8 @@ using namespace qe_gemv;
 
 // Tiles per wave RT: the weight tiles of RT consecutive 16-row tiles share one wave's staged activations and B
 // operand reads (the activation traffic per tile halves at RT = 2). Even slices can take RT = 2 (the host picks it
-// in launch()), uneven slices (NG = 0) at MT = 2..8 (16 rows at RT = 2 spill in one block per tile: N = 5120, K = 17408 29.8 -> 55.9
-// us; in parts they do not: part_pays).
+// in launch()), uneven slices (NG = 0) at MT = 2..8 (16 rows at RT = 2 spill in one block per tile: N = 5120, K = 17408
+// 29.8 -> 55.9 us; in parts they do not: part_pays).
 // Measured on uneven slices, RT = 1 -> 2: N = 5120, K = 17408, m = 2 / 4 / 8 15.7 / 16.3 / 21.6 -> 14.8 / 14.8 / 16.0
 // us; K = 13824 13.0 / 13.7 / 17.6 -> 12.2 / 12.2 / 13.1 us; N = 8192, K = 17408, m = 8 24.5 -> 17.5 us. Weight
 // groups in flight per wave D and the occupancy hint WPE, measured on the BASELINE shapes (K = 5120, 5-group slices;
@@ -483,7 +483,8 @@ __global__ void __launch_bounds__(256) skinny_sum_kernel(const float* __restrict
 // waves stage 9 KB each (12 waves: 108 KB of the CU's 160), so one block runs per CU and the tiles past the last whole
 // round of CUs run in a round of their own (320 tiles: 64 CUs hold two); and with up to 16 waves a block has no
 // registers for two tiles a wave, so every tile stages all activation rows (178 MB at N = 5120, K = 17408 for 45 MB of
-// weights). Blocks of four waves run four to a CU and hold two tiles a wave (135 VGPRs, no spill) where n / 16 is even.
+// weights). Blocks of four waves run four to a CU at one tile a wave (105 VGPRs); where n / 16 is even they hold two tiles
+// a wave (135 VGPRs, no spill: three to a CU).
 // us, one block -> RT = 1 -> RT = 2, with the second launch:
 //   N x K           m = 9                 m = 12                m = 16
 //   4608 x 17408    24.4 -> 19.4 -> 17.2  26.0 ->      -> 17.6  29.2 -> 23.0 -> 18.5
@@ -492,7 +493,7 @@ __global__ void __launch_bounds__(256) skinny_sum_kernel(const float* __restrict
 //   5120 x 28672    35.6 -> 30.4 -> 24.3  39.1 -> 31.7 -> 25.5  44.6 -> 34.1 -> 28.1
 //   8192 x 17408    27.2 -> 29.2 -> 23.1  28.0 ->      -> 23.8  30.9 -> 32.8 -> 26.7
 //  12288 x 13824    31.1 ->      -> 26.6  31.9 ->      -> 27.5  33.6 ->      -> 30.2
-// One tile a wave: only where the parts are all resident (four to a CU). Tiles that fill one round of CUs stay (N =
+// One tile a wave: only where the parts are all resident. Tiles that fill one round of CUs stay (N =
 // 4096, K = 13824, m = 9 / 16: 12.2 / 13.7 -> 13.0 / 14.6); fewer, shorter K than 12288 and more tiles than three
 // rounds were not measured and stay too (on a short K the second launch, ~2 us, is not paid back).
 inline bool part_pays(int n, int k, int S) {

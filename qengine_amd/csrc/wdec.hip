@@ -310,11 +310,12 @@ __global__ void __launch_bounds__(NTH, 2) wdec_kernel(const uint4* __restrict__ 
 // ran 34816 x 5120 (GLU, 89 MB) in 58 us and 5120 x 17408 in 44.5 us. This kernel takes 49 and 28 us (1.8 and 1.6
 // TB/s of records). What bounds it (variants that skip one part, 32768 x 5120, 44.5 us): without activation DMAs
 // 35.7, without record DMAs 34.7, without the MFMAs and their operands 30.9, records alone 22.4 us: matrix cores
-// (20 MFMAs a wave and step, 0.6 us of a 1.3 us step), LDS and DMA add up across the step's barrier. Records three
-// steps ahead with 48 staged rows, and whole-record LDS reads, measured the same. Here block = 8 waves = 2 row waves (64 weight rows
-// each, a 128-row slab) x 4 K parts; the two row waves of a K part share one staged activation tile [64][64], so a CU
-// stages half the activations per weight and holds 32 KB of records in flight (2 steps x 8 waves x 2 KB), and every
-// operand feeds two MFMAs. The bias -136 sum x is built once per pair (row wave rw does token block rw) and exchanged
+// (20 MFMAs a wave and step, 0.6 us of a 1.3 us step), LDS and DMA add up across the step's barrier. Counters of the
+// gated MLP of 48 rows (both matrices): MFMA busy 33 %, 33 % of the wave cycles waiting. Records three
+// steps ahead with 48 staged rows, and whole-record LDS reads, measured the same. Here block = 8 waves = 2 row waves (64
+// weight rows each, a 128-row slab) x 4 K parts; the two row waves of a K part share one staged activation tile
+// [64][64], so a CU stages half the activations per weight and holds 32 KB of records in flight (2 steps x 8 waves x
+// 2 KB), and every operand feeds two MFMAs. The bias -136 sum x is built once per pair (row wave rw does token block rw) and exchanged
 // through LDS at the group's end, so a k16 step is 5 MFMAs a wave for 4 of product. A step ends with a barrier (the
 // pair shares its tile); the group's flush acc += s (c + b) runs at the top of the next step. K parts are whole
 // groups, uneven where they do not divide; a wave whose part is shorter idles through the last steps' barriers.
@@ -700,11 +701,12 @@ bool wdec_w4_pick(const W4& w, const uint16_t* x, int ldx, int m) {
 
 // Slabs past the last whole round of CUs (N / 64 = 272 on 256 CUs: 16) would give 16 CUs two slabs; they run as P
 // K parts each instead (tail blocks, sharing CUs with the whole slabs), so no CU gets two slabs' work: P the first
-// of 5, 4, 8, 10, 2 with the tail blocks at most one round and an even number of steps per wave, if the stream's
-// zero-initialised workspace (kWsDec: counters, then the parts' sums) is at hand (without memory for it P = 1). The last part's in-order sum reads the P parts from the device-coherent level, one part at
-// a time, so fewer parts finish sooner: on C0's matrix (16 tail slabs, 80 K steps) P = 5 measured m = 32 / 64
-// 20.7 / 31.7 us against 22.9 / 36.9 us at P = 10, 23.1 / 33.3 us at P = 2, and 26.7 / 40.0 us with no tail split.
-// (wdec2_kernel: two_parts, summed by a kernel of their own.)
+// of 5, 4, 8, 10, 2 with the tail blocks at most one round and an even number of steps per wave, if the call has its
+// zero-initialised workspace (kWsDec: counters, then the parts' sums; without memory for it P = 1). The last part's
+// in-order sum reads the P parts from the device-coherent level, one part at a time, so fewer parts finish sooner: on
+// C0's matrix (16 tail slabs, 80 K steps) P = 5 measured m = 32 / 64 20.7 / 31.7 us against 22.9 / 36.9 us at P = 10,
+// 23.1 / 33.3 us at P = 2, and 26.7 / 40.0 us with no tail split. (wdec2_kernel: two_parts, summed by a kernel of its
+// own.)
 void wdec_w4(const W4& w, const uint16_t* x, int ldx, void* y, int ldy, int m, bool out_bf16, hipStream_t st) {
     using namespace qe_wdec;
     CHECK(wdec_w4_fits(w, x, ldx, m), "wdec_w4: n %d k %d m %d ldx %d", w.n, w.k, m, ldx);
